@@ -42,20 +42,14 @@ int kk_q4_gemv_pair_swiglu(const void *w_gate, const void *w_up, const float *x,
 int kk_swiglu(void *y, const void *gate, const void *up, int width, int rows, int gate_stride, int up_stride,
               int output_stride, int bytes, hipStream_t stream);
 
-// Q4_0 GEMV for batch 1..16 on fp16 MFMA (one pass over W): K % 64 == 0,
-// 4-byte aligned weights; workspace of kk_q4_mfma_gemv_workspace_bytes(k)
-// holds the activation fragments; `cus` sizes the grid.
-size_t kk_q4_mfma_gemv_workspace_bytes(int k);
-int kk_q4_mfma_gemv(const void *w, const float *x, float *y, int k, int n, int batch, void *workspace, int cus,
-                    hipStream_t stream);
-
-// The gate/up pair on the LDS-staged Q4_0 MFMA GEMV (K % 512 == 0, 16-byte
-// aligned weights and X, batch <= 16): one activation prepass into
-// `workspace` (kk_q4_mfma_gemv_workspace_bytes), then both products with
-// SwiGLU in the epilogue: y = [batch][n] = SiLU(X w_gate^T) * (X w_up^T).
-int kk_q4_mfma_pair_swiglu_supported(const void *w_gate, const void *w_up, const float *x, int k, int n, int batch);
-int kk_q4_mfma_gemv_pair_swiglu(const void *w_gate, const void *w_up, const float *x, float *y, int k, int n,
-                                int batch, void *workspace, hipStream_t stream);
+// Q4_0 GEMV for batch 1..32 on fp16 MFMA, one pass over the weights, K split
+// over workgroups (any K % 32 == 0, any weight alignment, 4-byte aligned X);
+// `workspace` of kk_q4_split_workspace_bytes holds partial sums (at most the
+// no-allocation entry point's scratch for one matrix). w_up null: y =
+// X w^T; else y = SiLU(X w^T) * (X w_up^T), both matrices [n,k].
+size_t kk_q4_split_workspace_bytes(int k, int n, int batch, int pair, int cus);
+int kk_q4_split_gemv(const void *w, const void *w_up, const float *x, float *y, int k, int n, int batch,
+                     void *workspace, int cus, hipStream_t stream);
 
 // Q4_0 GEMV for batch 1..16 on fp16 MFMA with block-diagonal activation
 // operands (one pass over W, lanes streaming whole block pairs, no

@@ -5,6 +5,8 @@
 #include "runtime_internal.h"
 #include "tuning.h"
 
+#include <kunlun/k200_c.h>
+
 #include <algorithm>
 #include <climits>
 #include <cstdint>
@@ -35,6 +37,16 @@ void * grow(int id, detail::DeviceContext & ctx, void *& ptr, size_t & size, siz
     return ptr;
 }
 
+// The split GEMV's partial sums differ from call to call of one program: what
+// needs more than 1 MiB takes the no-allocation scratch's size at once, so a
+// decode loop's first pass allocates once (each regrowth waits for the stream
+// and frees, 25 us and at times some hundred).
+void grow_split(int id, detail::DeviceContext & ctx, Kernel::Impl & impl, size_t need) {
+    if (need > impl.gemm_workspace_size)
+        need = std::max<size_t>(need, need > (1u << 20) ? KUNLUN_NOALLOC_SCRATCH_BYTES : 1u << 20);
+    grow(id, ctx, impl.gemm_workspace, impl.gemm_workspace_size, need);
+}
+
 } // namespace
 } // namespace kunlun
 
@@ -58,6 +70,20 @@ bool q4_mfma_batch(int batch, bool streamed) {
     const int max_b = std::min(16, kk::tuning_or(kk::kQ4MfmaMax, 16));
     return batch >= min_b && batch <= max_b;
 }
+
+// Whether the K-split Q4_0 MFMA GEMV takes a call no faster route took: above
+// 16 columns always; up to 16 the single-pass MFMA GEMV's batch range, where
+// shapes the batch-1 kernels cannot take (K % 64 != 0, weights off a dword)
+// count from 3 columns (K5600 x N3000: 3 / 8 / 16 columns 27 / 63 / 123 us on
+// the general GEMV, 13 / 13 / 14 us split).
+bool q4_split_route(const void * w, int k, int batch) {
+    if (batch > 16) return true;
+    const bool whole = k % 64 == 0 && ((uintptr_t)w & 3) == 0;
+    return q4_mfma_batch(batch, !whole || (k % 256 == 0 && ((uintptr_t)w & 15) == 0));
+}
+
+// Columns of one pass of batches above the small-batch kernels and off the GEMM.
+int gemv_chunk(int type) { return type == 2 && kk::tuning_or(kk::kQ4MfmaMax, 16) >= 16 ? 32 : 16; }
 
 // Batch range of the block-diagonal Q4_0 MFMA GEMV (the single-pass kernel's
 // range, unless KUNLUN_Q4_BDIAG=0 leaves it to the LDS-staged kernels).
@@ -128,15 +154,16 @@ static void dispatch_dense(Kernel::Impl & impl, detail::DeviceContext & ctx, int
                     const void * x, int k, int n, int batch, WeightType type) {
     const bool gemm = (type == WeightType::q4_0 || (type == WeightType::f16 && ((uintptr_t)w & 15) == 0)) &&
                       batch >= gemm_min_batch() && ((uintptr_t)x & 15) == 0;
-    if (!gemm && batch > 16) {
-        // batches between the small-batch kernels and the GEMM: chunks of 16
-        // columns, each on the route a 16-column call takes (one pass over
-        // the weights per chunk, against one per 2-4 columns on the general
-        // GEMV). X and Y chunks keep their alignment (K % 32 == 0).
+    const int chunk = kk::gemv_chunk((int)type);
+    if (!gemm && batch > chunk) {
+        // batches between the small-batch kernels and the GEMM: chunks of 32
+        // (Q4_0) or 16 columns, each on the route a call of that many columns
+        // takes (one pass over the weights per chunk). X and Y chunks keep
+        // their alignment (K % 32 == 0).
         const char * first = nullptr;
-        for (int b0 = 0; b0 < batch; b0 += 16) {
+        for (int b0 = 0; b0 < batch; b0 += chunk) {
             dispatch_dense(impl, ctx, id, static_cast<char *>(y) + (size_t)b0 * n * 4, w,
-                           static_cast<const char *>(x) + (size_t)b0 * k * 4, k, n, std::min(16, batch - b0), type);
+                           static_cast<const char *>(x) + (size_t)b0 * k * 4, k, n, std::min(chunk, batch - b0), type);
             if (!first) first = impl.route;
         }
         impl.route = first;
@@ -165,12 +192,12 @@ static void dispatch_dense(Kernel::Impl & impl, detail::DeviceContext & ctx, int
                                                        batch, ctx.cus, ctx.stream),
                           "kk_q4_bdiag_gemv");
         impl.route = "q4_bdiag_gemv";
-    } else if (type == WeightType::q4_0 && q4_mfma_batch(batch, k % 256 == 0 && ((uintptr_t)w & 15) == 0) &&
-               k % 64 == 0 && ((uintptr_t)w & 3) == 0) {
-        grow(id, ctx, impl.gemm_workspace, impl.gemm_workspace_size, kk_q4_mfma_gemv_workspace_bytes(k));
-        detail::check_hip((hipError_t)kk_q4_mfma_gemv(w, static_cast<const float *>(x), static_cast<float *>(y), k, n,
-                                                      batch, impl.gemm_workspace, ctx.cus, ctx.stream),
-                          "kk_q4_mfma_gemv");
+    } else if (type == WeightType::q4_0 && kk::q4_split_route(w, k, batch)) {
+        grow_split(id, ctx, impl, kk_q4_split_workspace_bytes(k, n, batch, 0, ctx.cus));
+        detail::check_hip((hipError_t)kk_q4_split_gemv(w, nullptr, static_cast<const float *>(x),
+                                                       static_cast<float *>(y), k, n, batch, impl.gemm_workspace,
+                                                       ctx.cus, ctx.stream),
+                          "kk_q4_split_gemv");
         impl.route = "q4_mfma_gemv";
     } else {
         detail::check_hip((hipError_t)kk_dense_matmul((int)type, w, static_cast<const float *>(x),
@@ -233,11 +260,10 @@ void matmul(Kernel & kernel, int id, void * y, const void * w, const void * x, i
     detail::count_matmul(id);
 }
 
-// Q4_0 gate/up pair of `batch` columns in one launch (both products and
-// SwiGLU), batch 1..16: the batch-1/2 GEMV's, the streamed, block-diagonal or
-// LDS-staged GEMV's pair form, whichever takes the shape; none: two GEMVs and
-// SwiGLU instead.
-enum class Q4PairRoute { none, dot8, stream, bdiag, mfma };
+// Q4_0 gate/up pair of `batch` columns, batch 1..32: the batch-1/2 GEMV's, the
+// streamed, block-diagonal or K-split GEMV's pair form, whichever takes the
+// shape; none: two GEMVs and SwiGLU instead.
+enum class Q4PairRoute { none, dot8, stream, bdiag, split };
 
 static Q4PairRoute q4_pair_route(const void * w_gate, const void * w_up, const float * x, int k, int n, int batch) {
     if (kk_q4_gemv_pair_swiglu_supported(w_gate, w_up, x, k, n, batch)) return Q4PairRoute::dot8;
@@ -247,8 +273,8 @@ static Q4PairRoute q4_pair_route(const void * w_gate, const void * w_up, const f
     if (kk::q4_bdiag_batch(batch) && kk_q4_bdiag_gemv_supported(w_gate, x, k, n, batch) &&
         kk_q4_bdiag_gemv_supported(w_up, x, k, n, batch))
         return Q4PairRoute::bdiag;
-    if (q4_mfma_batch(batch, true) && kk_q4_mfma_pair_swiglu_supported(w_gate, w_up, x, k, n, batch))
-        return Q4PairRoute::mfma;
+    if (batch > 16 || (kk::q4_split_route(w_gate, k, batch) && kk::q4_split_route(w_up, k, batch)))
+        return Q4PairRoute::split;
     return Q4PairRoute::none;
 }
 
@@ -271,13 +297,12 @@ static void run_q4_pair(Q4PairRoute route, Kernel::Impl & impl, detail::DeviceCo
                           "kk_q4_bdiag_gemv_pair_swiglu");
         impl.route = "q4_bdiag_pair_swiglu";
         break;
-    case Q4PairRoute::mfma:
-        // the LDS-staged MFMA GEMV: one activation prepass, both products and
-        // SwiGLU in one launch
-        grow(id, ctx, impl.gemm_workspace, impl.gemm_workspace_size, kk_q4_mfma_gemv_workspace_bytes(k));
-        detail::check_hip((hipError_t)kk_q4_mfma_gemv_pair_swiglu(w_gate, w_up, x, y, k, n, batch, impl.gemm_workspace,
-                                                                  ctx.stream),
-                          "kk_q4_mfma_gemv_pair_swiglu");
+    case Q4PairRoute::split:
+        // both products' K ranges in one launch, their sums and SwiGLU in the next
+        grow_split(id, ctx, impl, kk_q4_split_workspace_bytes(k, n, batch, 1, ctx.cus));
+        detail::check_hip((hipError_t)kk_q4_split_gemv(w_gate, w_up, x, y, k, n, batch, impl.gemm_workspace, ctx.cus,
+                                                       ctx.stream),
+                          "kk_q4_split_gemv");
         impl.route = "q4_mfma_pair_swiglu";
         break;
     case Q4PairRoute::none:
@@ -297,6 +322,7 @@ void matmul_swiglu(Kernel & kernel, int id, void * y, const void * w_gate, const
     detail::DeviceContext & ctx = detail::context(id);
     Kernel::Impl & impl = *kernel.impl_;
     impl.id = id;
+    const int chunk = kk::gemv_chunk((int)type);
     const bool f16_aligned = ((uintptr_t)w_gate & 15) == 0 && ((uintptr_t)w_up & 15) == 0;
     if ((type == WeightType::q4_0 || (type == WeightType::f16 && f16_aligned)) && batch >= gemm_min_batch() &&
         ((uintptr_t)x & 15) == 0) {
@@ -305,21 +331,21 @@ void matmul_swiglu(Kernel & kernel, int id, void * y, const void * w_gate, const
                                                      static_cast<float *>(y), k, n, batch, impl.gemm_workspace,
                                                      ctx.stream, &impl.route),
                           "kk_gemm_swiglu");
-    } else if (type == WeightType::q4_0 &&
+    } else if (type == WeightType::q4_0 && batch <= chunk &&
                q4_pair_route(w_gate, w_up, static_cast<const float *>(x), k, n, batch) != Q4PairRoute::none) {
         // decode and small batch: both products and SwiGLU in one launch
         run_q4_pair(q4_pair_route(w_gate, w_up, static_cast<const float *>(x), k, n, batch), impl, ctx, id,
                     static_cast<float *>(y), w_gate, w_up, static_cast<const float *>(x), k, n, batch);
-    } else if (type == WeightType::q4_0 && batch > 16 &&
-               q4_pair_route(w_gate, w_up, static_cast<const float *>(x), k, n, 16) != Q4PairRoute::none &&
-               (batch % 16 == 0 || q4_pair_route(w_gate, w_up, static_cast<const float *>(x), k, n, batch % 16) !=
-                                       Q4PairRoute::none)) {
-        // batches between the small-batch kernels and the GEMM: chunks of 16
-        // columns, each in one pair launch (X and Y chunks keep their
+    } else if (type == WeightType::q4_0 && batch > chunk &&
+               q4_pair_route(w_gate, w_up, static_cast<const float *>(x), k, n, chunk) != Q4PairRoute::none &&
+               (batch % chunk == 0 || q4_pair_route(w_gate, w_up, static_cast<const float *>(x), k, n, batch % chunk) !=
+                                          Q4PairRoute::none)) {
+        // batches between the small-batch kernels and the GEMM: chunks of
+        // columns, each on its own pair route (X and Y chunks keep their
         // alignment: K % 32 == 0)
         const char * first = nullptr;
-        for (int b0 = 0; b0 < batch; b0 += 16) {
-            const int cols = std::min(16, batch - b0);
+        for (int b0 = 0; b0 < batch; b0 += chunk) {
+            const int cols = std::min(chunk, batch - b0);
             const float * xc = reinterpret_cast<const float *>(static_cast<const char *>(x) + (size_t)b0 * k * 4);
             run_q4_pair(q4_pair_route(w_gate, w_up, xc, k, n, cols), impl, ctx, id,
                         reinterpret_cast<float *>(static_cast<char *>(y) + (size_t)b0 * n * 4), w_gate, w_up, xc, k, n,

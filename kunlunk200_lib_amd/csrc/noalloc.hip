@@ -3,8 +3,8 @@
 // graph capture, tight serving loops). It takes the routes and kernels of
 // kunlun::matmul (matmul.cpp); the routes that need device memory beyond the
 // inputs and outputs -- the fp16-MFMA prefill GEMM (fp16 activations and row
-// scales, kk_gemm_workspace_bytes) and the LDS-staged Q4_0 MFMA GEMV
-// (activation fragments, kk_q4_mfma_gemv_workspace_bytes) -- take it from `scratch`, a
+// scales, kk_gemm_workspace_bytes) and the K-split Q4_0 MFMA GEMV (partial
+// sums, kk_q4_split_workspace_bytes) -- take it from `scratch`, a
 // file-scope device array of kScratchBytes, instead of a Kernel's workspace.
 //
 // Every GPU the library runs on holds its own copy of the array until the
@@ -65,7 +65,7 @@ int too_large(size_t need) {
     return KUNLUN_NOALLOC_TOO_LARGE;
 }
 
-// kunlun_matmul's route for at most 16 columns (X 16-byte aligned or not),
+// kunlun_matmul's route for one chunk of columns (X 16-byte aligned or not),
 // with its scratch in the device's array
 hipError_t small_batch(DeviceScratch &d, int type, const void *w, const float *xf, float *yf, int k, int n, int batch,
                        uintptr_t wa, hipStream_t s, const char **taken) {
@@ -82,11 +82,11 @@ hipError_t small_batch(DeviceScratch &d, int type, const void *w, const float *x
         *taken = "q4_bdiag_gemv";
         return static_cast<hipError_t>(kk_q4_bdiag_gemv(w, xf, yf, k, n, batch, d.cus, s));
     }
-    if (type == 2 && kk::q4_mfma_batch(batch, k % 256 == 0 && (wa & 15) == 0) && k % 64 == 0 && (wa & 3) == 0) {
-        const size_t need = kk_q4_mfma_gemv_workspace_bytes(k);
+    if (type == 2 && kk::q4_split_route(w, k, batch)) {
+        const size_t need = kk_q4_split_workspace_bytes(k, n, batch, 0, d.cus);
         if (need > kScratchBytes) return static_cast<hipError_t>(too_large(need));
         *taken = "q4_mfma_gemv";
-        return static_cast<hipError_t>(kk_q4_mfma_gemv(w, xf, yf, k, n, batch, d.ptr, d.cus, s));
+        return static_cast<hipError_t>(kk_q4_split_gemv(w, nullptr, xf, yf, k, n, batch, d.ptr, d.cus, s));
     }
     return static_cast<hipError_t>(kk_dense_matmul(type, w, xf, yf, k, n, batch, s, taken));
 }
@@ -126,10 +126,11 @@ extern "C" int kunlun_matmul_noalloc(int device, void *y, const void *w, const v
         if (need > kScratchBytes) return too_large(need);
         rc = static_cast<hipError_t>(kk_gemm(type, w, xf, yf, k, n, batch, d.ptr, s, &taken));
     } else {
-        // kunlun_matmul's small-batch routes; above 16 columns, chunks of 16
-        // (as kunlun_matmul runs them), in stream order on the one array
-        for (int b0 = 0; b0 < batch && rc == hipSuccess; b0 += 16) {
-            const int bc = std::min(16, batch - b0);
+        // kunlun_matmul's small-batch routes, in its chunks of columns, in
+        // stream order on the one array
+        const int chunk = kk::gemv_chunk(type);
+        for (int b0 = 0; b0 < batch && rc == hipSuccess; b0 += chunk) {
+            const int bc = std::min(chunk, batch - b0);
             const char *chunk_route = nullptr;
             rc = small_batch(d, type, w, xf + static_cast<size_t>(b0) * k, yf + static_cast<size_t>(b0) * n, k, n, bc,
                              wa, s, &chunk_route);

@@ -44,6 +44,8 @@ namespace kk {
 // aligned weights) and the F32/F16 single-pass MFMA GEMVs.
 int gemm_min_batch();
 bool q4_mfma_batch(int batch, bool streamed);
+bool q4_split_route(const void * w, int k, int batch);
+int gemv_chunk(int type);
 bool q4_bdiag_batch(int batch);
 bool q4_stream_batch(int batch);
 bool dense_mfma_batch(int batch);
@@ -55,7 +57,7 @@ struct Kernel::Impl {
     int id = -1;
     void * i8_workspace = nullptr;      // rowwise_i8 activation codes and maxima
     size_t i8_workspace_size = 0;
-    void * gemm_workspace = nullptr;    // fp16 activations of the prefill GEMM
+    void * gemm_workspace = nullptr;    // fp16 activations of the prefill GEMM; partial sums of the split GEMV
     size_t gemm_workspace_size = 0;
     void * pair_workspace = nullptr;    // gate/up GEMV outputs of matmul_swiglu; elementwise copy of b
     size_t pair_workspace_size = 0;

@@ -1,0 +1,68 @@
+"""GPU parity of the K-split Q4_0 MFMA GEMV (3..32 columns per pass, route
+q4_mfma_gemv) and its gate/up pair: partial last steps and blocks (K % 256,
+K % 64), weights and activations off their natural alignment, one and several
+K ranges and LDS chunks, tiles of several rounds, and the cap on partial sums.
+
+Bound: the F32-accumulate GEMV's, |y - gold| <= 1e-4 * ||x_b|| * ||w_r||, gold
+the FP64 dot of the exactly decoded weights.
+"""
+import numpy as np
+import pytest
+
+import kunlunk200_lib_amd as kl
+from gpu_util import check_f32_accumulate, run_matmul
+from test_gpu_swiglu import check_pair, run_pair
+
+pytestmark = pytest.mark.gpu
+
+Q4 = kl.WeightType.q4_0
+
+# (k, n, batch, w_offset, x_offset)
+SHAPES = [(32, 7, 9, 0, 0), (96, 33, 17, 0, 0), (544, 70, 3, 0, 0), (1056, 65, 24, 0, 0),    # K % 64 == 32
+          (2048, 129, 20, 2, 0), (1024, 50, 12, 1, 0), (512, 40, 7, 3, 4), (4096, 33, 31, 4, 8),   # misaligned
+          (4096, 16, 16, 0, 0), (4096, 17, 32, 0, 0), (4096, 300, 33, 0, 0), (4096, 300, 63, 0, 0),
+          (11008, 257, 8, 0, 0), (11008, 40, 12, 0, 0), (16384, 48, 32, 0, 0), (2304, 33000, 32, 0, 0),
+          (512, 20000, 30, 0, 0), (8192, 1, 5, 0, 0)]
+
+
+@pytest.mark.parametrize("k,n,batch,w_offset,x_offset", SHAPES)
+def test_split_shapes(gpu, oracle, k, n, batch, w_offset, x_offset):
+    rng = np.random.default_rng(k + 3 * n + batch)
+    q4 = kl.quantize_q4_0((rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    x = rng.standard_normal((batch, k)).astype(np.float32)
+    x[batch - 1] *= 1e-20                      # each column and step has its own scale
+    x[0, : k // 2] *= 1e8
+    y, route, guard_ok = run_matmul(Q4, q4, x, k, n, batch, w_offset=w_offset, x_offset=x_offset)
+    dec = oracle.q4_decode(q4, k, n)
+    res = check_f32_accumulate(y, oracle.gold(dec, x, threads=16), dec, x)
+    print(f"  split k={k} n={n} b={batch} route={route} {res}", flush=True)
+    assert route in ("q4_mfma_gemv", "q4_bdiag_gemv", "q4_stream_gemv")
+    assert guard_ok and res["finite"] and res["north_star"]
+
+
+@pytest.mark.parametrize("k,batch", [(4096, 20), (11008, 6), (1056, 12)])
+def test_split_nonfinite(gpu, oracle, k, batch):
+    # a non-finite activation makes its column NaN and no other; an infinite
+    # block scale makes its row's outputs infinite or NaN and no other's
+    n = 40
+    rng = np.random.default_rng(k)
+    q4 = kl.quantize_q4_0((rng.standard_normal((n, k)) * 0.02).astype(np.float32)).reshape(n, k // 32, 18)
+    q4[5, k // 32 - 1, :2] = np.array([np.inf], np.float16).view(np.uint8)
+    x = rng.standard_normal((batch, k)).astype(np.float32)
+    x[1, 3], x[2, k - 1] = np.nan, -np.inf
+    y, _, guard_ok = run_matmul(Q4, q4.reshape(n, -1), x, k, n, batch)
+    rows = np.arange(n) != 5
+    assert guard_ok and np.all(np.isnan(y[1])) and np.all(np.isnan(y[2]))
+    rest = np.delete(y, (1, 2), axis=0)
+    assert np.all(np.isfinite(rest[:, rows])) and not np.any(np.isfinite(rest[:, 5]))
+
+
+@pytest.mark.parametrize("k,n,batch", [(1056, 65, 24), (4096, 300, 32), (11008, 50, 5), (2048, 1000, 30), (96, 20, 40)])
+def test_split_pair(gpu, oracle, k, n, batch):
+    rng = np.random.default_rng(k + n + batch)
+    pg, pu = (kl.quantize_q4_0((rng.standard_normal((n, k)) * 0.02).astype(np.float32)) for _ in range(2))
+    x = rng.standard_normal((batch, k)).astype(np.float32)
+    y, route = run_pair(Q4, pg, pu, x, k, n, batch)
+    finite, ok, worst = check_pair(y, x, oracle.q4_decode(pg, k, n), oracle.q4_decode(pu, k, n), oracle, 1e-4)
+    print(f"  split pair k={k} n={n} b={batch} {route} worst/bound={worst:.3g}", flush=True)
+    assert route == "q4_mfma_pair_swiglu" and finite and ok
