@@ -69,7 +69,7 @@ struct ActivationStorage {
     size_t quant_bytes = 0;
     void * scale = nullptr;
     size_t scale_bytes = 0;
-    void * tiled = nullptr;             // M > 1 codes in the GEMM's operand order
+    void * tiled = nullptr;             // M > 1 codes as the GEMM's fp16 operands
     size_t tiled_bytes = 0;
     uint64_t epoch = 0;
     bool valid = false;
@@ -204,7 +204,7 @@ struct CommonQ4ActivationLease::Impl {
     const void * input = nullptr;
     size_t input_bytes = 0;
     std::vector<CommonQ4ActivationChunk> chunks;
-    std::vector<const void *> tiled;       // per chunk: M > 1 codes in the GEMM's operand order
+    std::vector<const void *> tiled;       // per chunk: M > 1 codes as the GEMM's fp16 operands
 };
 
 struct CommonQ4Workspace::Impl {
@@ -301,24 +301,31 @@ int gemm_path(int padded, int kp) {
 
 bool exact_route(const CommonQ4Info & a) { return (size_t)a.np * a.kp > kExactRoute; }
 
-// Quantizes one chunk of rows into (values, scales); returns launches made.
-void quantize_chunk(CommonQ4Workspace::Impl & s, hipStream_t stream, const void * x, int x_f16, const CommonQ4Info & a,
-                    int m, int rows, int padded, void * values, void * scales, void * tiled) {
+// Rows quantized and multiplied in one launch each: what the workspace holds.
+constexpr int kGroupRows = 512;
+
+// Quantizes `rows` rows (chunks of 128, chunk_stride apart in `values`; M = 1:
+// the per-tensor pair). The counters are the reference's, one chunk at a time.
+void quantize_rows(CommonQ4Workspace::Impl & s, hipStream_t stream, const void * x, int x_f16, const CommonQ4Info & a,
+                   int m, int rows, size_t chunk_stride, void * values, void * scales, void * tiled) {
     ActivationStorage & st = *s.activation;
     const uint64_t t0 = st.profile ? now_ns() : 0;
+    const int last = (rows - 1) % 128 + 1;
     if (m == 1)
         detail::check_hip((hipError_t)kk_common_quant_pair(x, x_f16, a.k, a.kp, values, scales, stream),
                           "kk_common_quant_pair");
     else
-        detail::check_hip((hipError_t)kk_common_quant_rows(x, x_f16, a.k, a.kp, rows, round_up(padded, 32), values,
-                                                           scales, tiled, stream),
+        detail::check_hip((hipError_t)kk_common_quant_rows(x, x_f16, a.k, a.kp, rows,
+                                                           rows - last + round_up(padded_rows(m, last), 32),
+                                                           chunk_stride, values, scales, tiled, stream),
                           "kk_common_quant_rows");
     if (st.profile) {
         detail::check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize");
         st.stats.quantization_ns += now_ns() - t0;
     }
-    ++st.stats.quantized_chunks;
-    ++st.stats.quant_kernel_launches;
+    const size_t chunks = ((size_t)rows + 127) / 128;
+    st.stats.quantized_chunks += chunks;
+    st.stats.quant_kernel_launches += chunks;
 }
 
 // Runs every chunk of Y = X W^T. `prepared` supplies quantized chunks (or
@@ -330,62 +337,69 @@ bool execute(CommonQ4Workspace::Impl & s, int id, void * y, const CommonQ4Info &
     detail::DeviceContext & ctx = detail::context(id);
     ActivationStorage & st = *s.activation;
     if (m == 1 && exact_route(a) && prepared) return false;
-    size_t index = 0;
-    for (int first = 0; first < m;) {
-        const int rows = std::min(128, m - first), padded = padded_rows(m, rows);
-        const void * x = static_cast<const char *>(input) + (size_t)first * a.k * bytes;
-        float * out = static_cast<float *>(y) + (size_t)first * a.n;
-        const CommonQ4ActivationChunk * chunk = prepared ? &prepared->chunks[index++] : nullptr;
-        if (m == 1 && exact_route(a)) {
-            detail::check_hip((hipError_t)kk_common_gemv(w, out, nullptr, nullptr, x, 2, x_f16, nullptr, nullptr, a.k,
-                                                         a.kp, a.n, a.np, ctx.stream),
-                              "kk_common_gemv");
-            s.last_components = 0;
-            ++s.stats.paths[7];
-        } else {
-            const void * values;
-            const void * scales;
-            const void * tiled = nullptr;
-            if (chunk) {
-                values = chunk->values;
-                scales = chunk->scales;
-                tiled = prepared->tiled[index - 1];
-            } else {
-                reserve(st, id, st.quant, st.quant_bytes, m == 1 ? (size_t)4 * a.kp + 1024 : (size_t)128 * a.kp + 1024);
-                reserve(st, id, st.scale, st.scale_bytes, m == 1 ? 64 : 128 * 64);
-                if (m != 1) reserve(st, id, st.tiled, st.tiled_bytes, (size_t)128 * a.kp);
-                // M = 1 quantizes inside the GEMV (every workgroup for itself,
-                // workgroup 0 writes the view); M > 1 runs the row kernel first
-                if (m != 1) quantize_chunk(s, ctx.stream, x, x_f16, a, m, rows, padded, st.quant, st.scale, st.tiled);
-                else ++st.stats.quantized_chunks;
-                values = st.quant;
-                scales = st.scale;
-                tiled = st.tiled;
-            }
-            if (m == 1) {
-                const bool fused = chunk == nullptr;
-                detail::check_hip((hipError_t)kk_common_gemv(w, out, nullptr, nullptr, fused ? x : values, fused ? 1 : 0,
-                                                             x_f16, const_cast<void *>(scales),
-                                                             const_cast<void *>(values), a.k, a.kp, a.n, a.np,
-                                                             ctx.stream),
-                                  "kk_common_gemv");
-                s.last_components = 2;
-                ++s.stats.paths[0];
-            } else {
-                detail::check_hip((hipError_t)kk_common_gemm(w, tiled, scales, out, rows, round_up(padded, 32), a.kp,
-                                                             a.n, a.np, ctx.stream),
-                                  "kk_common_gemm");
-                s.last_components = 1;
-                ++s.stats.paths[gemm_path(padded, a.kp)];
-            }
-            s.last_values = values;
-            s.last_scales = scales;
-        }
-        s.last_rows = rows;
-        s.last_kp = a.kp;
-        first += rows;
+    if (m == 1 && exact_route(a)) {
+        detail::check_hip((hipError_t)kk_common_gemv(w, static_cast<float *>(y), nullptr, nullptr, input, 2, x_f16,
+                                                     nullptr, nullptr, a.k, a.kp, a.n, a.np, ctx.stream),
+                          "kk_common_gemv");
+        s.last_components = 0;
+        s.last_rows = 1;
+        ++s.stats.paths[7];
         ++s.stats.chunks;
+    } else if (m == 1) {
+        if (!prepared) {
+            reserve(st, id, st.quant, st.quant_bytes, (size_t)4 * a.kp + 1024);
+            reserve(st, id, st.scale, st.scale_bytes, 64);
+            // quantized inside the GEMV (every workgroup for itself, workgroup 0
+            // writes the view)
+            ++st.stats.quantized_chunks;
+        }
+        s.last_values = prepared ? prepared->chunks[0].values : st.quant;
+        s.last_scales = prepared ? prepared->chunks[0].scales : st.scale;
+        detail::check_hip((hipError_t)kk_common_gemv(w, static_cast<float *>(y), nullptr, nullptr,
+                                                     prepared ? s.last_values : input, prepared ? 0 : 1, x_f16,
+                                                     const_cast<void *>(s.last_scales),
+                                                     const_cast<void *>(s.last_values), a.k, a.kp, a.n, a.np,
+                                                     ctx.stream),
+                          "kk_common_gemv");
+        s.last_components = 2;
+        s.last_rows = 1;
+        ++s.stats.paths[0];
+        ++s.stats.chunks;
+    } else {
+        // a lease's rows in one GEMM (its chunks' fragments and scales are
+        // contiguous), else groups of rows quantized here
+        const int group = prepared ? m : std::min(m, kGroupRows);
+        const size_t capacity = (size_t)round_up(group, 128);
+        if (!prepared) {
+            reserve(st, id, st.quant, st.quant_bytes, capacity * a.kp + 1024);
+            reserve(st, id, st.scale, st.scale_bytes, capacity * 64);
+            reserve(st, id, st.tiled, st.tiled_bytes, capacity * a.kp * 2);
+        }
+        for (int first = 0; first < m; first += group) {
+            const int rows = std::min(group, m - first);
+            if (!prepared)
+                quantize_rows(s, ctx.stream, static_cast<const char *>(input) + (size_t)first * a.k * bytes, x_f16, a, m,
+                              rows, (size_t)128 * a.kp, st.quant, st.scale, st.tiled);
+            const void * frags = prepared ? prepared->tiled[0] : st.tiled;
+            const void * scales = prepared ? prepared->chunks[0].scales : st.scale;
+            detail::check_hip((hipError_t)kk_common_gemm(w, frags, scales, static_cast<float *>(y) + (size_t)first * a.n,
+                                                         rows, a.kp, a.n, a.np, ctx.cus, ctx.stream),
+                              "kk_common_gemm");
+            for (int r = 0; r < rows; r += 128) {
+                ++s.stats.paths[gemm_path(padded_rows(m, std::min(128, rows - r)), a.kp)];
+                ++s.stats.chunks;
+            }
+            // the view is the last chunk's
+            const size_t last = ((size_t)rows - 1) / 128;
+            s.last_values = prepared ? prepared->chunks[last].values
+                                     : static_cast<const char *>(st.quant) + last * 128 * a.kp;
+            s.last_scales = prepared ? prepared->chunks[last].scales
+                                     : static_cast<const char *>(st.scale) + last * 128 * 64;
+            s.last_rows = rows - (int)last * 128;
+        }
+        s.last_components = 1;
     }
+    s.last_kp = a.kp;
     detail::check_hip(hipStreamSynchronize(ctx.stream), "hipStreamSynchronize");
     ++s.stats.calls;
     detail::count_matmul(id);
@@ -452,7 +466,7 @@ bool common_q4_prepare(CommonQ4Workspace & work, int id, const void * input, int
     detail::DeviceContext & ctx = detail::context(id);
     reserve(st, id, st.quant, st.quant_bytes, chunks * qstride);
     reserve(st, id, st.scale, st.scale_bytes, chunks * sstride);
-    if (m != 1) reserve(st, id, st.tiled, st.tiled_bytes, chunks * 128 * (size_t)a.kp);
+    if (m != 1) reserve(st, id, st.tiled, st.tiled_bytes, chunks * 128 * (size_t)a.kp * 2);
     CommonQ4ActivationLease::Impl & l = *lease.impl_;
     l.storage = s.activation;
     l.epoch = st.epoch;
@@ -463,15 +477,13 @@ bool common_q4_prepare(CommonQ4Workspace & work, int id, const void * input, int
     l.type = type;
     l.input = input;
     l.input_bytes = input_bytes;
+    quantize_rows(s, ctx.stream, input, bytes == 2, a, m, m, qstride, st.quant, st.scale, st.tiled);
     size_t index = 0;
     for (int first = 0; first < m; ++index) {
         const int rows = std::min(128, m - first), padded = padded_rows(m, rows);
-        const void * x = static_cast<const char *>(input) + (size_t)first * k * bytes;
         void * q = static_cast<char *>(st.quant) + index * qstride;
         void * sc = static_cast<char *>(st.scale) + index * sstride;
-        void * tl = m == 1 ? nullptr : static_cast<char *>(st.tiled) + index * 128 * (size_t)a.kp;
-        quantize_chunk(s, ctx.stream, x, bytes == 2, a, m, rows, padded, q, sc, tl);
-        l.tiled.push_back(tl);
+        l.tiled.push_back(m == 1 ? nullptr : static_cast<char *>(st.tiled) + index * 128 * (size_t)a.kp * 2);
         const int defined = m == 1 ? 1 : round_up(padded, 32);
         l.chunks.push_back({q, sc, first, rows, padded, a.kp, m == 1 ? 2 : 1,
                             m == 1 ? qstride : (size_t)defined * a.kp, m == 1 ? sstride : (size_t)defined * 64});

@@ -14,10 +14,11 @@
 //          q0 = rnd(x * (127/max0)), r = x - q0 * (max0/127), q1 the same on r;
 //   M > 1: per row, one component q = rnd(x * (127/max_row)).
 // rnd rounds half away from zero and clamps to [-127, 127]. Products with the
-// weights are exact int32 block sums (v_dot4_i32_i8 / v_mfma_i32_16x16x32_i8
-// on weights widened to 16*q), then y = sum_b d_b * (S0 s0 + S1 s1) in F32.
+// weights are exact integer block sums (M = 1: v_dot4_i32_i8 on weights widened
+// to 16*q; M > 1: fp16 MFMA), then y = sum_b d_b * (S0 s0 + S1 s1) in F32.
 #include "device_common.h"
 #include "launch.h"
+#include "lds_opt_in.h"
 
 #include <algorithm>
 
@@ -170,21 +171,17 @@ __global__ __launch_bounds__(kQuantThreads) void common_quant_pair(const void *_
 
 // ---------------------------------------------------------------------------
 // M > 1: Row A8. Workgroup r quantizes row r of X (rows >= `rows` are the
-// zero padding rows: scale 1/127, codes 0) into values[r*kp ..] and writes the
-// row scale to all 16 floats of params[r*16 ..]. The same codes also go to
-// `tiled` in the GEMM's A-operand order, two blocks per lane: row r, K j at
-// (((r/16) * (kp/64) + j/64) * 64 + r%16 + 16 * (j%32/8)) * 16 + (j/32 % 2) * 8 + j%8,
-// so one wave reads a 16-row x 64-K operand pair as 1 KB contiguous.
-__device__ __forceinline__ size_t tiled_offset(int r, int j, int blocks) {
-    return ((static_cast<size_t>(r / 16) * (blocks / 2) + j / 64) * 64 + r % 16 + 16 * ((j % 32) / 8)) * 16 +
-           ((j / 32) % 2) * 8 + j % 8;
-}
-
+// zero padding rows: scale 1/127, codes 0) into values[(r/128) * chunk_stride +
+// (r%128) * kp ..] and writes the row scale to all 16 floats of params[r*16 ..].
+// The same codes also go to `frags` as the GEMM's fp16 A operands (an int8 is
+// exact in fp16): fragment (r/16, block b) is 64 lanes x 8 halves at
+// ((r/16) * (kp/32) + b) * 512, lane r%16 + 16 g holding K 8g + (0, 4, 2, 6, 1, 5,
+// 3, 7) of the block, the order in which a weight dword's nibbles decode.
 template <bool F16>
-__global__ __launch_bounds__(kRowThreads) void common_quant_rows(const void *__restrict__ x, int x_f16, int k,
-                                                                int kp, int rows, int8_t *__restrict__ values,
+__global__ __launch_bounds__(kRowThreads) void common_quant_rows(const void *__restrict__ x, int k, int kp, int rows,
+                                                                size_t chunk_stride, int8_t *__restrict__ values,
                                                                 float *__restrict__ params,
-                                                                int8_t *__restrict__ tiled) {
+                                                                _Float16 *__restrict__ frags) {
 #pragma clang fp contract(off)
     __shared__ uint32_t scratch[kRowThreads / 64];
     const int row = blockIdx.x;
@@ -201,19 +198,21 @@ __global__ __launch_bounds__(kRowThreads) void common_quant_rows(const void *__r
     m = block_max_bits<kRowThreads>(m, scratch);
     const float mx = m ? __uint_as_float(m) : 1.0f;
     const float scale = mx / 127.0f, inv = 127.0f / mx;
-    // four values per thread per step, written as one dword
-    uint32_t *out = reinterpret_cast<uint32_t *>(values + static_cast<size_t>(row) * kp);
-    for (int d = threadIdx.x; d < kp / 4; d += kRowThreads) {
-        int q[4];
+    // eight values per thread and step: two code dwords and one lane's 16 fragment bytes
+    uint2 *out = reinterpret_cast<uint2 *>(values + static_cast<size_t>(row >> 7) * chunk_stride +
+                                           static_cast<size_t>(row & 127) * kp);
+    kk::half8 *frag = reinterpret_cast<kk::half8 *>(frags) + static_cast<size_t>(row >> 4) * (kp >> 5) * 64 + (row & 15);
+    for (int d = threadIdx.x; d < kp / 8; d += kRowThreads) {
+        int q[8];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int j = 4 * d + t;
-            const float v = x_value<F16>(xr, j);
-            q[t] = kk::round_clamp(v * inv, 127);
-        }
-        const uint32_t word = pack4(q[0], q[1], q[2], q[3]);
-        out[d] = word;
-        *reinterpret_cast<uint32_t *>(tiled + tiled_offset(row, 4 * d, kp / 32)) = word;
+        for (int t = 0; t < 8; ++t) q[t] = kk::round_clamp(x_value<F16>(xr, 8 * d + t) * inv, 127);
+        out[d] = make_uint2(pack4(q[0], q[1], q[2], q[3]), pack4(q[4], q[5], q[6], q[7]));
+        kk::half8 h;
+        h[0] = static_cast<_Float16>(q[0]); h[1] = static_cast<_Float16>(q[4]);
+        h[2] = static_cast<_Float16>(q[2]); h[3] = static_cast<_Float16>(q[6]);
+        h[4] = static_cast<_Float16>(q[1]); h[5] = static_cast<_Float16>(q[5]);
+        h[6] = static_cast<_Float16>(q[3]); h[7] = static_cast<_Float16>(q[7]);
+        frag[(d >> 2) * 64 + 16 * (d & 3)] = h;
     }
     if (threadIdx.x < 16) params[row * 16 + threadIdx.x] = scale;
 }
@@ -452,175 +451,193 @@ __global__ __launch_bounds__(kCqThreads) void common_gemv(GemvMatrix m0, GemvMat
 }
 
 // ---------------------------------------------------------------------------
-// M > 1 GEMM on v_mfma_i32_16x16x32_i8 (one K32 block per MFMA, so each
-// block's int32 sums get their own FP16 scale). A workgroup is one N32 tile x
-// up to 128 rows: wave w owns rows 32w .. 32w+31 (two 16-row tiles).
+// M > 1 GEMM on v_mfma_f32_16x16x32_f16, one K32 block per MFMA: int8 codes and
+// 4-bit weights are exact in fp16 and a block's sum (at most 32 * 127 * 8) is
+// exact in F32, so D is the block's integer sum and needs one fma per output
+// with the block's FP16 scale. (v_mfma_i32_16x16x32_i8, used before, needs a
+// conversion as well: twice the VALU work, which is what bounds this kernel.)
 //
-// Data path (wide loads only; narrow per-lane loads cost one L1 tag access
-// per few lanes and starve this kernel): per stage of 8 blocks the tile's 4 KB
-// of weights and 512 B of scales are copied into LDS by the 4 waves
-// (global_load_lds, 16 B per lane, 2 copies per wave), two stages ahead into
-// a ring of 3 buffers; each wave loads its activation operands with one
-// dwordx4 per lane per row tile and block pair (the tiled order of
-// common_quant_rows), one stage ahead. MFMA operand layout (wave64):
-// A[l%16][8(l/16) .. +8), B[8(l/16) .. +8)[l%16], D[4(l/16) + r][l%16]; B
-// lane l: column 16g + l%16 of the tile, K dword l/16 of the block, widened
-// to 8 int8 = 16 * q.
-constexpr int kGemmChunk = 8;                    // blocks per stage
-constexpr int kGemmBufs = 3;                     // LDS stage buffers
-constexpr int kGemmStageBytes = kGemmChunk * 512 + kGemmChunk * 64;
+// A workgroup of 8 waves takes 16 RT rows x 16 CG CW columns, CW = 8 / KG: wave
+// (wn, kg) sums its 16 CG columns over BPW of every stage's SB = KG BPW blocks, and
+// the k-groups' sums meet in LDS at the end in a fixed order. Per stage each
+// wave copies RT SB / 8 fragments (1 KB each, in operand order), 1 KB of weights
+// and 128 B of scales into LDS (global_load_lds), into a ring of SLOTS stages.
+//
+// Bound: MFMA and VALU issue, which hardly overlap here (a probe of independent
+// chains, two waves per SIMD: 16 MFMAs 253 cycles, 64 fmas 158, both 380): K4096
+// x N11008 at 512 rows needs 29 us of it. 16 CG columns per fragment read keep
+// the LDS reads (CG = 2: 85 B per cycle and CU, which bound the kernel) below
+// that; KG splits K over the waves rather than the tile, so that few rows and
+// columns per workgroup still fill the CUs. kk_common_gemm has the times.
+template <int RT, int CG, int KG, int BPW, int SLOTS>
+struct CgShape {
+    static constexpr int CW = 8 / KG;                                   // column waves
+    static constexpr int Cols = 16 * CG * CW;
+    static constexpr int SB = KG * BPW;                                 // blocks per stage
+    static constexpr int ABytes = RT * SB * 1024;
+    static constexpr int StageBytes = ABytes + 8 * 1024 + 1024;         // + weights + scales
+    static constexpr int ACopies = RT * SB / 8;                         // per wave
+    static constexpr int LdsBytes = SLOTS * StageBytes;
+    static_assert(Cols * SB == 512 && CG % 2 == 0, "8 KB of weights per stage, whole 32-column tiles");
+    static_assert(RT * SB % 8 == 0 && LdsBytes <= 160 * 1024 && ACopies <= 8, "stage");
+    static constexpr int RP = RT * CG * 8 * 1024 <= LdsBytes ? RT : RT * CG * 4 * 1024 <= LdsBytes ? RT / 2 : RT / 4;
+    static_assert(RP >= 1 && RP * CG * 8 * 1024 <= LdsBytes, "k-group exchange");
+};
 
-__device__ __forceinline__ void gemm_lds_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("" ::: "memory");
+template <int RT, int CG, int KG, int BPW, int SLOTS>
+__device__ __forceinline__ void cg_copy_stage(const uint8_t *w, const uint8_t *scales, const uint8_t *frags, int blocks,
+                                              int np, int row_tile0, int col_tile0, int wid, int lane, int stage) {
+    using S = CgShape<RT, CG, KG, BPW, SLOTS>;
+    extern __shared__ __attribute__((aligned(16))) uint8_t cg_lds[];
+    uint8_t *buf = cg_lds + (stage % SLOTS) * S::StageBytes;
+    const int b0 = stage * S::SB;
+#pragma unroll
+    for (int t = 0; t < S::ACopies; ++t) {
+        const int c = wid + 8 * t, i = c / S::SB, j = c % S::SB;        // row tile, block
+        __builtin_amdgcn_global_load_lds(frags + (static_cast<size_t>(row_tile0 + i) * blocks + b0 + j) * 1024 + lane * 16,
+                                         buf + c * 1024, 16, 0, 0);
+    }
+    constexpr int kPer = S::SB / 2;                                     // 1 KB weight copies per column tile
+    const int ct = wid / kPer, part = wid % kPer;
+    __builtin_amdgcn_global_load_lds(w + (static_cast<size_t>(col_tile0 + ct) * blocks + b0) * 512 + part * 1024 + lane * 16,
+                                     buf + S::ABytes + wid * 1024, 16, 0, 0);
+    // scales [block][column]: bytes 128 wid .. +127 of the stage's 1 KB
+    constexpr int kRow = 2 * S::Cols;                                   // bytes per block
+    if (lane < 8) {
+        const int pos = wid * 128 + lane * 16, b = pos / kRow, off = pos % kRow;
+        __builtin_amdgcn_global_load_lds(scales + (static_cast<size_t>(b0 + b) * np + col_tile0 * 32) * 2 + off,
+                                         buf + S::ABytes + 8 * 1024 + wid * 128, 16, 0, 0);
+    }
 }
 
-// KS = 2 doubles the waves: wave 4h + g takes row group g over K half h
-// (its own staging ring); the halves' sums meet in LDS and are added in a
-// fixed order.
-template <int KS>
-__global__ __launch_bounds__(256 * KS) void common_gemm(const uint8_t *__restrict__ w, const int8_t *__restrict__ tiled,
-                                                       const float *__restrict__ row_scales, float *__restrict__ y,
-                                                       int rows, int defined_rows, int kp, int n, int np) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds_all[KS * kGemmBufs * kGemmStageBytes];
+template <int RT, int CG, int KG, int BPW, int SLOTS>
+__global__ __launch_bounds__(512, (SLOTS * (RT * KG * BPW + 9) <= 80 ? 4 : 2)) void common_gemm(const uint8_t *__restrict__ w, const uint8_t *__restrict__ frags,
+                                                   const float *__restrict__ row_scales, float *__restrict__ y,
+                                                   int rows, int blocks, int n, int np, int col_groups, int per_xcd,
+                                                   int total) {
+    using S = CgShape<RT, CG, KG, BPW, SLOTS>;
+    typedef float float4v __attribute__((ext_vector_type(4)));
+    extern __shared__ __attribute__((aligned(16))) uint8_t cg_lds[];
+    const int idx = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;        // contiguous ranges per XCD
+    if (idx >= total) return;                                           // whole workgroup, before any barrier
+    const int row_groups = total / col_groups;
+    const int cg = idx / row_groups, rg = idx - cg * row_groups;        // one column group's rows share its weights in L2
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-    const int wid = wave & 3, half = wave >> 2;
-    uint8_t *const stage_lds = lds_all + half * kGemmBufs * kGemmStageBytes;
-    const int tile = blockIdx.x;
-    const int row0 = 32 * wid;
-    const bool active = row0 < defined_rows;
-    const int blocks = kp >> 5;
-    const int chunks = blocks / kGemmChunk / KS;   // per K half (kp % (256 * KS) == 0)
-    const int chunk0 = half * chunks;
-    const int pairs = blocks / 2;
-    const uint8_t *scales = w + static_cast<size_t>(np) * kp / 2;
+    const int wid = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int wn = wid % S::CW, kg = wid / S::CW;
     const int q = lane >> 4, c16 = lane & 15;
+    const int row_tile0 = rg * RT, col_tile0 = cg * (S::Cols / 32);     // 16-row and 32-column tiles
+    const int stages = blocks / S::SB;
+    const uint8_t *scales = w + static_cast<size_t>(np) * blocks * 16;  // after the np * kp / 2 weight bytes
 
-    // copies of stage c into buffer c % 3: wave w takes blocks 2w, 2w+1 (1 KB
-    // of weights) and their scales (lanes 0..7: block 2w + lane/4, 16 B each)
-    auto copy_stage = [&](int c) {
-        const int cc = chunk0 + min(c, chunks - 1);        // past the end: a copy nobody reads
-        uint8_t *buf = stage_lds + (c % kGemmBufs) * kGemmStageBytes;
-        const int b0 = cc * kGemmChunk + 2 * wid;
-        __builtin_amdgcn_global_load_lds(w + (static_cast<size_t>(tile) * blocks + b0) * 512 + lane * 16,
-                                         buf + wid * 1024, 16, 0, 0);
-        const int sl = min(lane, 7);                       // lanes 8.. repeat lane 7's copy
-        const uint8_t *ssrc = scales + (static_cast<size_t>(b0 + sl / 4) * np + tile * 32) * 2 + (sl % 4) * 16;
-        if (lane < 8) __builtin_amdgcn_global_load_lds(ssrc, buf + kGemmChunk * 512 + wid * 128, 16, 0, 0);
-    };
-    // activation operands of stage c: [row tile][block pair] as uint4
-    const int8_t *abase = tiled + (static_cast<size_t>(row0 / 16) * pairs * 64 + lane) * 16;
-    auto load_a = [&](int c, uint4 (&a)[2][kGemmChunk / 2]) {
-        const int cc = chunk0 + min(c, chunks - 1);
+    float4v acc[RT][CG];
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < RT; ++i)
 #pragma unroll
-            for (int p = 0; p < kGemmChunk / 2; ++p)
-                a[i][p] = *reinterpret_cast<const uint4 *>(abase + (static_cast<size_t>(i) * pairs +
-                                                                    cc * (kGemmChunk / 2) + p) * 64 * 16);
-    };
-    auto widen = [](uint32_t wd) -> long {
-        const uint32_t ev = (wd << 4) & 0xf0f0f0f0u, od = wd & 0xf0f0f0f0u;
-        const uint32_t lo = __builtin_amdgcn_perm(od, ev, 0x05010400u);   // K 0..3
-        const uint32_t hi = __builtin_amdgcn_perm(od, ev, 0x07030602u);   // K 4..7
-        return static_cast<long>((static_cast<unsigned long>(hi) << 32) | lo);
-    };
+        for (int h = 0; h < CG; ++h) acc[i][h] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
 
-    float acc[2][2][4];
+    for (int s = 0; s < min(SLOTS - 1, stages); ++s)
+        cg_copy_stage<RT, CG, KG, BPW, SLOTS>(w, scales, frags, blocks, np, row_tile0, col_tile0, wid, lane, s);
+    for (int s = 0; s < stages; ++s) {
+        // this wave's copies of stage s landed (with three slots those of s + 1
+        // may be in flight), then every wave's; all reads of the buffer filled
+        // next are done
+        if (SLOTS == 3 && s + 1 < stages) __builtin_amdgcn_s_waitcnt(0x0F70 | (S::ACopies + 2));
+        else __builtin_amdgcn_s_waitcnt(0x0F70);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+        if (s + SLOTS - 1 < stages)
+            cg_copy_stage<RT, CG, KG, BPW, SLOTS>(w, scales, frags, blocks, np, row_tile0, col_tile0, wid, lane,
+                                                  s + SLOTS - 1);
+        const uint8_t *buf = cg_lds + (s % SLOTS) * S::StageBytes;
+        // every operand read, then MFMA m + kAhead beside the fmas of MFMA m (left to
+        // itself the compiler pairs each MFMA with its own fmas and waits for it)
+        constexpr int kB = RT * CG, kM = BPW * kB, kAhead = kM < 6 ? kM : 6;
+        kk::half8 b[BPW][CG], a[BPW][RT];
+        float d[BPW][CG];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+        for (int jj = 0; jj < BPW; ++jj) {
+            const int j = BPW * kg + jj;
+            // 32-column tiles of the stage: [tile][block][column % 16][column / 16][16 bytes]
+            const uint8_t *wb = buf + S::ABytes + (wn * (CG / 2) * S::SB + j) * 512 + c16 * 32 + 4 * q;
+            const uint16_t *sc = reinterpret_cast<const uint16_t *>(buf + S::ABytes + 8 * 1024 + j * 2 * S::Cols) +
+                                 wn * 16 * CG + c16;
+            uint32_t nib[CG];
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.0f;
-    const int32x4 zero = {0, 0, 0, 0};
-
-    uint4 a_cur[2][kGemmChunk / 2], a_next[2][kGemmChunk / 2];
-    // issue order: copies 0, A 0, copies 1; then per step c: A c+1, copies c+2.
-    // At the top of step c only copies c+1 (2 per wave) may still be in flight.
-    copy_stage(0);
-    if (active) load_a(0, a_next);
-    copy_stage(1);
-    for (int c = 0; c < chunks; ++c) {
-        __builtin_amdgcn_s_waitcnt(0x0F70 | 2);            // vmcnt(2): all but copies c+1
-        gemm_lds_barrier();                                // every wave's copies of c landed,
-                                                           // and reads of buffer (c-1)%3 are done
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int p = 0; p < kGemmChunk / 2; ++p) a_cur[i][p] = a_next[i][p];
-        if (active) load_a(c + 1, a_next);
-        copy_stage(c + 2);
-        if (!active) continue;
-        const uint8_t *buf = stage_lds + (c % kGemmBufs) * kGemmStageBytes;
-#pragma unroll
-        for (int j = 0; j < kGemmChunk; ++j) {
-            const uint32_t w0 = *reinterpret_cast<const uint32_t *>(buf + j * 512 + c16 * 32 + 4 * q);
-            const uint32_t w1 = *reinterpret_cast<const uint32_t *>(buf + j * 512 + c16 * 32 + 16 + 4 * q);
-            const uint16_t *sc = reinterpret_cast<const uint16_t *>(buf + kGemmChunk * 512 + j * 64);
-            const float d0 = kk::half_bits_to_float(sc[c16]) * 0.0625f;
-            const float d1 = kk::half_bits_to_float(sc[16 + c16]) * 0.0625f;
-            const long b0 = widen(w0), b1 = widen(w1);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const uint4 v = a_cur[i][j / 2];
-                const long a = (j & 1) ? static_cast<long>((static_cast<unsigned long>(v.w) << 32) | v.z)
-                                       : static_cast<long>((static_cast<unsigned long>(v.y) << 32) | v.x);
-                const int32x4 p0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b0, zero, 0, 0, 0);
-                const int32x4 p1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b1, zero, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    acc[i][0][r] = fmaf(static_cast<float>(p0[r]), d0, acc[i][0][r]);
-                    acc[i][1][r] = fmaf(static_cast<float>(p1[r]), d1, acc[i][1][r]);
-                }
+            for (int h = 0; h < CG; ++h) {                              // columns 16 h + c16 of the wave
+                nib[h] = *reinterpret_cast<const uint32_t *>(wb + (h / 2) * S::SB * 512 + 16 * (h % 2));
+                d[jj][h] = kk::half_bits_to_float(sc[16 * h]);
+                asm("" : "+v"(d[jj][h]));                               // a plain F32 fma below: v_fma_mix issues at half its rate
             }
+#pragma unroll
+            for (int i = 0; i < RT; ++i) a[jj][i] = reinterpret_cast<const kk::half8 *>(buf)[(j + i * S::SB) * 64 + lane];
+            // signed nibble + 8 is the nibble with its top bit flipped
+#pragma unroll
+            for (int h = 0; h < CG; ++h) b[jj][h] = kk::q4_dword_halves(nib[h] ^ 0x88888888u);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float4v p[kM];
+#pragma unroll
+        for (int m = 0; m < kM + kAhead; ++m) {
+            if (m < kM) {
+                const float4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                p[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[m / kB][m % kB / CG], b[m / kB][m % CG], zero, 0, 0, 0);
+            }
+            if (m >= kAhead) {
+                const int o = m - kAhead, i = o % kB / CG, h = o % CG;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[i][h][r] = fmaf(p[o][r], d[o / kB][h], acc[i][h][r]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
-    __builtin_amdgcn_s_waitcnt(0);                         // the trailing copies land before exit
-    if (KS > 1) {
-        // half 1 hands its sums to half 0 through the (now idle) staging LDS
-        gemm_lds_barrier();
-        float4 *xfer = reinterpret_cast<float4 *>(lds_all);     // [group][i*2+j][lane]
-        if (half == 1 && active) {
+    // the k-groups' sums meet in LDS, RP row tiles at a time; every wave adds
+    // (in k-group order) and stores its share of the 16 x 16 tiles
+    constexpr int kTiles = S::CW * S::RP * CG;                          // per pass
+    float4v *xfer = reinterpret_cast<float4v *>(cg_lds);
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+    for (int i0 = 0; i0 < RT; i0 += S::RP) {
+        __syncthreads();                                                // the ring, or the pass before, is read
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    xfer[(wid * 4 + i * 2 + j) * 64 + lane] =
-                        make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
-        }
+        for (int i = 0; i < S::RP; ++i)
+#pragma unroll
+            for (int h = 0; h < CG; ++h) xfer[((kg * S::CW + wn) * S::RP * CG + i * CG + h) * 64 + lane] = acc[i0 + i][h];
         __syncthreads();
-        if (half == 1) return;
-        if (active) {
+        for (int t = wid; t < kTiles; t += 8) {
+            float4v v = xfer[t * 64 + lane];
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int o = 1; o < KG; ++o) v += xfer[(o * kTiles + t) * 64 + lane];
+            const int tn = t / (S::RP * CG), i = t / CG % S::RP, h = t % CG;
+            const int col = col_tile0 * 32 + (tn * CG + h) * 16 + c16;
+            const int row0 = (row_tile0 + i0 + i) * 16 + 4 * q;
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const float4 v = xfer[(wid * 4 + i * 2 + j) * 64 + lane];
-                    acc[i][j][0] += v.x;
-                    acc[i][j][1] += v.y;
-                    acc[i][j][2] += v.z;
-                    acc[i][j][3] += v.w;
-                }
+            for (int r = 0; r < 4; ++r)
+                if (row0 + r < rows && col < n) y[static_cast<size_t>(row0 + r) * n + col] = v[r] * row_scales[(row0 + r) * 16];
         }
     }
-    if (!active) return;
-    const int col[2] = {tile * 32 + c16, tile * 32 + 16 + c16};
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = row0 + 16 * i + 4 * q + r;
-            if (row >= rows) continue;
-            const float s = row_scales[row * 16];
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                if (col[j] < n) y[static_cast<size_t>(row) * n + col[j]] = acc[i][j][r] * s;
-        }
+}
+
+struct CgArgs {
+    const uint8_t *w, *frags;
+    const float *row_scales;
+    float *y;
+    int rows, blocks, n, np;
+};
+
+template <int RT, int CG, int KG, int BPW, int SLOTS>
+hipError_t launch_common_gemm(const CgArgs &a, hipStream_t stream) {
+    using S = CgShape<RT, CG, KG, BPW, SLOTS>;
+    const hipError_t rc = kk::opt_in_lds(reinterpret_cast<const void *>(&common_gemm<RT, CG, KG, BPW, SLOTS>), S::LdsBytes);
+    if (rc != hipSuccess) return rc;
+    const int col_groups = (a.n + S::Cols - 1) / S::Cols;
+    const int total = col_groups * ((a.rows + 16 * RT - 1) / (16 * RT));
+    const int per_xcd = (total + 7) / 8;
+    hipLaunchKernelGGL((common_gemm<RT, CG, KG, BPW, SLOTS>), dim3(per_xcd * 8), dim3(512), S::LdsBytes, stream, a.w, a.frags,
+                       a.row_scales, a.y, a.rows, a.blocks, a.n, a.np, col_groups, per_xcd, total);
+    return hipGetLastError();
 }
 
 } // namespace
@@ -638,18 +655,19 @@ extern "C" int kk_common_quant_pair(const void *x, int x_f16, int k, int kp, voi
 }
 
 extern "C" int kk_common_quant_rows(const void *x, int x_f16, int k, int kp, int rows, int defined_rows,
-                                    void *values, void *params, void *tiled, hipStream_t stream) {
-    if (!x || !values || !params || !tiled || k <= 0 || kp < k || kp % 256 != 0 || rows <= 0 ||
-        defined_rows < rows || defined_rows % 32 != 0)
+                                    size_t chunk_stride, void *values, void *params, void *frags, hipStream_t stream) {
+    if (!x || !values || !params || !frags || k <= 0 || kp < k || kp % 256 != 0 || rows <= 0 ||
+        defined_rows < rows || defined_rows % 32 != 0 || (reinterpret_cast<uintptr_t>(values) & 7) || (chunk_stride & 7) ||
+        (reinterpret_cast<uintptr_t>(frags) & 15))
         return hipErrorInvalidValue;
     if (x_f16)
-        hipLaunchKernelGGL(common_quant_rows<true>, dim3(defined_rows), dim3(kRowThreads), 0, stream, x, x_f16, k, kp,
-                           rows, static_cast<int8_t *>(values), static_cast<float *>(params),
-                           static_cast<int8_t *>(tiled));
+        hipLaunchKernelGGL(common_quant_rows<true>, dim3(defined_rows), dim3(kRowThreads), 0, stream, x, k, kp, rows,
+                           chunk_stride, static_cast<int8_t *>(values), static_cast<float *>(params),
+                           static_cast<_Float16 *>(frags));
     else
-        hipLaunchKernelGGL(common_quant_rows<false>, dim3(defined_rows), dim3(kRowThreads), 0, stream, x, x_f16, k,
-                           kp, rows, static_cast<int8_t *>(values), static_cast<float *>(params),
-                           static_cast<int8_t *>(tiled));
+        hipLaunchKernelGGL(common_quant_rows<false>, dim3(defined_rows), dim3(kRowThreads), 0, stream, x, k, kp, rows,
+                           chunk_stride, static_cast<int8_t *>(values), static_cast<float *>(params),
+                           static_cast<_Float16 *>(frags));
     return hipGetLastError();
 }
 
@@ -687,24 +705,38 @@ extern "C" int kk_common_gemv(const void *w0, float *y0, const void *w1, float *
     return hipGetLastError();
 }
 
-extern "C" int kk_common_gemm(const void *w, const void *tiled, const void *row_scales, float *y, int rows,
-                              int defined_rows, int kp, int n, int np, hipStream_t stream) {
-    // kp % 256 == 0 also makes the block count a multiple of the GEMM's ring depth
-    if (!w || !tiled || !row_scales || !y || rows <= 0 || rows > 128 || defined_rows < rows ||
-        defined_rows % 32 != 0 || defined_rows > 128 || kp % 256 != 0 || np % 256 != 0 || n > np ||
-        (reinterpret_cast<uintptr_t>(w) & 255) != 0 || (reinterpret_cast<uintptr_t>(tiled) & 15) != 0)
+// Tiles, and their times per workgroup and K block fitted to the sweep below (us;
+// with one resident per CU, and with two where LDS allows). Measured, K4096 x
+// N11008 at 32 / 128 / 512 / 1024 rows: 128 x 64 tile 30 / 32 / 94 / 187 us, 64 x
+// 128 34 / 35 / 75 / 140, 32 x 64 13 / 29 / 90 / 201, 32 x 32 17 / 48 / 174 / 385;
+// K4096 x N4096 29 / 31 / 34 / 64, 34 / 34 / 35 / 52, 13 / 14 / 36 / 78, 9 / 18 /
+// 64 / 151. (Before: chunks of 128 rows on the int8 MFMA, 36 us each at N11008.)
+extern "C" int kk_common_gemm(const void *w, const void *frags, const void *row_scales, float *y, int rows, int kp, int n,
+                              int np, int cus, hipStream_t stream) {
+    if (!w || !frags || !row_scales || !y || rows <= 0 || kp <= 0 || kp % 256 != 0 || np % 256 != 0 || n > np ||
+        cus <= 0 || (reinterpret_cast<uintptr_t>(w) & 255) != 0 || (reinterpret_cast<uintptr_t>(frags) & 15) != 0)
         return hipErrorInvalidValue;
-    const int tiles = (n + 31) / 32;
-    const uint8_t *wb = static_cast<const uint8_t *>(w);
-    const int8_t *tb = static_cast<const int8_t *>(tiled);
-    const float *rs = static_cast<const float *>(row_scales);
-    // two K halves per tile when Kp splits into whole stages (and the tiles
-    // alone would leave compute units idle)
-    if (kp % 512 == 0 && tiles < 1024)
-        hipLaunchKernelGGL(common_gemm<2>, dim3(tiles), dim3(512), 0, stream, wb, tb, rs, y, rows, defined_rows, kp,
-                           n, np);
-    else
-        hipLaunchKernelGGL(common_gemm<1>, dim3(tiles), dim3(256), 0, stream, wb, tb, rs, y, rows, defined_rows, kp,
-                           n, np);
-    return hipGetLastError();
+    const CgArgs a = {static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(frags),
+                      static_cast<const float *>(row_scales), y, rows, kp / 32, n, np};
+    static const struct { int rows, cols, stage; double one, two; } kAll[] = {
+        {128, 64, 8, 0.235, 0.0}, {64, 128, 4, 0.255, 0.39}, {32, 64, 8, 0.095, 0.145}, {32, 32, 16, 0.062, 0.0}};
+    int pick = 0;
+    double best = 0.0;
+    for (int i = 0; i < 4; ++i) {
+        if (a.blocks % kAll[i].stage != 0) continue;
+        const long wgs = static_cast<long>((n + kAll[i].cols - 1) / kAll[i].cols) * ((rows + kAll[i].rows - 1) / kAll[i].rows);
+        const double cost = wgs <= cus             ? kAll[i].one
+                            : kAll[i].two == 0.0 ? kAll[i].one * static_cast<double>((wgs + cus - 1) / cus)
+                                                 : kAll[i].two * std::max(1.0, static_cast<double>(wgs) / (2 * cus));
+        if (best == 0.0 || cost < best) {
+            best = cost;
+            pick = i;
+        }
+    }
+    switch (pick) {
+    case 0: return launch_common_gemm<8, 4, 8, 1, 2>(a, stream);
+    case 1: return launch_common_gemm<4, 2, 2, 2, 3>(a, stream);
+    case 2: return launch_common_gemm<2, 2, 4, 2, 3>(a, stream);
+    default: return launch_common_gemm<2, 2, 8, 2, 3>(a, stream);
+    }
 }

@@ -319,3 +319,23 @@ print("NOT REJECTED", flush=True)
     assert "NOT REJECTED" not in proc.stdout
     assert proc.returncode == -signal.SIGABRT, (proc.returncode, proc.stderr[-400:])
     assert "invalid argument" in proc.stderr
+
+
+# Each GEMM tile (128 x 64, 64 x 128, 32 x 64, 32 x 32), with rows and columns that end inside
+# one, and calls of more rows than are quantized at a time (512).
+@pytest.mark.parametrize("k,n,m", [(256, 4033, 509), (256, 11000, 500), (256, 2048, 70), (512, 1000, 40), (33, 70, 513),
+                                   (768, 300, 1100)])
+@pytest.mark.parametrize("type_", [F32, F16], ids=["f32", "f16"])
+def test_gemm_tiles(gpu, oracle, k, n, m, type_):
+    case = Case(oracle, k, n)
+    x = oracle.fixture_input(k, m, 1)
+    if type_ == F16:
+        x = x.astype(np.float16).astype(np.float32)
+    y = case.run(kl.CommonQ4Workspace(), x, m, type_)
+    kp, _ = oracle.common_dims(k, n)
+    qa = np.empty((m, k), np.float32)
+    for first in range(0, m, 128):
+        rows = min(128, m - first)
+        values, params = oracle.common_quant_rows(x[first:first + rows], k, rows, 128)
+        qa[first:first + rows] = values.reshape(128, kp)[:rows, :k].astype(np.float32) * params.reshape(128, 16)[:rows, :1]
+    check_against(oracle, y, case.w, qa, f"m={m}")
