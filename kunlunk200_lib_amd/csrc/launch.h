@@ -78,6 +78,11 @@ int kk_q4_stream_gemv_pair_swiglu(const void *w_gate, const void *w_up, const fl
 int kk_dense_mfma_gemv(int type, const void *w, const float *x, float *y, int k, int n, int batch,
                        hipStream_t stream);
 
+// F32 weights at any batch (meant for more than 16 columns) on fp32 MFMA, 64
+// columns per pass over W; 16-byte aligned weights and activations; `cus`
+// decides whether two workgroups share a CU.
+int kk_f32_gemm(const void *w, const float *x, float *y, int k, int n, int batch, int cus, hipStream_t stream);
+
 // Elementwise F32 op over `count` values: 0 add, 1 multiply (b of b_count
 // values repeated), 2 silu, 3 rms_norm of each `width` row (eps =
 // parameter), 4 scale by parameter.

@@ -82,6 +82,12 @@ bool q4_split_route(const void * w, int k, int batch) {
     return q4_mfma_batch(batch, !whole || (k % 256 == 0 && ((uintptr_t)w & 15) == 0));
 }
 
+// F32 weights above the single-pass GEMV's 16 columns (K4096 x N4096 at 17
+// columns: 28.4 us in passes of 16, 18.4 us).
+bool f32_gemm_route(int type, const void * w, const void * x, int batch) {
+    return type == 0 && batch > 16 && dense_mfma_batch(16) && (((uintptr_t)w | (uintptr_t)x) & 15) == 0;
+}
+
 // Columns of one pass of batches above the small-batch kernels and off the GEMM.
 int gemv_chunk(int type) { return type == 2 && kk::tuning_or(kk::kQ4MfmaMax, 16) >= 16 ? 32 : 16; }
 
@@ -154,6 +160,13 @@ static void dispatch_dense(Kernel::Impl & impl, detail::DeviceContext & ctx, int
                     const void * x, int k, int n, int batch, WeightType type) {
     const bool gemm = (type == WeightType::q4_0 || (type == WeightType::f16 && ((uintptr_t)w & 15) == 0)) &&
                       batch >= gemm_min_batch() && ((uintptr_t)x & 15) == 0;
+    if (kk::f32_gemm_route((int)type, w, x, batch)) {
+        detail::check_hip((hipError_t)kk_f32_gemm(w, static_cast<const float *>(x), static_cast<float *>(y), k, n, batch,
+                                                  ctx.cus, ctx.stream),
+                          "kk_f32_gemm");
+        impl.route = "f32_mfma_gemv";
+        return;
+    }
     const int chunk = kk::gemv_chunk((int)type);
     if (!gemm && batch > chunk) {
         // batches between the small-batch kernels and the GEMM: chunks of 32

@@ -125,6 +125,9 @@ extern "C" int kunlun_matmul_noalloc(int device, void *y, const void *w, const v
         const size_t need = kk_gemm_workspace_bytes(k, n, batch);
         if (need > kScratchBytes) return too_large(need);
         rc = static_cast<hipError_t>(kk_gemm(type, w, xf, yf, k, n, batch, d.ptr, s, &taken));
+    } else if (kk::f32_gemm_route(type, w, x, batch)) {
+        taken = "f32_mfma_gemv";
+        rc = static_cast<hipError_t>(kk_f32_gemm(w, xf, yf, k, n, batch, d.cus, s));
     } else {
         // kunlun_matmul's small-batch routes, in its chunks of columns, in
         // stream order on the one array
