@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
+#include <type_traits>
 
 namespace {
 
@@ -1149,6 +1150,298 @@ __global__ __launch_bounds__(128 * CW) void q4_lds_gemm(const uint8_t *__restric
     }
 }
 
+// ---------------------------------------------------------------------------
+// q4_wide_gemm: Q4_0, K % 256 == 0, 16-byte aligned weights, for calls with enough
+// 256-row (KG = 1) or 128-row (KG = 2) tiles of 256 weight rows.
+//
+// Eight waves, each a 128 x 64 wave tile (128 accumulators): KG = 1, waves 0..3
+// and 4..7 take the two row halves of 256 rows over every K32 step; KG = 2, the
+// two K32 blocks of every K64 step of 128 rows, summed at the end. Against the
+// 128 x 48 wave tile this reads a third less of the activations from LDS per MFMA
+// (64 against 85 B per cycle and CU) and decodes as much per MFMA.
+//
+// Measured (us; the 128 x 48 tiles before): K4096, 2048 rows: pair 2 x N11008 460 -> 371
+// (996 TFLOP/s), N4096 85 -> 73 and K11008 x N4096 219 -> 174 (1060) with KG = 2; a
+// library fp16 GEMM without the decode takes 203 and 177 for N11008 and K11008 x
+// N4096. What bounds it: MFMA issue and the clock under it (256 tiles run a step in
+// 1.0 us, 24 tiles in 0.75, against 0.45 of MFMA at 2.25 GHz).
+//
+// One barrier per step, with everything a step's MFMAs need in registers before
+// it: while row tile i is multiplied, its fragment for the next step is read
+// behind it, and the next step's four weight fragments are decoded between the
+// row tiles from bytes read at the step's start. The accumulators are tied with
+// inline asm: with the builtin the compiler moves them between registers every
+// step and spills.
+//
+// A ring of four activation steps (16 KiB: KG = 1 256 rows x K32, KG = 2 128 rows x
+// K64) and two weight super-stages (256 K: 144 bytes per row, 36 copies of 1 KiB
+// and 4 empty ones, so that every wave issues five).
+constexpr int kWdABytes = 16 * 1024, kWdBBytes = 40 * 1024;
+constexpr int kWdRing = 4 * kWdABytes + 2 * kWdBBytes;              // 144 KiB
+constexpr int kWdFixStride = 68;                                     // floats per row of a wave's 64 x 64 correction tile
+constexpr int kWdFix = 256 * kTinyMaskWords * 4 + 8 * 64 * kWdFixStride * 4;
+constexpr int kWdLds = (kWdRing > kWdFix ? kWdRing : kWdFix) + 256 * 4;
+static_assert(kWdLds <= 160 * 1024, "LDS");
+
+template <int KG>
+struct WdShape {
+    static constexpr int Rows = 256 / KG;                            // activation rows per tile
+    static constexpr int StepK = 32 * KG;
+    static constexpr int Super = 8 / KG;                             // steps per weight super-stage
+    // weight copies issued in step i of a super-stage, the first of them
+    static constexpr int copies(int i) { return KG == 1 ? (i <= 4 ? 1 : 0) : i == 0 ? 3 : i == 1 ? 2 : 0; }
+    static constexpr int first(int i) { return KG == 1 ? i : i == 0 ? 0 : 3; }
+    // copies that may be in flight at the top of step i: those issued after the
+    // activations of step i + 1 (two steps ago)
+    static constexpr int in_flight(int i) { return 2 + copies((i + Super - 1) % Super); }
+};
+
+__device__ __forceinline__ void wd_copy_a(_Float16 *a_tile, int a_extent, const uint32_t (&a_off)[2], int wid, int soff, int buf) {
+    extern __shared__ __align__(16) uint8_t wd_lds[];
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(a_tile, 0, a_extent, 0x00020000);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) uint8_t *)wd_lds + buf * kWdABytes +
+                                                 (wid + 8 * t) * 1024, 16, a_off[t], soff, 0, 0);
+}
+// weight copy wid + 8t of super-stage p (PAIR: below 18 the gate rows, then the up rows)
+template <bool PAIR>
+__device__ __forceinline__ void wd_copy_b(uint8_t *b_tile, uint8_t *b_tile2, int b_extent, uint32_t off, int wid, int t, int p) {
+    extern __shared__ __align__(16) uint8_t wd_lds[];
+    const int i = wid + 8 * t;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(PAIR && i >= 18 ? b_tile2 : b_tile, 0, b_extent, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) uint8_t *)wd_lds + 4 * kWdABytes +
+                                             (p & 1) * kWdBBytes + i * 1024, 16, off, p * kQlRowPair, 0, 0);
+}
+__device__ __forceinline__ void wd_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+}
+
+template <bool PAIR, int KG>
+__global__ __launch_bounds__(512) void q4_wide_gemm(const uint8_t *__restrict__ w, const uint8_t *__restrict__ w2,
+                                                    const _Float16 *__restrict__ x16, const float *__restrict__ row_inv,
+                                                    float *__restrict__ y, int m_rows, int m_pad, int n_rows, int k_pad,
+                                                    int k, int m_tiles, int tiles, int tiles_per_xcd) {
+    using S = WdShape<KG>;
+    extern __shared__ __align__(16) uint8_t wd_lds[];
+    constexpr int kOut = PAIR ? 128 : 256;                           // output columns per tile
+    const int bid = blockIdx.x;
+    const int tile = (bid % kXcds) * tiles_per_xcd + bid / kXcds;
+    if (tile >= tiles) return;                                       // whole workgroup, before any barrier
+    const int nt = tile / m_tiles, mt = tile - nt * m_tiles;
+    const int m0 = mt * S::Rows, n0 = nt * kOut;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wid = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int grp = wid >> 2, wn = wid & 3;                          // row half (KG = 1) or k-group; columns
+    const int g = lane >> 4, c16 = lane & 15;
+    const uint32_t row_bytes = static_cast<uint32_t>(k / 32 * 18);
+    const int steps = k / S::StepK;
+
+    // activation copy i: 1 KiB of whole rows of a step (16 of 64 B, KG = 2 8 of 128 B); chunk
+    // c of row r sits at position c ^ (r / 4) % 4 (KG = 2 c ^ (r / 2) % 8): an operand
+    // read's 16 rows then cover all banks
+    constexpr int kChunks = S::StepK / 8;
+    auto swizzle = [](int r) { return KG == 1 ? (r >> 2) & 3 : (r >> 1) & 7; };
+    _Float16 *const a_tile = const_cast<_Float16 *>(x16 + static_cast<size_t>(m0) * k_pad);
+    const int a_extent = min(S::Rows, m_pad - m0) * k_pad * 2;       // rows past m_pad read as zero
+    uint32_t a_off[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int r = 64 / kChunks * (wid + 8 * t) + lane / kChunks, pos = lane % kChunks;
+        a_off[t] = static_cast<uint32_t>(r * k_pad * 2 + 16 * (pos ^ swizzle(r)));
+    }
+    // weight copies: 16-byte chunks of [row][144 B]; rows past n repeat the last row, the
+    // four empty copies lie past the extent (zeros, no memory access)
+    constexpr int kRows = PAIR ? 128 : 256;
+    const int b_extent = min(kRows, n_rows - n0) * static_cast<int>(row_bytes);
+    uint8_t *const b_tile = const_cast<uint8_t *>(w + static_cast<size_t>(n0) * row_bytes);
+    uint8_t *const b_tile2 = const_cast<uint8_t *>(w2 + static_cast<size_t>(n0) * row_bytes);
+    uint32_t b_off[5];
+#pragma unroll
+    for (int t = 0; t < 5; ++t) {
+        const int i = wid + 8 * t;
+        const int q = (PAIR && i >= 18 ? i - 18 : i) * 64 + lane;
+        const int row = min(q / 9, kRows - 1), chunk = q - q / 9 * 9;
+        b_off[t] = i < 36 ? static_cast<uint32_t>(min(n0 + row, n_rows - 1) - n0) * row_bytes + 16 * chunk : 0x80000000u;
+    }
+    const uint32_t a_read = static_cast<uint32_t>(((KG == 1 ? 128 * grp : 0) + c16) * (S::StepK * 2) +
+                                                  16 * ((KG == 1 ? g : 4 * grp + g) ^ swizzle(c16)));
+    // this wave's 64 LDS weight rows (PAIR: 32 gate rows from 32 wn, 32 up rows from 128 + 32 wn)
+    const uint32_t b_read = static_cast<uint32_t>(4 * kWdABytes + ((PAIR ? 32 : 64) * wn + c16) * kQlRowPair);
+    // KG = 2: k-group 0 has the even blocks, 1 the odd ones; nibble dword g starts 2 bytes
+    // into a dword in an even block, on one in an odd block
+    const uint32_t odd = KG == 2 ? static_cast<uint32_t>(grp) : 0u;
+    const uint32_t raw_read = b_read + 4 * g + (KG == 2 ? 20 * odd : 0), scale_read = b_read + (KG == 2 ? 18 * odd : 0);
+
+    float4v acc[8][4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    bool tiny = false;   // set once this lane decoded a block with a subnormal scale
+    half8 a[8], b[2][4];
+    uint32_t lo[4], hi[4], sb[4];
+
+    // the weight bytes of step J of the super-stage in buffer offset `buf`: the dwords around
+    // nibble dword g of each column's block, and its scale
+    auto read_raw = [&](auto jc, uint32_t buf) {
+        constexpr int J = decltype(jc)::value;
+        const uint8_t *bl = wd_lds + raw_read + buf, *sl = wd_lds + scale_read + buf;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int row = PAIR ? (c >> 1) * 128 + (c & 1) * 16 : c * 16;
+            const int off = row * kQlRowPair + 18 * J * KG;
+            sb[c] = *reinterpret_cast<const uint16_t *>(sl + off);
+            const uint32_t *p = reinterpret_cast<const uint32_t *>(bl + off + (KG == 1 && (J & 1) ? 2 : 0));
+            lo[c] = p[0];
+            if (KG == 2 || (J & 1) == 0) hi[c] = p[1];
+        }
+    };
+    auto decode = [&](auto jc, int c) {
+        constexpr int J = decltype(jc)::value;
+        const uint32_t nib = KG == 2 ? (odd ? lo[c] : __builtin_amdgcn_alignbyte(hi[c], lo[c], 2))
+                             : (J & 1) ? lo[c] : __builtin_amdgcn_alignbyte(hi[c], lo[c], 2);
+        note_tiny_scale(sb[c], tiny);
+        return decode_q4_scaled(nib, sb[c]);
+    };
+    auto read_a = [&](auto jc, int i) {
+        constexpr int J = decltype(jc)::value;
+        return *reinterpret_cast<const half8 *>(wd_lds + (J & 3) * kWdABytes + a_read + i * 16 * (S::StepK * 2));
+    };
+    // Step s (I = s % Super): issues the copies of step s + 3 (and a share of the next
+    // super-stage), multiplies step s, reads and decodes step s + 1. What lies past
+    // K is copied from the next rows or as zeros, and not used.
+    uint32_t buf = 0;
+    auto step = [&](auto ic, int s) {
+        constexpr int I = decltype(ic)::value, C = I & 1;
+        using Next = std::integral_constant<int, (I + 1) % S::Super>;
+        __builtin_amdgcn_s_waitcnt(0x0F70 | S::in_flight(I));
+        wd_barrier();
+#pragma unroll
+        for (int t = 0; t < S::copies(I); ++t)
+            wd_copy_b<PAIR>(b_tile, b_tile2, b_extent, b_off[S::first(I) + t], wid, S::first(I) + t, s / S::Super + 1);
+        wd_copy_a(a_tile, a_extent, a_off, wid, (s + 3) * (S::StepK * 2), (I + 3) & 3);
+        read_raw(Next{}, buf);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc[i][c]) : "v"(a[i]), "v"(b[C][c]));
+            __builtin_amdgcn_sched_barrier(0);
+            a[i] = read_a(std::integral_constant<int, (I + 1) & 3>{}, i);
+            if (i >= 2 && i < 6) b[C ^ 1][i - 2] = decode(Next{}, i - 2);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+#pragma unroll
+    for (int t = 0; t < 5; ++t) wd_copy_b<PAIR>(b_tile, b_tile2, b_extent, b_off[t], wid, t, 0);
+#pragma unroll
+    for (int s = 0; s < 3; ++s) wd_copy_a(a_tile, a_extent, a_off, wid, s * (S::StepK * 2), s);
+    __builtin_amdgcn_s_waitcnt(0x0F70 | 4);
+    wd_barrier();
+    using Zero = std::integral_constant<int, 0>;
+    read_raw(Zero{}, 0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a[i] = read_a(Zero{}, i);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) b[0][c] = decode(Zero{}, c);
+    for (int s0 = 0; s0 < steps; s0 += S::Super) {
+        const uint32_t here = ((s0 / S::Super) & 1) * kWdBBytes;
+        buf = here;
+        step(std::integral_constant<int, 0>{}, s0);
+        step(std::integral_constant<int, 1>{}, s0 + 1);
+        step(std::integral_constant<int, 2>{}, s0 + 2);
+        if constexpr (KG == 1) {
+            step(std::integral_constant<int, 3 % S::Super>{}, s0 + 3);
+            step(std::integral_constant<int, 4 % S::Super>{}, s0 + 4);
+            step(std::integral_constant<int, 5 % S::Super>{}, s0 + 5);
+            step(std::integral_constant<int, 6 % S::Super>{}, s0 + 6);
+        }
+        buf = kWdBBytes - here;                                      // the last step reads the next super-stage
+        step(std::integral_constant<int, S::Super - 1>{}, s0 + S::Super - 1);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);                              // the trailing copies land,
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");               // the last MFMAs' results too (asm: no automatic wait)
+    const bool any_tiny = __syncthreads_or(tiny) != 0;               // workgroup-uniform; the ring is idle
+    float *scale_lds = reinterpret_cast<float *>(wd_lds + kWdLds - 256 * 4);
+    if (threadIdx.x < S::Rows) scale_lds[threadIdx.x] = row_inv[min(m0 + static_cast<int>(threadIdx.x), m_pad - 1)] * 8.0f;
+    if constexpr (KG == 2) {
+        // each k-group hands the other half its row tiles, and finishes its own half
+        float4v *xfer = reinterpret_cast<float4v *>(wd_lds);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                float4v &mine = grp ? acc[i][c] : acc[i + 4][c];
+                xfer[((wid * 4 + i) * 4 + c) * kWave + lane] = mine;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float4v other = xfer[(((wid ^ 4) * 4 + i) * 4 + c) * kWave + lane];
+                acc[i][c] = (grp ? acc[i + 4][c] : acc[i][c]) + other;
+            }
+    }
+    __syncthreads();
+    // the 64-row halves this wave finishes: KG = 1 both of its 128 rows, KG = 2 rows 64 grp ..
+    constexpr int kHalves = KG == 1 ? 2 : 1;
+    const int row_base = KG == 1 ? 128 * grp : 64 * grp;
+    if (any_tiny) {
+        // Q4_0 blocks with subnormal scales, corrected in F32 as q4_lds_gemm does, a wave
+        // working on its own 64 x 64 sums in LDS
+        uint32_t *tiny_masks = reinterpret_cast<uint32_t *>(wd_lds);
+        float *fix = reinterpret_cast<float *>(wd_lds + 256 * kTinyMaskWords * 4) + wid * 64 * kWdFixStride;
+        auto wrow_at = [&](int j) -> const uint8_t * {               // LDS weight row j
+            const int up = PAIR && j >= 128, r = n0 + (up ? j - 128 : j);
+            return r < n_rows ? (up ? w2 : w) + static_cast<size_t>(r) * row_bytes : nullptr;
+        };
+        build_tiny_masks_rows<8>(256, k / 32, wrow_at, tiny_masks);
+        auto lds_row = [&](int it) { return PAIR ? (it >> 5) * 128 + 32 * wn + (it & 31) : 64 * wn + it; };
+#pragma unroll
+        for (int h = 0; h < kHalves; ++h) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) fix[(16 * i + 4 * g + r) * kWdFixStride + 16 * c + c16] = acc[4 * h + i][c][r];
+            tiny_fix_items<2>(0, 1, 64, k / 32, [&](int it) { return tiny_masks + lds_row(it) * kTinyMaskWords; },
+                              [&](int it) { return wrow_at(lds_row(it)); },
+                              [&](int) { return x16 + static_cast<size_t>(min(m0 + row_base + 64 * h + lane, m_pad - 1)) * k_pad; },
+                              [&](int it) { return fix + lane * kWdFixStride + it; });
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[4 * h + i][c][r] = fix[(16 * i + 4 * g + r) * kWdFixStride + 16 * c + c16];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4 * kHalves; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = row_base + 16 * i + 4 * g + r, m = m0 + row;
+            if (m >= m_rows) continue;
+            const float sc = scale_lds[row];
+            float *dst = y + static_cast<size_t>(m) * n_rows;
+#pragma unroll
+            for (int c = 0; c < (PAIR ? 2 : 4); ++c) {
+                const int n = n0 + (PAIR ? 32 : 64) * wn + 16 * c + c16;
+                const float v = PAIR ? kk::swiglu_value(acc[i][c][r] * sc, acc[i][(c + 2) & 3][r] * sc) : acc[i][c][r] * sc;
+                if (n < n_rows) __builtin_nontemporal_store(v, dst + n);
+            }
+        }
+}
+
 struct GemmPlan {
     int m_pad, k_pad, m_tiles, bn, n_tiles;
     size_t x16_bytes, row_inv_bytes;
@@ -1195,24 +1488,27 @@ struct QlTile {
 
 // The candidate with the smallest estimated time: whole rounds of tiles over
 // the CUs x tile work, with penalties for the LDS activation reads per MFMA
-// (~1/WN) and the weight decode per MFMA (~1/BM). The kGemmTile knob
-// (KUNLUN_GEMM_TILE=BMxWN, e.g. 128x48) forces a candidate.
+// (~1/WN) and the weight decode per MFMA (~1/BM); for the wide tiles (256 and 128
+// rows x 256 weight rows, WN = 64) the factors measured against those: at K4096 a
+// round takes 57 us of 128x48, 43 of 64x32, 113 of 256x64 and 66 of 128x64. The
+// kGemmTile knob (KUNLUN_GEMM_TILE=BMxWN, e.g. 128x48) forces a candidate.
 QlTile pick_ql_tile(int batch, int n, bool pair) {
-    static const QlTile kAll[] = {{128, 48}, {128, 32}, {64, 64}, {64, 32}};
-    auto allowed = [](const QlTile &) { return true; };
+    static const QlTile kAll[] = {{128, 48}, {128, 32}, {64, 64}, {64, 32}, {256, 64}, {128, 64}};
     const int forced = kk::tuning(kk::kGemmTile);
     if (forced > 0)
         for (const QlTile &t : kAll)
-            if (t.bm * 1000 + t.wn == forced && allowed(t)) return t;
+            if (t.bm * 1000 + t.wn == forced) return t;
     const long cus = device_cus();
     QlTile pick = {128, 32};
     double best = 0.0;
     for (const QlTile &t : kAll) {
-        if (!allowed(t)) continue;
         const long out = pair ? 2 * t.wn : 4 * t.wn;
         const long tiles = (static_cast<long>(batch) + t.bm - 1) / t.bm * ((n + out - 1) / out);
         const long rounds = (tiles + cus - 1) / cus;
-        const double cost = static_cast<double>(rounds) * t.bm * 4 * t.wn * (1.0 + 16.0 / t.wn) * (1.0 + 32.0 / t.bm);
+        const double factor = t.bm == 256                ? 1.26
+                              : t.bm * t.wn == 128 * 64 ? 1.44
+                                                        : (1.0 + 16.0 / t.wn) * (1.0 + 32.0 / t.bm);
+        const double cost = static_cast<double>(rounds) * t.bm * 4 * t.wn * factor;
         if (best == 0.0 || cost < best) {
             best = cost;
             pick = t;
@@ -1238,6 +1534,22 @@ hipError_t launch_ql_gemm(const void *w, const void *w2, const _Float16 *x16, co
     return hipGetLastError();
 }
 
+template <bool PAIR, int KG>
+hipError_t launch_wide(const void *w, const void *w2, const _Float16 *x16, const float *row_inv, float *y, int batch,
+                       int n, int k, int k_pad, hipStream_t stream) {
+    const hipError_t rc = kk::opt_in_lds(reinterpret_cast<const void *>(&q4_wide_gemm<PAIR, KG>), kWdLds);
+    if (rc != hipSuccess) return rc;
+    const int rows = WdShape<KG>::Rows, out = PAIR ? 128 : 256;
+    const int m_tiles = (batch + rows - 1) / rows;
+    const int tiles = m_tiles * ((n + out - 1) / out);
+    const int tiles_per_xcd = (tiles + kXcds - 1) / kXcds;
+    const int m_pad = static_cast<int>(round_up(static_cast<size_t>(batch), kBM));
+    hipLaunchKernelGGL((q4_wide_gemm<PAIR, KG>), dim3(tiles_per_xcd * kXcds), dim3(512), kWdLds, stream,
+                       static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(w2), x16, row_inv, y, batch, m_pad, n,
+                       k_pad, k, m_tiles, tiles, tiles_per_xcd);
+    return hipGetLastError();
+}
+
 template <bool PAIR>
 hipError_t launch_ql(const void *w, const void *w2, const _Float16 *x16, const float *row_inv, float *y, int batch,
                      int n, int k, int k_pad, hipStream_t stream) {
@@ -1250,6 +1562,8 @@ hipError_t launch_ql(const void *w, const void *w2, const _Float16 *x16, const f
         if constexpr (PAIR) return launch_ql_gemm<64, 32, true, true>(w, w2, x16, row_inv, y, batch, n, k, k_pad, stream);
         else return launch_ql_gemm<64, 16, false, true, 8>(w, w2, x16, row_inv, y, batch, n, k, k_pad, stream);
     }
+    if (t.bm == 256) return launch_wide<PAIR, 1>(w, w2, x16, row_inv, y, batch, n, k, k_pad, stream);
+    if (t.bm == 128 && t.wn == 64) return launch_wide<PAIR, 2>(w, w2, x16, row_inv, y, batch, n, k, k_pad, stream);
     if (t.bm == 128 && t.wn == 48) return launch_ql_gemm<128, 48, PAIR>(w, w2, x16, row_inv, y, batch, n, k, k_pad, stream);
     return hipErrorInvalidValue;
 }
