@@ -14,12 +14,15 @@
 //    |value| <= 65504 for any F16 scale; undone in the epilogue) and writes
 //    both to double-buffered LDS; eight waves run v_mfma_f32_32x32x16_f16
 //    tiles, two k-groups of four. Epilogue: y = acc * row_inv[m] * 8.
+//    A call with too few tiles for the chip splits K (pick_ranges) and
+//    gemm_split_sum adds the ranges' partial sums in order.
 // Precision: fp16 inputs, f32 accumulation: relative error ~2^-11 per
 // product (the fp16-MFMA tolerance of the path is 2e-3 relative).
 #include "device_common.h"
 #include "launch.h"
 #include "lds_opt_in.h"
 #include "tuning.h"
+#include <kunlun/k200_c.h>
 
 #include <algorithm>
 #include <cstdio>
@@ -332,7 +335,11 @@ __device__ void tiny_scale_dots(const uint8_t *wrow, const uint32_t *mask, int b
 //
 // Tiles are numbered m-major and dealt to the 8 XCDs in contiguous ranges,
 // so the workgroups of one XCD share few activation row tiles in its L2.
+//
+// A call with few tiles splits K (pick_ranges): range_tiles tiles per range of
+// range_k values, `part` = partial sums [range][matrix][m_rows][part_stride].
 constexpr int kLdsA = kBM * kLdsStride;
+__host__ __device__ inline int part_stride(int n) { return (n + 3) & ~3; }
 #ifndef KUNLUN_GEMM_STAGES
 #define KUNLUN_GEMM_STAGES 2
 #endif
@@ -358,7 +365,8 @@ __global__ __launch_bounds__(kGemmThreads) void mfma_gemm(const uint8_t *__restr
                                                          const float *__restrict__ row_inv,
                                                          float *__restrict__ y, int m_rows, int n_rows,
                                                          int k, int k_pad, size_t w_bytes, int n_tiles,
-                                                         int tiles, int tiles_per_xcd) {
+                                                         int tiles, int tiles_per_xcd, int range_tiles,
+                                                         int range_k, float *__restrict__ part) {
     static_assert(BN == 64 || BN == 128, "tile N");
     static_assert(!PAIR || BN == 128, "a pair tile holds 64 rows of each matrix");
     constexpr int kLdsB = BN * kLdsStride;
@@ -367,8 +375,20 @@ __global__ __launch_bounds__(kGemmThreads) void mfma_gemm(const uint8_t *__restr
     extern __shared__ __align__(16) _Float16 lds[];      // 2 x (A tile + B tile)
 
     const int bid = blockIdx.x;
-    const int tile = (bid % kXcds) * tiles_per_xcd + bid / kXcds;
+    int tile = (bid % kXcds) * tiles_per_xcd + bid / kXcds;
     if (tile >= tiles) return;                           // whole workgroup, before any barrier
+    const size_t row_bytes = F16W ? static_cast<size_t>(k) * 2 : static_cast<size_t>(k >> 5) * 18;
+    // this workgroup's K range (all of K without a split): from here on k, the
+    // weight rows and the activations begin there
+    const int range = tile / range_tiles;
+    tile -= range * range_tiles;
+    const int k0 = range * range_k;
+    k = min(range_k, k - k0);
+    const size_t w_skip = F16W ? static_cast<size_t>(k0) * 2 : static_cast<size_t>(k0 >> 5) * 18;
+    w += w_skip;
+    w2 += w_skip;
+    w_bytes -= w_skip;
+    x16 += k0;
     const int mt = tile / n_tiles;
     const int nt = tile - mt * n_tiles;
 
@@ -380,8 +400,7 @@ __global__ __launch_bounds__(kGemmThreads) void mfma_gemm(const uint8_t *__restr
     const int m0 = mt * kBM;
     const int n0 = nt * kOutN;
     const int blocks = k >> 5;
-    const size_t row_bytes = F16W ? static_cast<size_t>(k) * 2 : static_cast<size_t>(blocks) * 18;
-    const int steps = k_pad / kBK;                       // multiple of kStages
+    const int steps = (k + kKAlign - 1) / kKAlign * kStages;   // whole main-loop iterations
 
     // A: 16-byte chunks tid + 512 i of the 128 x 128 tile (16 chunks per row)
     const _Float16 *a_src[4];
@@ -589,6 +608,23 @@ __global__ __launch_bounds__(kGemmThreads) void mfma_gemm(const uint8_t *__restr
                 }
             }
         }
+    }
+    if (part) {   // split K: this range's plain sums, for gemm_split_sum
+        const int stride = part_stride(n_rows);
+#pragma unroll
+        for (int it = 0; it < 2; ++it)
+#pragma unroll
+            for (int jt = 0; jt < kNT; ++jt) {
+                const int n = n0 + (PAIR ? wn * 32 : wn * (BN / 2) + jt * 32) + (lane & 31);
+                float *dst = part + static_cast<size_t>(PAIR ? 2 * range + jt : range) * m_rows * stride + n;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int m = m0 + wm * 64 + it * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                    const float v = acc[it][jt][r] + red[(((sw * 2 + it) * kNT + jt) * 16 + r) * kWave + lane];
+                    if (m < m_rows && n < n_rows) dst[static_cast<size_t>(m) * stride] = v;
+                }
+            }
+        return;
     }
     if constexpr (PAIR) {
         const int n = n0 + wn * 32 + (lane & 31);
@@ -864,15 +900,26 @@ __global__ __launch_bounds__(128 * CW) void q4_lds_gemm(const uint8_t *__restric
                                                          const _Float16 *__restrict__ x16,
                                                          const float *__restrict__ row_inv, float *__restrict__ y,
                                                          int m_rows, int n_rows, int k_pad, int stages,
-                                                         uint32_t row_bytes, int m_tiles, int tiles, int tiles_per_xcd) {
+                                                         uint32_t row_bytes, int m_tiles, int tiles, int tiles_per_xcd,
+                                                         int range_tiles, int range_stages, float *__restrict__ part) {
     using S = QlShape<BM, WN, PAIR, LONG, CW>;
     constexpr int kOut = PAIR ? S::BN / 2 : S::BN;             // output columns per tile
     constexpr int kQlThreads = S::Threads;
     extern __shared__ __align__(16) uint8_t ql_lds[];
 
     const int bid = blockIdx.x;
-    const int tile = (bid % kXcds) * tiles_per_xcd + bid / kXcds;
+    int tile = (bid % kXcds) * tiles_per_xcd + bid / kXcds;
     if (tile >= tiles) return;                                  // whole workgroup, before any barrier
+    // this workgroup's K range of whole stages (all of K without a split): from here
+    // on the stages, the weight rows and the activations begin there
+    const int range = tile / range_tiles;
+    tile -= range * range_tiles;
+    const int stage0 = range * range_stages;
+    stages = min(range_stages, stages - stage0);
+    const uint32_t w_skip = static_cast<uint32_t>(stage0) * (S::KS / 32 * 18);
+    w += w_skip;
+    w2 += w_skip;
+    x16 += static_cast<size_t>(stage0) * S::KS;
     const int nt = tile / m_tiles;
     const int mt = tile - nt * m_tiles;
     const int m0 = mt * BM, n0 = nt * kOut;
@@ -896,7 +943,7 @@ __global__ __launch_bounds__(128 * CW) void q4_lds_gemm(const uint8_t *__restric
     // A copy i: rows 4i .. 4i+3 of the tile, lane -> row 4i + lane/16, LDS
     // position lane%16, which holds chunk (lane%16) ^ (row & 15).
     _Float16 *const a_tile = const_cast<_Float16 *>(x16 + static_cast<size_t>(m0) * k_pad);
-    const int a_extent = BM * k_pad * 2;
+    const int a_extent = (BM * k_pad - stage0 * S::KS) * 2;
     uint32_t a_off[S::ACopiesPerWave];
 #pragma unroll
     for (int t = 0; t < S::ACopiesPerWave; ++t) {
@@ -907,7 +954,7 @@ __global__ __launch_bounds__(128 * CW) void q4_lds_gemm(const uint8_t *__restric
     // B copy i: 16-byte chunks 64c .. 64c+63 (c = i, or i - HalfCopies for the
     // up rows of PAIR) of the [row][144 B] stage-pair bytes, 9 chunks per row.
     constexpr int kRows = PAIR ? S::BN / 2 : S::BN;             // weight rows per matrix and tile
-    const int b_extent = min(kRows, n_rows - n0) * static_cast<int>(row_bytes);
+    const int b_extent = min(kRows, n_rows - n0) * static_cast<int>(row_bytes) - static_cast<int>(w_skip);
     uint8_t *const b_tile = const_cast<uint8_t *>(w + static_cast<size_t>(n0) * row_bytes);
     uint8_t *const b_tile2 = const_cast<uint8_t *>(w2 + static_cast<size_t>(n0) * row_bytes);
     uint32_t b_off[S::BCopiesPerWave];
@@ -1079,7 +1126,7 @@ __global__ __launch_bounds__(128 * CW) void q4_lds_gemm(const uint8_t *__restric
     __syncthreads();                                            // ring idle
     constexpr int kTs = S::TileStride;
     float *tile_lds = reinterpret_cast<float *>(ql_lds);
-    if (threadIdx.x < BM) scale_lds[threadIdx.x] = row_inv_raw * 8.0f;
+    if (threadIdx.x < BM) scale_lds[threadIdx.x] = part ? 1.0f : row_inv_raw * 8.0f;
     if (kh == 1) {
 #pragma unroll
         for (int rg = 0; rg < S::RG; ++rg)
@@ -1095,7 +1142,7 @@ __global__ __launch_bounds__(128 * CW) void q4_lds_gemm(const uint8_t *__restric
         // of each B tile row j.
         static_assert(S::XferBytes + S::BN * kTinyMaskWords * 4 <= S::RingBytes, "mask space");
         uint32_t *tiny_masks = reinterpret_cast<uint32_t *>(ql_lds + S::XferBytes);
-        const int nblocks = static_cast<int>(row_bytes / 18);
+        const int nblocks = stages * (S::KS / 32);
         build_tiny_masks_rows<S::Waves>(S::BN, nblocks, [&](int j) -> const uint8_t * {
             const int h = PAIR ? j / (S::BN / 2) : 0, jr = PAIR ? j % (S::BN / 2) : j;
             return n0 + jr < n_rows ? (h ? w2 : w) + static_cast<size_t>(n0 + jr) * row_bytes : nullptr;
@@ -1128,6 +1175,19 @@ __global__ __launch_bounds__(128 * CW) void q4_lds_gemm(const uint8_t *__restric
     __syncthreads();
     // PAIR: output column c is SiLU(tile column c) * (tile column BN/2 + c)
     constexpr int kQuads = kOut / 4;
+    if (part) {   // split K: this range's plain sums, for gemm_split_sum
+        const int stride = part_stride(n_rows);
+        const size_t plane = static_cast<size_t>(m_rows) * stride;
+        float *const base = part + static_cast<size_t>(PAIR ? 2 * range : range) * plane;
+        for (int i = threadIdx.x; i < BM * S::BN / 4; i += kQlThreads) {
+            const int row = i / (S::BN / 4), q = i - row * (S::BN / 4);
+            const int up = PAIR && q >= kQuads, m = m0 + row, n = n0 + 4 * (up ? q - kQuads : q);
+            if (m >= m_rows || n >= n_rows) continue;   // columns past n (below the stride) are not read
+            *reinterpret_cast<float4v *>(base + (up ? plane : 0) + static_cast<size_t>(m) * stride + n) =
+                *reinterpret_cast<const float4v *>(tile_lds + row * kTs + 4 * q);
+        }
+        return;
+    }
     const bool vec = (n_rows & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
     for (int i = threadIdx.x; i < BM * kQuads; i += kQlThreads) {
         const int row = i / kQuads, q = i - row * kQuads;
@@ -1442,9 +1502,49 @@ __global__ __launch_bounds__(512) void q4_wide_gemm(const uint8_t *__restrict__ 
         }
 }
 
+// y[m][n] = the ranges' partial sums, added in range order, times the row's scale
+// (PAIR: SiLU(gate) * up of the two matrices' values). Four columns per thread.
+constexpr int kSumThreads = 256;
+constexpr int kMinUnitsSaved = 3;              // see pick_ranges
+
+template <bool PAIR>
+__global__ __launch_bounds__(kSumThreads) void gemm_split_sum(const float *__restrict__ part,
+                                                              const float *__restrict__ row_inv, float wscale,
+                                                              float *__restrict__ y, int m_rows, int n_rows, int ranges) {
+    const int stride = part_stride(n_rows), quads = stride >> 2;
+    const size_t i = static_cast<size_t>(blockIdx.x) * kSumThreads + threadIdx.x;
+    if (i >= static_cast<size_t>(m_rows) * quads) return;
+    const int m = static_cast<int>(i / quads), n = 4 * static_cast<int>(i - static_cast<size_t>(m) * quads);
+    const size_t plane = static_cast<size_t>(m_rows) * stride;
+    const float *src = part + 4 * i;
+    const float sc = row_inv[m] * wscale;
+    float4v a = {0.0f, 0.0f, 0.0f, 0.0f}, b = a;
+#pragma unroll 4
+    for (int r = 0; r < ranges; ++r) {
+        a += *reinterpret_cast<const float4v *>(src + static_cast<size_t>(PAIR ? 2 * r : r) * plane);
+        if (PAIR) b += *reinterpret_cast<const float4v *>(src + static_cast<size_t>(2 * r + 1) * plane);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) a[t] = PAIR ? kk::swiglu_value(a[t] * sc, b[t] * sc) : a[t] * sc;
+    float *dst = y + static_cast<size_t>(m) * n_rows + n;
+    if ((n_rows & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
+        *reinterpret_cast<float4v *>(dst) = a;
+    } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            if (n + t < n_rows) dst[t] = a[t];
+    }
+}
+
 struct GemmPlan {
     int m_pad, k_pad, m_tiles, bn, n_tiles;
     size_t x16_bytes, row_inv_bytes;
+};
+
+// K ranges of a call: how many, and the 256-K units of each.
+struct KRanges {
+    int ranges, units;
+    size_t part_bytes;
 };
 
 // Tile N: 128 (fewer LDS reads per MFMA) when that still gives every CU a
@@ -1462,17 +1562,56 @@ GemmPlan plan(int k, int n, int batch) {
     return p;
 }
 
-template <bool F16W, int BN, bool PAIR = false>
-hipError_t launch_gemm(const void *w, const void *w2, const _Float16 *x16, const float *row_inv, float *y, int batch,
-                       int n, int k, const GemmPlan &p, size_t w_bytes, hipStream_t stream) {
-    const hipError_t rc =
-        kk::opt_in_lds(reinterpret_cast<const void *>(&mfma_gemm<F16W, BN, PAIR>), gemm_lds_bytes<BN>());
-    if (rc != hipSuccess) return rc;
-    const int tiles = p.m_tiles * p.n_tiles;
-    const int tiles_per_xcd = (tiles + kXcds - 1) / kXcds;
-    hipLaunchKernelGGL((mfma_gemm<F16W, BN, PAIR>), dim3(tiles_per_xcd * kXcds), dim3(kGemmThreads),
-                       gemm_lds_bytes<BN>(), stream, static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(w2),
-                       x16, row_inv, y, batch, n, k, p.k_pad, w_bytes, p.n_tiles, tiles, tiles_per_xcd);
+int device_cus();
+
+// K ranges for `tiles` tiles of at most 128 rows (64 x 128 or 128 x 64 outputs each):
+// as many as the CUs hold in one round, of at least two units of 256; none where
+// the split would not take three units off every tile's serial loop (the summing
+// launch costs 2 - 4 us, a unit 1.1 - 2.2), nor for a forced tile. The partial sums
+// of one call, with the activations, stay within the no-allocation entry point's
+// scratch, so both entry points split alike (and a call that it refuses is not split).
+//
+// Without the split such a call leaves CUs idle and each tile's loop is a chain of
+// barriers and load latencies. us per call before / after: Q4_0 K5600 x N2999
+// b77 (47 tiles, 5 ranges) 52.1 / 21.7, K4096 x N4096 b64 (8 ranges) 26.0 / 15.6,
+// b128 (4) 27.3 / 18.3, b256 (2) 27.7 / 24.3, K11008 x N4096 b128 57.9 / 29.4,
+// K4096 x N11008 b64 (2) 26.4 / 21.8, K2048 x N4096 b64 16.4 / 14.0, K1280 x N4096
+// b100 13.7 / 13.4 (the line: 3 units saved; K1024 is not split); F16 K4096 x N4096
+// b64 32.1 / 18.5, b256 34.2 / 27.5.
+KRanges pick_ranges(const GemmPlan &p, int tiles, int k, int n, int batch, bool pair) {
+    const int units = (k + kKAlign - 1) / kKAlign;
+    KRanges r = {1, units, 0};
+    const size_t one = static_cast<size_t>(pair ? 2 : 1) * batch * part_stride(n) * 4;
+    const size_t fixed = p.x16_bytes + p.row_inv_bytes;
+    if (fixed >= KUNLUN_NOALLOC_SCRATCH_BYTES || tiles <= 0) return r;
+    const long room = static_cast<long>((KUNLUN_NOALLOC_SCRATCH_BYTES - fixed) / one);
+    const long want = std::min<long>(std::min<long>(device_cus() / tiles, units / 2), room);
+    if (want < 2) return r;
+    const int per = static_cast<int>((units + want - 1) / want);
+    if (units - per < kMinUnitsSaved) return r;
+    r.units = per;
+    r.ranges = (units + per - 1) / per;
+    r.part_bytes = r.ranges * one;
+    return r;
+}
+
+// Tiles of one K range: the LDS-copy kernel's 64 x 128, the register-staged
+// kernel's 128 x 64 (pair: 64 columns of each matrix in both).
+int range_tiles_ql(int n, int batch, bool pair) { return (batch + 63) / 64 * ((n + (pair ? 63 : 127)) / (pair ? 64 : 128)); }
+KRanges ranges_ql(const GemmPlan &p, int k, int n, int batch, bool pair) {
+    if (kk::tuning(kk::kGemmTile) > 0) return {1, k / 256, 0};
+    return pick_ranges(p, range_tiles_ql(n, batch, pair), k, n, batch, pair);
+}
+KRanges ranges_staged(const GemmPlan &p, int k, int n, int batch, bool pair) {
+    return pick_ranges(p, p.m_tiles * (pair ? (n + 63) / 64 : p.n_tiles), k, n, batch, pair);
+}
+
+template <bool PAIR>
+hipError_t launch_split_sum(const float *part, const float *row_inv, float wscale, float *y, int batch, int n, int ranges,
+                            hipStream_t stream) {
+    const size_t quads = static_cast<size_t>(batch) * (part_stride(n) / 4);
+    hipLaunchKernelGGL(gemm_split_sum<PAIR>, dim3(static_cast<unsigned>((quads + kSumThreads - 1) / kSumThreads)),
+                       dim3(kSumThreads), 0, stream, part, row_inv, wscale, y, batch, n, ranges);
     return hipGetLastError();
 }
 
@@ -1480,6 +1619,24 @@ int device_cus() {
     int device = 0;
     if (hipGetDevice(&device) != hipSuccess) return 256;
     return kk::cu_count(device);
+}
+
+template <bool F16W, int BN, bool PAIR = false>
+hipError_t launch_gemm(const void *w, const void *w2, const _Float16 *x16, const float *row_inv, float *y, float *part,
+                       int batch, int n, int k, const GemmPlan &p, const KRanges &kr, size_t w_bytes,
+                       hipStream_t stream) {
+    const hipError_t rc =
+        kk::opt_in_lds(reinterpret_cast<const void *>(&mfma_gemm<F16W, BN, PAIR>), gemm_lds_bytes<BN>());
+    if (rc != hipSuccess) return rc;
+    const int range_tiles = p.m_tiles * p.n_tiles, tiles = range_tiles * kr.ranges;
+    const int tiles_per_xcd = (tiles + kXcds - 1) / kXcds;
+    hipLaunchKernelGGL((mfma_gemm<F16W, BN, PAIR>), dim3(tiles_per_xcd * kXcds), dim3(kGemmThreads),
+                       gemm_lds_bytes<BN>(), stream, static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(w2),
+                       x16, row_inv, y, batch, n, k, p.k_pad, w_bytes, p.n_tiles, tiles, tiles_per_xcd, range_tiles,
+                       kr.units * kKAlign, kr.ranges > 1 ? part : nullptr);
+    const hipError_t launched = hipGetLastError();
+    if (launched != hipSuccess || kr.ranges == 1) return launched;
+    return launch_split_sum<PAIR>(part, row_inv, F16W ? 1.0f : 8.0f, y, batch, n, kr.ranges, stream);
 }
 
 struct QlTile {
@@ -1519,18 +1676,19 @@ QlTile pick_ql_tile(int batch, int n, bool pair) {
 
 template <int BM, int WN, bool PAIR, bool LONG = false, int CW = 4>
 hipError_t launch_ql_gemm(const void *w, const void *w2, const _Float16 *x16, const float *row_inv, float *y, int batch,
-                          int n, int k, int k_pad, hipStream_t stream) {
+                          int n, int k, int k_pad, hipStream_t stream, const KRanges *kr = nullptr, float *part = nullptr) {
     using S = QlShape<BM, WN, PAIR, LONG, CW>;
     hipError_t rc = kk::opt_in_lds(reinterpret_cast<const void *>(&q4_lds_gemm<BM, WN, PAIR, LONG, CW>), S::LdsBytes);
     if (rc != hipSuccess) return rc;
     const int out = PAIR ? S::BN / 2 : S::BN;
     const int m_tiles = (batch + BM - 1) / BM;
-    const int tiles = m_tiles * ((n + out - 1) / out);
+    const int range_tiles = m_tiles * ((n + out - 1) / out), tiles = range_tiles * (kr ? kr->ranges : 1);
     const int tiles_per_xcd = (tiles + kXcds - 1) / kXcds;
     const uint32_t row_bytes = static_cast<uint32_t>(k / 32 * 18);
+    const int stages = k / S::KS, range_stages = kr ? kr->units * (2 * kQlK / S::KS) : stages;
     hipLaunchKernelGGL((q4_lds_gemm<BM, WN, PAIR, LONG, CW>), dim3(tiles_per_xcd * kXcds), dim3(S::Threads), S::LdsBytes,
                        stream, static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(w2), x16, row_inv, y, batch,
-                       n, k_pad, k / S::KS, row_bytes, m_tiles, tiles, tiles_per_xcd);
+                       n, k_pad, stages, row_bytes, m_tiles, tiles, tiles_per_xcd, range_tiles, range_stages, part);
     return hipGetLastError();
 }
 
@@ -1552,7 +1710,15 @@ hipError_t launch_wide(const void *w, const void *w2, const _Float16 *x16, const
 
 template <bool PAIR>
 hipError_t launch_ql(const void *w, const void *w2, const _Float16 *x16, const float *row_inv, float *y, int batch,
-                     int n, int k, int k_pad, hipStream_t stream) {
+                     int n, int k, const GemmPlan &p, float *part, hipStream_t stream) {
+    const int k_pad = p.k_pad;
+    const KRanges kr = ranges_ql(p, k, n, batch, PAIR);
+    if (kr.ranges > 1) {   // few tiles: K split over workgroups, 64 x 128 tiles (as below)
+        hipError_t rc;
+        if constexpr (PAIR) rc = launch_ql_gemm<64, 32, true, true>(w, w2, x16, row_inv, y, batch, n, k, k_pad, stream, &kr, part);
+        else rc = launch_ql_gemm<64, 16, false, true, 8>(w, w2, x16, row_inv, y, batch, n, k, k_pad, stream, &kr, part);
+        return rc != hipSuccess ? rc : launch_split_sum<PAIR>(part, row_inv, 8.0f, y, batch, n, kr.ranges, stream);
+    }
     const QlTile t = pick_ql_tile(batch, n, PAIR);
     if (t.bm == 128 && t.wn == 32) return launch_ql_gemm<128, 32, PAIR>(w, w2, x16, row_inv, y, batch, n, k, k_pad, stream);
     if (t.bm == 64 && t.wn == 64) return launch_ql_gemm<64, 64, PAIR>(w, w2, x16, row_inv, y, batch, n, k, k_pad, stream);
@@ -1577,9 +1743,10 @@ bool ql_shape(int k, const void *w, const void *w2) {
 
 } // namespace
 
-extern "C" size_t kk_gemm_workspace_bytes(int k, int n, int batch) {
+extern "C" size_t kk_gemm_workspace_bytes(int k, int n, int batch, int pair) {
     const GemmPlan p = plan(k, n, batch);
-    return p.x16_bytes + p.row_inv_bytes;
+    return p.x16_bytes + p.row_inv_bytes + std::max(ranges_ql(p, k, n, batch, pair != 0).part_bytes,
+                                                    ranges_staged(p, k, n, batch, pair != 0).part_bytes);
 }
 
 extern "C" int kk_gemm(int type, const void *w, const float *x, float *y, int k, int n, int batch, void *workspace,
@@ -1593,17 +1760,19 @@ extern "C" int kk_gemm(int type, const void *w, const float *x, float *y, int k,
     char *ws = static_cast<char *>(workspace);
     _Float16 *x16 = reinterpret_cast<_Float16 *>(ws);
     float *row_inv = reinterpret_cast<float *>(ws + p.x16_bytes);
+    float *part = reinterpret_cast<float *>(ws + p.x16_bytes + p.row_inv_bytes);
     launch_x_to_f16(type == 2, x, batch, k, p.m_pad, p.k_pad, x16, row_inv, stream);
     hipError_t rc = hipGetLastError();
     if (rc != hipSuccess) return rc;
     const size_t w_bytes = type == 1 ? static_cast<size_t>(n) * k * 2 : static_cast<size_t>(n) * (k / 32) * 18;
     if (route) *route = type == 2 ? "q4_gemm_mfma" : "f16_gemm_mfma";
-    if (type == 2 && ql_shape(k, w, w)) return launch_ql<false>(w, w, x16, row_inv, y, batch, n, k, p.k_pad, stream);
+    if (type == 2 && ql_shape(k, w, w)) return launch_ql<false>(w, w, x16, row_inv, y, batch, n, k, p, part, stream);
+    const KRanges kr = ranges_staged(p, k, n, batch, false);
     if (type == 2)
-        return p.bn == 128 ? launch_gemm<false, 128>(w, w, x16, row_inv, y, batch, n, k, p, w_bytes, stream)
-                           : launch_gemm<false, 64>(w, w, x16, row_inv, y, batch, n, k, p, w_bytes, stream);
-    return p.bn == 128 ? launch_gemm<true, 128>(w, w, x16, row_inv, y, batch, n, k, p, w_bytes, stream)
-                       : launch_gemm<true, 64>(w, w, x16, row_inv, y, batch, n, k, p, w_bytes, stream);
+        return p.bn == 128 ? launch_gemm<false, 128>(w, w, x16, row_inv, y, part, batch, n, k, p, kr, w_bytes, stream)
+                           : launch_gemm<false, 64>(w, w, x16, row_inv, y, part, batch, n, k, p, kr, w_bytes, stream);
+    return p.bn == 128 ? launch_gemm<true, 128>(w, w, x16, row_inv, y, part, batch, n, k, p, kr, w_bytes, stream)
+                       : launch_gemm<true, 64>(w, w, x16, row_inv, y, part, batch, n, k, p, kr, w_bytes, stream);
 }
 
 extern "C" int kk_gemm_swiglu(int type, const void *w_gate, const void *w_up, const float *x, float *y, int k, int n,
@@ -1620,13 +1789,15 @@ extern "C" int kk_gemm_swiglu(int type, const void *w_gate, const void *w_up, co
     char *ws = static_cast<char *>(workspace);
     _Float16 *x16 = reinterpret_cast<_Float16 *>(ws);
     float *row_inv = reinterpret_cast<float *>(ws + p.x16_bytes);
+    float *part = reinterpret_cast<float *>(ws + p.x16_bytes + p.row_inv_bytes);
     launch_x_to_f16(type == 2, x, batch, k, p.m_pad, p.k_pad, x16, row_inv, stream);
     hipError_t rc = hipGetLastError();
     if (rc != hipSuccess) return rc;
     const size_t w_bytes = type == 1 ? static_cast<size_t>(n) * k * 2 : static_cast<size_t>(n) * (k / 32) * 18;
     if (route) *route = type == 2 ? "q4_gemm_swiglu_mfma" : "f16_gemm_swiglu_mfma";
     if (type == 2 && ql_shape(k, w_gate, w_up))
-        return launch_ql<true>(w_gate, w_up, x16, row_inv, y, batch, n, k, p.k_pad, stream);
-    if (type == 2) return launch_gemm<false, 128, true>(w_gate, w_up, x16, row_inv, y, batch, n, k, p, w_bytes, stream);
-    return launch_gemm<true, 128, true>(w_gate, w_up, x16, row_inv, y, batch, n, k, p, w_bytes, stream);
+        return launch_ql<true>(w_gate, w_up, x16, row_inv, y, batch, n, k, p, part, stream);
+    const KRanges kr = ranges_staged(p, k, n, batch, true);
+    if (type == 2) return launch_gemm<false, 128, true>(w_gate, w_up, x16, row_inv, y, part, batch, n, k, p, kr, w_bytes, stream);
+    return launch_gemm<true, 128, true>(w_gate, w_up, x16, row_inv, y, part, batch, n, k, p, kr, w_bytes, stream);
 }

@@ -17,9 +17,9 @@ int kk_dense_matmul(int type, const void *w, const float *x, float *y, int k, in
 
 
 // Prefill GEMM on fp16 MFMA for Q4_0 (type 2) and F16 (type 1) weights. The
-// workspace (kk_gemm_workspace_bytes) holds the fp16 activations and their
-// row scales.
-size_t kk_gemm_workspace_bytes(int k, int n, int batch);
+// workspace (kk_gemm_workspace_bytes) holds the fp16 activations, their row
+// scales and, where a call has few tiles, partial sums over K ranges.
+size_t kk_gemm_workspace_bytes(int k, int n, int batch, int pair);
 int kk_gemm(int type, const void *w, const float *x, float *y, int k, int n, int batch, void *workspace,
             hipStream_t stream, const char **route);
 

@@ -183,7 +183,7 @@ static void dispatch_dense(Kernel::Impl & impl, detail::DeviceContext & ctx, int
         return;
     }
     if (gemm) {
-        grow(id, ctx, impl.gemm_workspace, impl.gemm_workspace_size, kk_gemm_workspace_bytes(k, n, batch));
+        grow(id, ctx, impl.gemm_workspace, impl.gemm_workspace_size, kk_gemm_workspace_bytes(k, n, batch, 0));
         detail::check_hip((hipError_t)kk_gemm((int)type, w, static_cast<const float *>(x), static_cast<float *>(y), k,
                                               n, batch, impl.gemm_workspace, ctx.stream, &impl.route),
                           "kk_gemm");
@@ -339,7 +339,7 @@ void matmul_swiglu(Kernel & kernel, int id, void * y, const void * w_gate, const
     const bool f16_aligned = ((uintptr_t)w_gate & 15) == 0 && ((uintptr_t)w_up & 15) == 0;
     if ((type == WeightType::q4_0 || (type == WeightType::f16 && f16_aligned)) && batch >= gemm_min_batch() &&
         ((uintptr_t)x & 15) == 0) {
-        grow(id, ctx, impl.gemm_workspace, impl.gemm_workspace_size, kk_gemm_workspace_bytes(k, n, batch));
+        grow(id, ctx, impl.gemm_workspace, impl.gemm_workspace_size, kk_gemm_workspace_bytes(k, n, batch, 1));
         detail::check_hip((hipError_t)kk_gemm_swiglu((int)type, w_gate, w_up, static_cast<const float *>(x),
                                                      static_cast<float *>(y), k, n, batch, impl.gemm_workspace,
                                                      ctx.stream, &impl.route),

@@ -122,7 +122,7 @@ extern "C" int kunlun_matmul_noalloc(int device, void *y, const void *w, const v
     const char *taken = nullptr;
     const bool gemm = (type == 2 || (type == 1 && (wa & 15) == 0)) && batch >= kk::gemm_min_batch() && (xa & 15) == 0;
     if (gemm) {
-        const size_t need = kk_gemm_workspace_bytes(k, n, batch);
+        const size_t need = kk_gemm_workspace_bytes(k, n, batch, 0);
         if (need > kScratchBytes) return too_large(need);
         rc = static_cast<hipError_t>(kk_gemm(type, w, xf, yf, k, n, batch, d.ptr, s, &taken));
     } else if (kk::f32_gemm_route(type, w, x, batch)) {
