@@ -11,7 +11,8 @@
 // scale s_b (kk::fixed_point_digits), so sum_j q_j X_j is an exact int32 from
 // 24 v_dot8_i32_i4 per row and block, and y_r += float(S) * (d_rb * s_b) in F32.
 //
-// Work split: one workgroup per half tile (16 rows); the two halves of a tile
+// native_q4_gemv (one column, two on small matrices; native_q4_mfma below takes the rest):
+// one workgroup per half tile (16 rows); the two halves of a tile
 // run on the same XCD (workgroup i runs on XCD i % 8), so the second reads the
 // tile's cache lines from L2. The workgroup's waves take items of 16 K32
 // blocks in turn. In an item, lane l owns block 16i + l/4 and rows
@@ -36,7 +37,7 @@ constexpr int kNqDepth = 2;                 // items in flight per wave
 constexpr int kNqLanesPerBlock = 4;         // 4 lanes x 4 rows = one half tile
 constexpr int kNqItemBlocks = 64 / kNqLanesPerBlock;
 constexpr int kNqRows = 16;                 // rows per workgroup
-constexpr int kNqMaxColumns = 4;            // batch columns per launch
+constexpr int kNqMaxColumns = 2;            // batch columns per launch (more: native_q4_mfma)
 constexpr int kNqMaxPasses = 6;             // activation staging passes (8 values per thread each)
 constexpr size_t kNqLdsLimit = 64 * 1024;
 
@@ -265,6 +266,263 @@ hipError_t launch_passes(int passes, const uint8_t *w, const uint16_t *scales, c
     }
 }
 
+// ---------------------------------------------------------------------------
+// native_q4_mfma: more than one column on int8 MFMA (v_mfma_i32_16x16x32_i8, one K32
+// block per instruction), up to 5 columns per workgroup.
+//
+// The activations are the same 23-bit block fixed point, here as three signed
+// base-256 digits: the digits of all columns are the 16 operand columns of one
+// MFMA, so every block's digit sums are exact as above; each operand column
+// accumulates in F32 with the digit's weight in the block scale, and a column's
+// three sums meet at the end. (Three MFMAs per block for 16 columns, put together
+// per block, need half the VALU operations per column but took 17.6 and 45 us where
+// this takes 11 and 29, K4096 and K11008 x N4096 at 16 columns.)
+//
+// One workgroup per 32-row tile and column group, its 8 waves taking blocks in turn. Lane l reads, for
+// K group g = l / 16 and row quad u = (l % 16) / 2, the dwords (4 rows of one pair) of
+// pairs g + 8 (l & 1) and that + 4: 128 contiguous bytes of the tile's 512 per 32 lanes and
+// instruction. One exchange with the neighbour lane and byte permutes make them rows 2c
+// and 2c + 1 (c = l % 16) over the pairs g, g + 4, g + 8, g + 12; each nibble stays in the
+// high half of its byte (16 q). D of row set i: register r of lane l is row
+// 8 (l / 16) + 2 r + i, column l % 16.
+//
+// Bound by the CU: the decode, two conversions and a multiply-add per block sum and the
+// three loads per block keep a CU busy for about 90 cycles per block of a tile, so 128
+// tiles (N4096) leave half the chip idle. us per call before (dot products, 4 columns per pass)
+// / after: K4096 x N11008 4 columns 33.8 / 25.4, 16 columns 94 / 47; K4096 x N4096 4 columns
+// 22.5 / 20.6, 16 columns 53 / 26; K11008 x N4096 4 columns 48.5 / 30.5, 16 columns 151 / 44;
+// about 15 of each are the launch and the wait for the result. 16 waves per workgroup
+// take as long (K4096 x N11008: 27.8).
+constexpr int kNmWaves = 8, kNmThreads = 64 * kNmWaves;
+constexpr int kNmDepth = 4;                  // blocks in flight per wave
+constexpr int kNmMaxColumns = 5;             // 15 of the 16 operand columns
+constexpr int kNmChunkColumns = 512;         // activation blocks x columns of a chunk, at most
+constexpr int kNmGroups = kNmChunkColumns * 4 / kNmThreads;   // groups of 8 activations per thread and chunk
+constexpr int kNmStep = kNmWaves * kNmDepth;                  // blocks per chunk are a multiple of this
+constexpr int kNmPart = kNmWaves * 16 * 33 * 4;               // the waves' sums
+static_assert(kNmChunkColumns / kNmMaxColumns >= kNmStep, "a chunk of every column count");
+
+// Activation blocks in LDS at a time (100 bytes per block and column, 50 KiB at most).
+int nm_chunk(int blocks, int columns) {
+    return std::min(kNmChunkColumns / columns / kNmStep * kNmStep, (blocks + kNmStep - 1) / kNmStep * kNmStep);
+}
+
+typedef int int4v __attribute__((ext_vector_type(4)));
+typedef float float2a4 __attribute__((ext_vector_type(2), aligned(4)));
+
+// A barrier after this wave's LDS accesses that leaves its global loads in flight
+// (__syncthreads waits for those too).
+__device__ __forceinline__ void nm_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+template <bool F16X>
+__global__ __launch_bounds__(kNmThreads, 4) void native_q4_mfma(const uint8_t *__restrict__ w,
+                                                            const uint16_t *__restrict__ scales,
+                                                            const void *__restrict__ x, float *__restrict__ y, int k,
+                                                            int n, int batch, int columns, int chunk, int column_groups,
+                                                            int tiles) {
+    extern __shared__ uint4 lds4[];
+    // workgroup -> (tile, column group): all groups of a tile, one after the other, on XCD tile % 8
+    const int unit = blockIdx.x >> 3;
+    const int tile = (unit / column_groups) * 8 + (blockIdx.x & 7), c0 = unit % column_groups * columns;
+    if (tile >= tiles) return;                                 // whole workgroup: no barrier reached yet
+    x = static_cast<const uint8_t *>(x) + static_cast<size_t>(c0) * k * (F16X ? 2 : 4);
+    y += static_cast<size_t>(c0) * n;
+    columns = min(columns, batch - c0);
+    const int blocks = k >> 5;
+    const int jn = 3 * columns;                                // operand columns: digit * columns + column
+    uint2 *digits = reinterpret_cast<uint2 *>(lds4);           // [chunk][4][jn]
+    float *block_scale = reinterpret_cast<float *>(digits + static_cast<size_t>(chunk) * 4 * jn);   // [chunk][columns]
+    const int lane = threadIdx.x & (kk::kWave - 1);
+    const int wid = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int g = lane >> 4, c16 = lane & 15, odd = lane & 1;
+
+    const uint8_t *wl = w + static_cast<size_t>(tile) * blocks * 512 + 32 * (g + 8 * odd) + 4 * (c16 >> 1);
+    const uint16_t *sl = scales + static_cast<size_t>(tile) * blocks * 32 + 8 * g;
+    uint32_t raw[kNmDepth][2];
+    uint4 sc[kNmDepth];
+    auto load = [&](int s, int d) {                            // block wid + 8 s; past K: the last block
+        const int blk = min(wid + kNmWaves * s, blocks - 1);
+        raw[d][0] = *reinterpret_cast<const uint32_t *>(wl + static_cast<size_t>(blk) * 512);
+        raw[d][1] = *reinterpret_cast<const uint32_t *>(wl + static_cast<size_t>(blk) * 512 + 128);
+        sc[d] = *reinterpret_cast<const uint4 *>(sl + static_cast<size_t>(blk) * 32);
+    };
+
+    float acc[2][4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][r] = 0.0f;
+    // operand column of this lane (the spare ones repeat the last), its column and digit
+    const int j0 = min(c16, jn - 1), col = j0 % columns;
+    const float digit_scale = j0 < columns ? 0.0625f : j0 < 2 * columns ? 16.0f : 4096.0f;   // 256^digit / 16
+    // even lanes keep rows 0, 1 of the quad and hold pairs 0, 1; odd lanes rows 2, 3 and pairs 2, 3
+    const uint32_t sel0 = odd ? 0x05040100u : 0x01000504u, sel1 = odd ? 0x07060302u : 0x03020706u;
+
+    // v_perm_b32(own, received): bytes of pairs 0 .. 3 of one row
+    auto compute = [&](int lb, int d) {                        // lb: block within the chunk
+        const uint32_t lo = __builtin_amdgcn_perm(raw[d][1], raw[d][0], 0x05010400u);   // rows 0 and 1, this lane's two pairs
+        const uint32_t hi = __builtin_amdgcn_perm(raw[d][1], raw[d][0], 0x07030602u);   // rows 2 and 3
+        const uint32_t keep = odd ? hi : lo, send = odd ? lo : hi;
+        const uint32_t got = __builtin_amdgcn_update_dpp(0, send, 0xb1, 0xf, 0xf, true);
+        const uint32_t row[2] = {__builtin_amdgcn_perm(keep, got, sel0), __builtin_amdgcn_perm(keep, got, sel1)};
+        const long b = *reinterpret_cast<const long *>(digits + (lb * 4 + g) * jn + j0);
+        const float sb = block_scale[lb * columns + col] * digit_scale;
+        const uint32_t sw[4] = {sc[d].x, sc[d].y, sc[d].z, sc[d].w};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            union { uint32_t u[2]; long v; } a;
+            a.u[0] = (row[i] << 4) & 0xf0f0f0f0u;
+            a.u[1] = row[i] & 0xf0f0f0f0u;
+            const int4v t = __builtin_amdgcn_mfma_i32_16x16x32_i8(a.v, b, int4v{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float dw = kk::half_bits_to_float(i ? sw[r] >> 16 : sw[r] & 0xffffu);
+                acc[i][r] = fmaf(static_cast<float>(t[r]), dw * sb, acc[i][r]);
+            }
+        }
+    };
+
+    // activations of a chunk: thread = up to kNmGroups (block, column, K group) of 8 values, the
+    // K group fastest, then the column: the digits' LDS writes then cover all banks (with the
+    // block before the column they hit two). Blocks past K: the last one again.
+    float v[kNmGroups][8];
+    int place[kNmGroups];                                      // block of the chunk << 8 | column
+#pragma unroll
+    for (int u = 0; u < kNmGroups; ++u) {
+        const int cb = (static_cast<int>(threadIdx.x) + u * kNmThreads) >> 2;
+        place[u] = (cb / columns) << 8 | cb % columns;
+    }
+    auto load_x = [&](int base) {
+#pragma unroll
+        for (int u = 0; u < kNmGroups; ++u) {
+            int at_place = place[u];
+            asm volatile("" : "+v"(at_place));                          // keeps what follows from being hoisted into spills
+            const uint32_t at = static_cast<uint32_t>(at_place & 255) * k + min(base + (at_place >> 8), blocks - 1) * 32 + 2 * (lane & 3);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if constexpr (F16X) {
+                    const uint16_t *xh = static_cast<const uint16_t *>(x) + at + 8 * q;
+                    v[u][2 * q] = kk::half_bits_to_float(xh[0]);
+                    v[u][2 * q + 1] = kk::half_bits_to_float(xh[1]);
+                } else {
+                    const float2a4 f = *reinterpret_cast<const float2a4 *>(static_cast<const float *>(x) + at + 8 * q);
+                    v[u][2 * q] = f.x;
+                    v[u][2 * q + 1] = f.y;
+                }
+            }
+        }
+    };
+    auto convert = [&](int here) {
+#pragma unroll
+        for (int u = 0; u < kNmGroups; ++u) {
+            if (kNmThreads * u + 64 * wid >= here * columns * 4) break;   // wave-uniform
+            int at_place = place[u];
+            asm volatile("" : "+v"(at_place));
+            const int b = at_place & 255, lb = at_place >> 8;
+            float m = 0.0f, bad = 0.0f;                        // bad: NaN once a value is not finite
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                bad = fmaf(v[u][t], 0.0f, bad);
+                m = fmaxf(m, fabsf(v[u][t]));
+            }
+            // the four threads of a block are the lanes of one quad
+            m = fmaxf(m, kk::dpp_move<0xb1>(m));
+            m = fmaxf(m, kk::dpp_move<0x4e>(m));
+            bad += kk::dpp_move<0xb1>(bad);
+            bad += kk::dpp_move<0x4e>(bad);
+            // 2^(e-1) <= m < 2^e; e >= -100 keeps 2^(22-e) finite
+            const int e = max(__builtin_amdgcn_frexp_expf(m), -100);
+            const float to_fixed = ldexpf(1.0f, 22 - e);
+            // v * 2^(22-e) rounded, + 0x808080: its bytes are the digits + 128
+            uint32_t z[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+                z[t] = (__float_as_uint(fmaf(v[u][t], to_fixed, 12582912.0f)) + (0x808080u - 0x4b400000u)) ^ 0x808080u;
+            uint32_t dig[3][2];                                // [digit][even / odd K], the four pairs' bytes
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t p01 = __builtin_amdgcn_perm(z[2 + h], z[h], 0x05010400u);       // z0.0 z1.0 z0.1 z1.1
+                const uint32_t p23 = __builtin_amdgcn_perm(z[6 + h], z[4 + h], 0x05010400u);
+                dig[0][h] = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+                dig[1][h] = __builtin_amdgcn_perm(p23, p01, 0x07060302u);
+                dig[2][h] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(z[6 + h], z[4 + h], 0x0c0c0602u),
+                                                  __builtin_amdgcn_perm(z[2 + h], z[h], 0x0c0c0602u), 0x05040100u);
+            }
+            if (lb < here) {
+                uint2 *dst = digits + (lb * 4 + (lane & 3)) * jn + b;
+#pragma unroll
+                for (int l = 0; l < 3; ++l) dst[l * columns] = make_uint2(dig[l][0], dig[l][1]);
+                if ((lane & 3) == 0) block_scale[lb * columns + b] = bad != 0.0f ? __builtin_nanf("") : ldexpf(1.0f, e - 22);
+            }
+        }
+    };
+
+    load_x(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int d = 0; d < kNmDepth; ++d) {                       // the first weights behind the first activations,
+        load(d, d);                                            // in the loop's order: the waits there count loads
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    int base = 0;
+    do {                                                       // (K has blocks: no test in front for the loads to sink behind)
+        const int here = min(chunk, blocks - base);
+        if (base) nm_barrier();
+        convert(here);
+        if (base + chunk < blocks) load_x(base + chunk);   // the next chunk's, behind this one's products
+        nm_barrier();
+        const int s0 = base / kNmWaves;                           // chunk % kNmStep == 0: the ring index stays static
+        int t = 0;
+        do {
+#pragma unroll
+            for (int d = 0; d < kNmDepth; ++d) {
+                const int lb = wid + kNmWaves * (t + d);
+                if (lb < here) compute(lb, d);                 // wave-uniform
+                load(s0 + t + d + kNmDepth, d);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            t += kNmDepth;
+        } while (kNmWaves * t < here);
+    } while ((base += chunk) < blocks);
+    nm_barrier();                                           // the digits are idle
+    float *part = reinterpret_cast<float *>(lds4);             // [wave][operand column][33]
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[(wid * 16 + c16) * 33 + 8 * g + 2 * r + i] = acc[i][r];
+    nm_barrier();
+    const int row = threadIdx.x & 31, b = threadIdx.x >> 5, gr = tile * 32 + row;
+    if (b < columns && gr < n) {
+        float v = 0.0f;                                        // the smallest digit's sum first, the waves' in pairs
+#pragma unroll
+        for (int l = 0; l < 3; ++l) {
+            float p[kNmWaves];
+#pragma unroll
+            for (int wv = 0; wv < kNmWaves; ++wv) p[wv] = part[(wv * 16 + l * columns + b) * 33 + row];
+            v += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+        }
+        y[static_cast<size_t>(b) * n + gr] = v;
+    }
+}
+
+template <bool F16X>
+hipError_t launch_mfma(const uint8_t *w, const uint16_t *scales, const void *x, float *y, int k, int n, int batch,
+                       hipStream_t stream) {
+    // columns in equal groups: the spare operand columns cost as much as used ones
+    const int groups = (batch + kNmMaxColumns - 1) / kNmMaxColumns, columns = (batch + groups - 1) / groups;
+    const int column_groups = (batch + columns - 1) / columns, tiles = (n + 31) / 32;
+    const int chunk = nm_chunk(k >> 5, columns);
+    const size_t lds = std::max<size_t>(static_cast<size_t>(chunk) * columns * 100, kNmPart);
+    hipLaunchKernelGGL(native_q4_mfma<F16X>, dim3(static_cast<unsigned>((tiles + 7) / 8) * 8 * column_groups),
+                       dim3(kNmThreads), lds, stream, w, scales, x, y, k, n, batch, columns, chunk, column_groups, tiles);
+    return hipGetLastError();
+}
+
 } // namespace
 
 extern "C" size_t kk_native_q4_payload_bytes(int k, int n) {
@@ -282,6 +540,14 @@ extern "C" int kk_native_q4_gemv(const void *weights, const void *x, int x_f16, 
     const uint8_t *w = static_cast<const uint8_t *>(weights);
     const uint16_t *scales = reinterpret_cast<const uint16_t *>(w + kk_native_q4_payload_bytes(k, n));
     const int blocks = k >> 5;
+    const size_t x_bytes = x_f16 ? 2 : 4;
+    // One column, and two on small matrices, stay on the dot product kernel (us per call,
+    // which ends with a wait of about 15: K4096 x N4096 one column 17.1 against 19.8, two
+    // 19.1 / 20.0, three 20.8 / 20.6; two columns of K4096 x N11008 26.0 / 24.9 and K11008 x
+    // N4096 31.0 / 28.0).
+    if (batch > 2 || (batch == 2 && static_cast<size_t>(k) * n >= (size_t{32} << 20)))
+        return x_f16 ? launch_mfma<true>(w, scales, x, y, k, n, batch, stream)
+                     : launch_mfma<false>(w, scales, x, y, k, n, batch, stream);
     // columns per launch: LDS within the limit and activation passes within the register budget
     auto fits = [&](int cols) {
         return lds_bytes(blocks, cols) <= kNqLdsLimit && passes_for(blocks, cols) <= kNqMaxPasses;
@@ -289,7 +555,6 @@ extern "C" int kk_native_q4_gemv(const void *weights, const void *x, int x_f16, 
     if (!fits(1)) return hipErrorInvalidValue;
     int fit = 1;
     while (fit < kNqMaxColumns && fits(fit + 1)) ++fit;
-    const size_t x_bytes = x_f16 ? 2 : 4;
     for (int c0 = 0; c0 < batch; c0 += fit) {
         const int cols = std::min(fit, batch - c0);
         const int passes = passes_for(blocks, cols);
@@ -298,9 +563,7 @@ extern "C" int kk_native_q4_gemv(const void *weights, const void *x, int x_f16, 
         hipError_t status;
         switch (cols) {
         case 1: status = launch_passes<1>(passes, w, scales, xc, x_f16, yc, k, n, stream); break;
-        case 2: status = launch_passes<2>(passes, w, scales, xc, x_f16, yc, k, n, stream); break;
-        case 3: status = launch_passes<3>(passes, w, scales, xc, x_f16, yc, k, n, stream); break;
-        default: status = launch_passes<4>(passes, w, scales, xc, x_f16, yc, k, n, stream); break;
+        default: status = launch_passes<2>(passes, w, scales, xc, x_f16, yc, k, n, stream); break;
         }
         if (status != hipSuccess) return status;
     }

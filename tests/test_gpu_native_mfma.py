@@ -1,0 +1,41 @@
+"""GPU parity of native_q4_matmul above one column (int8 MFMA, up to 16
+columns per launch): one column per digit slot and three MFMAs per block
+(1..5 and 6..16 columns), blocks that do not fill the waves, one and several
+LDS chunks of activations, remainders of N, unaligned F32 and F16 X, columns of
+very different size and non-finite activations. Same bounds as the other
+native Q4 tests: exact up to the activations' 23-bit block fixed point.
+"""
+import numpy as np
+import pytest
+
+import kunlunk200_lib_amd as kl
+from test_gpu_native_q4 import NativeCase, check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("f16,x_offset", [(False, 4), (True, 2)], ids=["f32", "f16"])
+@pytest.mark.parametrize("k,n,batch", [(32, 1, 2), (96, 33, 5), (288, 64, 6), (4096, 40, 5), (4096, 100, 15), (5152, 31, 16),
+                                       (2080, 65, 17), (16384, 32, 21), (1024, 31, 33), (11008, 70, 3)])
+def test_native_columns(gpu, oracle, k, n, batch, f16, x_offset):
+    case = NativeCase(oracle, k, n)
+    x = np.random.default_rng(k + n + batch).standard_normal((batch, k)).astype(np.float32)
+    x[1] *= 1e-3
+    x[0, : k // 2] *= 200.0
+    if f16:
+        x = x.astype(np.float16).astype(np.float32)
+    y, flag = case.run(kl.NativeQ4Workspace(), x, batch, f16=f16, x_offset=x_offset)
+    assert not flag
+    check(oracle, case, y, x)
+
+
+@pytest.mark.parametrize("batch", [4, 16])
+def test_native_columns_nonfinite(gpu, oracle, batch):
+    k, n = 4096, 70
+    case = NativeCase(oracle, k, n)
+    x = np.random.default_rng(batch).standard_normal((batch, k)).astype(np.float32)
+    x[1, 5], x[2, k - 1] = np.nan, np.inf
+    y, _ = case.run(kl.NativeQ4Workspace(), x, batch)
+    keep = np.delete(np.arange(batch), (1, 2))
+    assert np.all(np.isnan(y[1:3]))
+    check(oracle, case, y[keep], x[keep])
