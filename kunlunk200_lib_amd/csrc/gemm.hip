@@ -1502,6 +1502,192 @@ __global__ __launch_bounds__(512) void q4_wide_gemm(const uint8_t *__restrict__ 
         }
 }
 
+// ---------------------------------------------------------------------------
+// f16_wide_gemm: q4_wide_gemm for F16 weights: the same 128 x 64 wave tiles and one
+// barrier per step, the weight fragments read from LDS a step ahead as the activations'
+// are. KG = 1: 256 x 256 outputs, K32 steps; KG = 2: 128 x 256, K64 steps (K % 64 == 0).
+// Rings of four steps of 16 + 16 KiB (KG = 1) and three of 16 + 32 KiB (KG = 2), the copies of
+// step s + 3 issued in step s: with three buffers into the one whose fragments were
+// read in step s - 1, so those reads are waited for before the barrier.
+// Bound by the MFMAs, and the clock under them once all CUs run (K4096 x N4096: 192 tiles of
+// 128 x 256 take 57 us, 256 tiles 70); the register-staged kernel reads 85 - 128 bytes of
+// operands per cycle and CU from LDS at full MFMA rate, these 48 and 80. K4096 x N11008,
+// 2048 rows: 322 -> 205 us per call (930 TFLOP/s; a library fp16 GEMM 203).
+template <int KG>
+struct WfShape {
+    static constexpr int Rows = 256 / KG, StepK = 32 * KG, Bufs = KG == 1 ? 4 : 3;
+    static constexpr int ABytes = 16 * 1024, BBytes = 256 * StepK * 2, Bytes = ABytes + BBytes;
+    static constexpr int BCopies = BBytes / 8192;                    // 1 KiB copies per wave and step
+    static constexpr int Lds = (Bufs * Bytes > 128 * 1024 ? Bufs * Bytes : 128 * 1024) + 256 * 4;
+    static_assert(Lds <= 160 * 1024, "LDS");
+};
+
+template <typename S, bool PAIR>
+__device__ __forceinline__ void wf_copy(const uint32_t (&a_off)[2], const uint32_t (&b_off)[S::BCopies], _Float16 *a_tile,
+                                        int a_extent, uint8_t *b_tile, uint8_t *b_tile2, int b_extent, int wid, int soff,
+                                        int buf) {
+    extern __shared__ __align__(16) uint8_t wd_lds[];
+    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(a_tile, 0, a_extent, 0x00020000);
+    const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc(b_tile, 0, b_extent, 0x00020000);
+    const __amdgpu_buffer_rsrc_t b_rsrc2 = __builtin_amdgcn_make_buffer_rsrc(b_tile2, 0, b_extent, 0x00020000);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (__attribute__((address_space(3))) uint8_t *)wd_lds + buf * S::Bytes +
+                                                 (wid + 8 * t) * 1024, 16, a_off[t], soff, 0, 0);
+#pragma unroll
+    for (int t = 0; t < S::BCopies; ++t)                             // pair: the second half of the copies are up rows
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(PAIR && t >= S::BCopies / 2 ? b_rsrc2 : b_rsrc,
+                                                 (__attribute__((address_space(3))) uint8_t *)wd_lds + buf * S::Bytes +
+                                                 S::ABytes + (wid + 8 * t) * 1024, 16, b_off[t], soff, 0, 0);
+}
+
+template <bool PAIR, int KG>
+__global__ __launch_bounds__(512) void f16_wide_gemm(const uint8_t *__restrict__ w, const uint8_t *__restrict__ w2,
+                                                     const _Float16 *__restrict__ x16, const float *__restrict__ row_inv,
+                                                     float *__restrict__ y, int m_rows, int m_pad, int n_rows, int k_pad,
+                                                     int k, int m_tiles, int tiles, int tiles_per_xcd) {
+    using S = WfShape<KG>;
+    extern __shared__ __align__(16) uint8_t wd_lds[];
+    constexpr int kOut = PAIR ? 128 : 256;                           // output columns per tile
+    const int bid = blockIdx.x;
+    const int tile = (bid % kXcds) * tiles_per_xcd + bid / kXcds;
+    if (tile >= tiles) return;                                       // whole workgroup, before any barrier
+    const int nt = tile / m_tiles, mt = tile - nt * m_tiles;
+    const int m0 = mt * S::Rows, n0 = nt * kOut;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wid = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int grp = wid >> 2, wn = wid & 3;                          // row half (KG = 1) or k-group; columns
+    const int g = lane >> 4, c16 = lane & 15;
+    const uint32_t row_bytes = static_cast<uint32_t>(k) * 2;
+    const int steps = k / S::StepK;
+
+    // copy i of either operand: 1 KiB of whole rows of a step; chunk c of row r sits at
+    // position c ^ swizzle(r), as in q4_wide_gemm
+    constexpr int kChunks = S::StepK / 8, kRowsPerCopy = 64 / kChunks;
+    auto swizzle = [](int r) { return KG == 1 ? (r >> 2) & 3 : (r >> 1) & 7; };
+    _Float16 *const a_tile = const_cast<_Float16 *>(x16 + static_cast<size_t>(m0) * k_pad);
+    const int a_extent = min(S::Rows, m_pad - m0) * k_pad * 2;       // rows past m_pad read as zero
+    const int copy_row = lane / kChunks, copy_pos = lane % kChunks;
+    uint32_t a_off[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int r = kRowsPerCopy * (wid + 8 * t) + copy_row;
+        a_off[t] = static_cast<uint32_t>(r * k_pad * 2 + 16 * (copy_pos ^ swizzle(r)));
+    }
+    // weight rows 0 .. 255 of the tile (PAIR: 128 gate rows, then the up rows); past n the last row again
+    constexpr int kRows = PAIR ? 128 : 256;
+    const int b_extent = min(kRows, n_rows - n0) * static_cast<int>(row_bytes);
+    uint8_t *const b_tile = const_cast<uint8_t *>(w + static_cast<size_t>(n0) * row_bytes);
+    uint8_t *const b_tile2 = const_cast<uint8_t *>(w2 + static_cast<size_t>(n0) * row_bytes);
+    uint32_t b_off[S::BCopies];
+#pragma unroll
+    for (int t = 0; t < S::BCopies; ++t) {
+        const int r = kRowsPerCopy * (wid + 8 * t) + copy_row, wr = PAIR ? r & 127 : r;
+        b_off[t] = static_cast<uint32_t>(min(n0 + wr, n_rows - 1) - n0) * row_bytes + 16 * (copy_pos ^ swizzle(r));
+    }
+    const uint32_t chunk = 16 * ((KG == 1 ? g : 4 * grp + g) ^ swizzle(c16));
+    const uint32_t a_read = static_cast<uint32_t>(((KG == 1 ? 128 * grp : 0) + c16) * (S::StepK * 2)) + chunk;
+    const uint32_t b_read = static_cast<uint32_t>(S::ABytes + ((PAIR ? 32 : 64) * wn + c16) * (S::StepK * 2)) + chunk;
+
+    float4v acc[8][4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    half8 a[8], b[2][4];
+    auto read_a = [&](uint32_t at, int i) {
+        return *reinterpret_cast<const half8 *>(wd_lds + at + a_read + i * 16 * (S::StepK * 2));
+    };
+    auto read_b = [&](uint32_t at, int c) {
+        const int row = PAIR ? (c >> 1) * 128 + (c & 1) * 16 : c * 16;
+        return *reinterpret_cast<const half8 *>(wd_lds + at + b_read + row * (S::StepK * 2));
+    };
+    // Step s: issues the copies of step s + 3, multiplies step s, reads step s + 1 (past
+    // K: copied from the next rows or as zeros, and not used)
+    auto step = [&](auto ic, int s, int next_buf, int copy_buf) {
+        constexpr int C = decltype(ic)::value;
+        // all but the copies of step s + 2 have landed
+        __builtin_amdgcn_s_waitcnt((KG == 1 ? 0x0F70 : 0x0070) | (2 + S::BCopies));
+        wd_barrier();
+        wf_copy<S, PAIR>(a_off, b_off, a_tile, a_extent, b_tile, b_tile2, b_extent, wid, (s + 3) * (S::StepK * 2), copy_buf);
+        const uint32_t at = static_cast<uint32_t>(next_buf) * S::Bytes;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc[i][c]) : "v"(a[i]), "v"(b[C][c]));
+            __builtin_amdgcn_sched_barrier(0);
+            a[i] = read_a(at, i);
+            if (i < 4) b[C ^ 1][i] = read_b(at, i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+        wf_copy<S, PAIR>(a_off, b_off, a_tile, a_extent, b_tile, b_tile2, b_extent, wid, s * (S::StepK * 2), s);
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * (2 + S::BCopies)));
+    wd_barrier();
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a[i] = read_a(0, i);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) b[0][c] = read_b(0, c);
+    int buf = 0;                                                     // step s's
+    auto after = [](int v) { return v + 1 == S::Bufs ? 0 : v + 1; };
+    // step s + 3 goes into the buffer three on: with three buffers that of step s itself
+    int s = 0;
+    for (; s + 2 <= steps; s += 2) {
+        const int b1 = after(buf), b2 = after(b1);
+        step(std::integral_constant<int, 0>{}, s, b1, KG == 1 ? after(b2) : buf);
+        step(std::integral_constant<int, 1>{}, s + 1, b2, KG == 1 ? buf : b1);
+        buf = b2;
+    }
+    if (s < steps) step(std::integral_constant<int, 0>{}, s, after(buf), KG == 1 ? after(after(after(buf))) : buf);   // uniform
+    __builtin_amdgcn_s_waitcnt(0x0F70);                              // the trailing copies land,
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");               // the last MFMAs' results too (asm: no automatic wait)
+    __syncthreads();
+    float *scale_lds = reinterpret_cast<float *>(wd_lds + S::Lds - 256 * 4);
+    if (threadIdx.x < S::Rows) scale_lds[threadIdx.x] = row_inv[min(m0 + static_cast<int>(threadIdx.x), m_pad - 1)];
+    if constexpr (KG == 2) {
+        // each k-group hands the other half its row tiles, and finishes its own half
+        float4v *xfer = reinterpret_cast<float4v *>(wd_lds);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                float4v &mine = grp ? acc[i][c] : acc[i + 4][c];
+                xfer[((wid * 4 + i) * 4 + c) * kWave + lane] = mine;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float4v other = xfer[(((wid ^ 4) * 4 + i) * 4 + c) * kWave + lane];
+                acc[i][c] = (grp ? acc[i + 4][c] : acc[i][c]) + other;
+            }
+    }
+    __syncthreads();
+    constexpr int kHalves = KG == 1 ? 2 : 1;
+    const int row_base = KG == 1 ? 128 * grp : 64 * grp;
+#pragma unroll
+    for (int i = 0; i < 4 * kHalves; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = row_base + 16 * i + 4 * g + r, m = m0 + row;
+            if (m >= m_rows) continue;
+            const float sc = scale_lds[row];
+            float *dst = y + static_cast<size_t>(m) * n_rows;
+#pragma unroll
+            for (int c = 0; c < (PAIR ? 2 : 4); ++c) {
+                const int n = n0 + (PAIR ? 32 : 64) * wn + 16 * c + c16;
+                const float v = PAIR ? kk::swiglu_value(acc[i][c][r] * sc, acc[i][(c + 2) & 3][r] * sc) : acc[i][c][r] * sc;
+                if (n < n_rows) __builtin_nontemporal_store(v, dst + n);
+            }
+        }
+}
+
 // y[m][n] = the ranges' partial sums, added in range order, times the row's scale
 // (PAIR: SiLU(gate) * up of the two matrices' values). Four columns per thread.
 constexpr int kSumThreads = 256;
@@ -1734,6 +1920,60 @@ hipError_t launch_ql(const void *w, const void *w2, const _Float16 *x16, const f
     return hipErrorInvalidValue;
 }
 
+template <bool PAIR, int KG>
+hipError_t launch_f16_wide(const void *w, const void *w2, const _Float16 *x16, const float *row_inv, float *y, int batch,
+                           int n, int k, int k_pad, hipStream_t stream) {
+    using S = WfShape<KG>;
+    const hipError_t rc = kk::opt_in_lds(reinterpret_cast<const void *>(&f16_wide_gemm<PAIR, KG>), S::Lds);
+    if (rc != hipSuccess) return rc;
+    const int out = PAIR ? 128 : 256;
+    const int m_tiles = (batch + S::Rows - 1) / S::Rows;
+    const int tiles = m_tiles * ((n + out - 1) / out);
+    const int tiles_per_xcd = (tiles + kXcds - 1) / kXcds;
+    const int m_pad = static_cast<int>(round_up(static_cast<size_t>(batch), kBM));
+    hipLaunchKernelGGL((f16_wide_gemm<PAIR, KG>), dim3(tiles_per_xcd * kXcds), dim3(512), S::Lds, stream,
+                       static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(w2), x16, row_inv, y, batch, m_pad, n,
+                       k_pad, k, m_tiles, tiles, tiles_per_xcd);
+    return hipGetLastError();
+}
+
+// The wide F16 tile of a call (its rows: 256 or 128), or 0 for the register-staged
+// kernel: the least time in whole rounds of the CUs, a round of K4096 taking 37 us of 128 x
+// 64 register-staged tiles, 49 of 128 x 128, 78 of 256 x 256 and 44 of 128 x 256 wide
+// ones. us per call, register-staged / wide: K4096 x N4096 b1024 62 / 56 (128 rows; 88 with
+// 256), b2048 117 / 76, K4096 x N11008 b512 103 / 61, b1024 164 / 102 (256 rows; 114 with
+// 128), b2048 322 / 205, K4096 x N4096 b512 43 / 52 (stays). KUNLUN_GEMM_TILE=256x64 and
+// 128x64 force the wide tiles, another tile none of them.
+int pick_f16_wide(const GemmPlan &p, int batch, int n, int k, bool pair) {
+    const int forced = kk::tuning(kk::kGemmTile);
+    if (forced > 0) return forced == 256 * 1000 + 64 ? 256 : forced == 128 * 1000 + 64 && k % 64 == 0 ? 128 : 0;
+    const long cus = device_cus(), columns = (n + (pair ? 127 : 255)) / (pair ? 128 : 256);
+    auto rounds = [&](long tiles) { return (tiles + cus - 1) / cus; };
+    const bool wide_staged = pair || p.bn == 128;
+    const long staged = rounds(static_cast<long>(p.m_tiles) * (pair ? (n + 63) / 64 : p.n_tiles)) * (wide_staged ? 49 : 37);
+    const long rows256 = rounds((batch + 255) / 256 * columns) * 78;
+    const long rows128 = k % 64 == 0 ? rounds((batch + 127) / 128 * columns) * 44 : rows256 + 1;
+    if (std::min(rows256, rows128) >= staged) return 0;
+    // few tiles that each stream activations past an XCD's L2 (4 MiB) wait for them: 96
+    // tiles of K8192 x N8192 b300 (4.7 MiB) 119 against 117 register-staged, of K8128 120 / 115,
+    // 100 of K11008 x N5000 b640 (13 MiB) 170 / 152, but K6144 x N8192 b300 (3.5 MiB) 71 / 86 and
+    // 120 of K4096 x N6000 b520 (4.1 MiB) 51 / 68
+    const long tiles = (batch + 127) / 128 * columns;
+    if (tiles < cus / 2 && static_cast<size_t>(batch) * k * 2 > (size_t{9} << 19)) return 0;
+    return rows128 <= rows256 ? 128 : 256;
+}
+
+template <bool PAIR>
+hipError_t launch_f16(const void *w, const void *w2, const _Float16 *x16, const float *row_inv, float *y, float *part,
+                      int batch, int n, int k, const GemmPlan &p, const KRanges &kr, hipStream_t stream) {
+    const int wide = kr.ranges > 1 ? 0 : pick_f16_wide(p, batch, n, k, PAIR);
+    if (wide == 256) return launch_f16_wide<PAIR, 1>(w, w2, x16, row_inv, y, batch, n, k, p.k_pad, stream);
+    if (wide == 128) return launch_f16_wide<PAIR, 2>(w, w2, x16, row_inv, y, batch, n, k, p.k_pad, stream);
+    const size_t w_bytes = static_cast<size_t>(n) * k * 2;
+    if (PAIR || p.bn == 128) return launch_gemm<true, 128, PAIR>(w, w2, x16, row_inv, y, part, batch, n, k, p, kr, w_bytes, stream);
+    return launch_gemm<true, PAIR ? 128 : 64, PAIR>(w, w2, x16, row_inv, y, part, batch, n, k, p, kr, w_bytes, stream);
+}
+
 // The LDS-copy Q4_0 GEMM takes K in whole stage pairs (256) and 16-byte aligned
 // weights (rows of (K / 256) * 144 bytes, copied 16 bytes per lane).
 bool ql_shape(int k, const void *w, const void *w2) {
@@ -1764,15 +2004,14 @@ extern "C" int kk_gemm(int type, const void *w, const float *x, float *y, int k,
     launch_x_to_f16(type == 2, x, batch, k, p.m_pad, p.k_pad, x16, row_inv, stream);
     hipError_t rc = hipGetLastError();
     if (rc != hipSuccess) return rc;
-    const size_t w_bytes = type == 1 ? static_cast<size_t>(n) * k * 2 : static_cast<size_t>(n) * (k / 32) * 18;
+    const size_t w_bytes = static_cast<size_t>(n) * (k / 32) * 18;   // Q4_0
     if (route) *route = type == 2 ? "q4_gemm_mfma" : "f16_gemm_mfma";
     if (type == 2 && ql_shape(k, w, w)) return launch_ql<false>(w, w, x16, row_inv, y, batch, n, k, p, part, stream);
     const KRanges kr = ranges_staged(p, k, n, batch, false);
     if (type == 2)
         return p.bn == 128 ? launch_gemm<false, 128>(w, w, x16, row_inv, y, part, batch, n, k, p, kr, w_bytes, stream)
                            : launch_gemm<false, 64>(w, w, x16, row_inv, y, part, batch, n, k, p, kr, w_bytes, stream);
-    return p.bn == 128 ? launch_gemm<true, 128>(w, w, x16, row_inv, y, part, batch, n, k, p, kr, w_bytes, stream)
-                       : launch_gemm<true, 64>(w, w, x16, row_inv, y, part, batch, n, k, p, kr, w_bytes, stream);
+    return launch_f16<false>(w, w, x16, row_inv, y, part, batch, n, k, p, kr, stream);
 }
 
 extern "C" int kk_gemm_swiglu(int type, const void *w_gate, const void *w_up, const float *x, float *y, int k, int n,
@@ -1793,11 +2032,11 @@ extern "C" int kk_gemm_swiglu(int type, const void *w_gate, const void *w_up, co
     launch_x_to_f16(type == 2, x, batch, k, p.m_pad, p.k_pad, x16, row_inv, stream);
     hipError_t rc = hipGetLastError();
     if (rc != hipSuccess) return rc;
-    const size_t w_bytes = type == 1 ? static_cast<size_t>(n) * k * 2 : static_cast<size_t>(n) * (k / 32) * 18;
+    const size_t w_bytes = static_cast<size_t>(n) * (k / 32) * 18;   // Q4_0
     if (route) *route = type == 2 ? "q4_gemm_swiglu_mfma" : "f16_gemm_swiglu_mfma";
     if (type == 2 && ql_shape(k, w_gate, w_up))
         return launch_ql<true>(w_gate, w_up, x16, row_inv, y, batch, n, k, p, part, stream);
     const KRanges kr = ranges_staged(p, k, n, batch, true);
     if (type == 2) return launch_gemm<false, 128, true>(w_gate, w_up, x16, row_inv, y, part, batch, n, k, p, kr, w_bytes, stream);
-    return launch_gemm<true, 128, true>(w_gate, w_up, x16, row_inv, y, part, batch, n, k, p, kr, w_bytes, stream);
+    return launch_f16<true>(w_gate, w_up, x16, row_inv, y, part, batch, n, k, p, kr, stream);
 }

@@ -12,7 +12,7 @@ enum Knob {
     kQ4MfmaMax,
     kDenseMfmaMin,        // KUNLUN_DENSE_MFMA_MIN / _MAX: batch range of the F32/F16 MFMA GEMV
     kDenseMfmaMax,
-    kGemmTile,            // KUNLUN_GEMM_TILE=BMxWN: Q4_0 LDS GEMM tile, stored as BM * 1000 + WN
+    kGemmTile,            // KUNLUN_GEMM_TILE=BMxWN: prefill GEMM tile, stored as BM * 1000 + WN
     kGemmBn,              // KUNLUN_GEMM_BN=64|128: register-staged GEMM tile width
     kGemvGeneral,         // KUNLUN_GEMV_GENERAL=1: every GEMV on the general kernel
     kI8FusedQuantLimit,   // KUNLUN_I8_FUSED_QUANT_LIMIT: single-workgroup quantizer limit
