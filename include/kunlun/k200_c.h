@@ -224,7 +224,7 @@ int kunlun_get_tuning(const char *name);
  * forbid hipMalloc): kunlun_matmul for KUNLUN_F32, KUNLUN_F16 and KUNLUN_Q4_0
  * weights on the same routes and kernels, that allocates nothing. The
  * scratch of the routes that need it (the batch >= 64 fp16-MFMA GEMM and the
- * Q4_0 MFMA GEMV) is a fixed device array of KUNLUN_NOALLOC_SCRATCH_BYTES per
+ * K-split Q4_0 MFMA GEMV) is a fixed device array of KUNLUN_NOALLOC_SCRATCH_BYTES per
  * GPU, held until the process ends; a call that needs more returns
  * KUNLUN_NOALLOC_TOO_LARGE (the GEMM needs about 2 * batch * K bytes, so
  * batch * K <= 8M fits). The caller passes device pointers for y, w and x

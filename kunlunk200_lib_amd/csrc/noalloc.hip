@@ -2,8 +2,8 @@
 // any device allocation, for callers that cannot allocate (code under HIP
 // graph capture, tight serving loops). It takes the routes and kernels of
 // kunlun::matmul (matmul.cpp); the routes that need device memory beyond the
-// inputs and outputs -- the fp16-MFMA prefill GEMM (fp16 activations and row
-// scales, kk_gemm_workspace_bytes) and the K-split Q4_0 MFMA GEMV (partial
+// inputs and outputs -- the fp16-MFMA prefill GEMM (fp16 activations, row
+// scales and partial sums, kk_gemm_workspace_bytes) and the K-split Q4_0 MFMA GEMV (partial
 // sums, kk_q4_split_workspace_bytes) -- take it from `scratch`, a
 // file-scope device array of kScratchBytes, instead of a Kernel's workspace.
 //
@@ -12,7 +12,7 @@
 // hipGetSymbolAddress returns (taken once per device, with that device
 // current, on the entry point's first call there); the array's name in host
 // code is a host-side stand-in, not a device address. The kernels write every
-// scratch byte they read in the same call, so nothing needs clearing, but
+// scratch value they use in the same call, so nothing needs clearing, but
 // calls that overlap on one GPU share the array and race.
 #include "launch.h"
 #include "runtime_internal.h"
