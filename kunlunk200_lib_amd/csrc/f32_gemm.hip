@@ -63,15 +63,20 @@ __device__ __forceinline__ void dg_copy(const uint8_t *w, int w_bytes, const flo
                                         const uint32_t (&x_off)[DgShape<MT, SHARE>::XCopies], int wid, int s) {
     using D = DgShape<MT, SHARE>;
     extern __shared__ __align__(16) uint8_t dg_lds[];
-    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(w), 0, w_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(x), 0, x_bytes, 0x00020000);
+    // the stage's offset moves the base and the extent, so that a lane past the matrix (a
+    // last stage that K does not fill) is past the extent by its own offset
+    const int at = s * kDgRow;
+    const __amdgpu_buffer_rsrc_t w_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(w) + at, 0, w_bytes - at, 0x00020000);
+    const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(reinterpret_cast<const uint8_t *>(x)) + at, 0, x_bytes - at, 0x00020000);
     __attribute__((address_space(3))) uint8_t *buf =
         (__attribute__((address_space(3))) uint8_t *)dg_lds + (s % D::Slots) * D::StageBytes;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, buf + wid * 1024, 16, w_off, s * kDgRow, 0, 2);   // read once
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, buf + wid * 1024, 16, w_off, 0, 0, 2);   // read once
 #pragma unroll
     for (int t = 0; t < D::XCopies; ++t)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, buf + D::WBytes + (wid + kDgWaves * t) * 1024, 16, x_off[t],
-                                                 s * kDgRow, 0, 0);
+                                                 0, 0, 0);
 }
 
 template <int MT, bool SHARE>

@@ -18,6 +18,7 @@
 //    gemm_split_sum adds the ranges' partial sums in order.
 // Precision: fp16 inputs, f32 accumulation: relative error ~2^-11 per
 // product (the fp16-MFMA tolerance of the path is 2e-3 relative).
+#include "copy_bounds.h"
 #include "device_common.h"
 #include "launch.h"
 #include "lds_opt_in.h"
@@ -1264,14 +1265,16 @@ __device__ __forceinline__ void wd_copy_a(_Float16 *a_tile, int a_extent, const 
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) uint8_t *)wd_lds + buf * kWdABytes +
                                                  (wid + 8 * t) * 1024, 16, a_off[t], soff, 0, 0);
 }
-// weight copy wid + 8t of super-stage p (PAIR: below 18 the gate rows, then the up rows)
+// weight copy wid + 8t into super-stage p's buffer, of super-stage `from` (PAIR: below 18 the
+// gate rows, then the up rows)
 template <bool PAIR>
-__device__ __forceinline__ void wd_copy_b(uint8_t *b_tile, uint8_t *b_tile2, int b_extent, uint32_t off, int wid, int t, int p) {
+__device__ __forceinline__ void wd_copy_b(uint8_t *b_tile, uint8_t *b_tile2, int b_extent, uint32_t off, int wid, int t, int p,
+                                          int from) {
     extern __shared__ __align__(16) uint8_t wd_lds[];
     const int i = wid + 8 * t;
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(PAIR && i >= 18 ? b_tile2 : b_tile, 0, b_extent, 0x00020000);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) uint8_t *)wd_lds + 4 * kWdABytes +
-                                             (p & 1) * kWdBBytes + i * 1024, 16, off, p * kQlRowPair, 0, 0);
+                                             (p & 1) * kWdBBytes + i * 1024, 16, off, from * kQlRowPair, 0, 0);
 }
 __device__ __forceinline__ void wd_barrier() {
     asm volatile("" ::: "memory");
@@ -1299,7 +1302,7 @@ __global__ __launch_bounds__(512) void q4_wide_gemm(const uint8_t *__restrict__ 
     const int grp = wid >> 2, wn = wid & 3;                          // row half (KG = 1) or k-group; columns
     const int g = lane >> 4, c16 = lane & 15;
     const uint32_t row_bytes = static_cast<uint32_t>(k / 32 * 18);
-    const int steps = k / S::StepK;
+    const int steps = k / S::StepK, supers = steps / S::Super;
 
     // activation copy i: 1 KiB of whole rows of a step (16 of 64 B, KG = 2 8 of 128 B); chunk
     // c of row r sits at position c ^ (r / 4) % 4 (KG = 2 c ^ (r / 2) % 8): an operand
@@ -1322,12 +1325,7 @@ __global__ __launch_bounds__(512) void q4_wide_gemm(const uint8_t *__restrict__ 
     uint8_t *const b_tile2 = const_cast<uint8_t *>(w2 + static_cast<size_t>(n0) * row_bytes);
     uint32_t b_off[5];
 #pragma unroll
-    for (int t = 0; t < 5; ++t) {
-        const int i = wid + 8 * t;
-        const int q = (PAIR && i >= 18 ? i - 18 : i) * 64 + lane;
-        const int row = min(q / 9, kRows - 1), chunk = q - q / 9 * 9;
-        b_off[t] = i < 36 ? static_cast<uint32_t>(min(n0 + row, n_rows - 1) - n0) * row_bytes + 16 * chunk : 0x80000000u;
-    }
+    for (int t = 0; t < 5; ++t) b_off[t] = kk::wide_q4_weight<PAIR>(wid + 8 * t, lane, n_rows - n0, row_bytes);
     const uint32_t a_read = static_cast<uint32_t>(((KG == 1 ? 128 * grp : 0) + c16) * (S::StepK * 2) +
                                                   16 * ((KG == 1 ? g : 4 * grp + g) ^ swizzle(c16)));
     // this wave's 64 LDS weight rows (PAIR: 32 gate rows from 32 wn, 32 up rows from 128 + 32 wn)
@@ -1373,8 +1371,8 @@ __global__ __launch_bounds__(512) void q4_wide_gemm(const uint8_t *__restrict__ 
         return *reinterpret_cast<const half8 *>(wd_lds + (J & 3) * kWdABytes + a_read + i * 16 * (S::StepK * 2));
     };
     // Step s (I = s % Super): issues the copies of step s + 3 (and a share of the next
-    // super-stage), multiplies step s, reads and decodes step s + 1. What lies past
-    // K is copied from the next rows or as zeros, and not used.
+    // super-stage), multiplies step s, reads and decodes step s + 1. Past K the last
+    // step (super-stage) is copied again, and not used.
     uint32_t buf = 0;
     auto step = [&](auto ic, int s) {
         constexpr int I = decltype(ic)::value, C = I & 1;
@@ -1383,8 +1381,9 @@ __global__ __launch_bounds__(512) void q4_wide_gemm(const uint8_t *__restrict__ 
         wd_barrier();
 #pragma unroll
         for (int t = 0; t < S::copies(I); ++t)
-            wd_copy_b<PAIR>(b_tile, b_tile2, b_extent, b_off[S::first(I) + t], wid, S::first(I) + t, s / S::Super + 1);
-        wd_copy_a(a_tile, a_extent, a_off, wid, (s + 3) * (S::StepK * 2), (I + 3) & 3);
+            wd_copy_b<PAIR>(b_tile, b_tile2, b_extent, b_off[S::first(I) + t], wid, S::first(I) + t, s / S::Super + 1,
+                            kk::copied_step(s / S::Super + 1, supers));
+        wd_copy_a(a_tile, a_extent, a_off, wid, kk::copied_step(s + 3, steps) * (S::StepK * 2), (I + 3) & 3);
         read_raw(Next{}, buf);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1400,7 +1399,7 @@ __global__ __launch_bounds__(512) void q4_wide_gemm(const uint8_t *__restrict__ 
     };
 
 #pragma unroll
-    for (int t = 0; t < 5; ++t) wd_copy_b<PAIR>(b_tile, b_tile2, b_extent, b_off[t], wid, t, 0);
+    for (int t = 0; t < 5; ++t) wd_copy_b<PAIR>(b_tile, b_tile2, b_extent, b_off[t], wid, t, 0, 0);
 #pragma unroll
     for (int s = 0; s < 3; ++s) wd_copy_a(a_tile, a_extent, a_off, wid, s * (S::StepK * 2), s);
     __builtin_amdgcn_s_waitcnt(0x0F70 | 4);
@@ -1581,10 +1580,7 @@ __global__ __launch_bounds__(512) void f16_wide_gemm(const uint8_t *__restrict__
     uint8_t *const b_tile2 = const_cast<uint8_t *>(w2 + static_cast<size_t>(n0) * row_bytes);
     uint32_t b_off[S::BCopies];
 #pragma unroll
-    for (int t = 0; t < S::BCopies; ++t) {
-        const int r = kRowsPerCopy * (wid + 8 * t) + copy_row, wr = PAIR ? r & 127 : r;
-        b_off[t] = static_cast<uint32_t>(min(n0 + wr, n_rows - 1) - n0) * row_bytes + 16 * (copy_pos ^ swizzle(r));
-    }
+    for (int t = 0; t < S::BCopies; ++t) b_off[t] = kk::wide_f16_weight<KG, PAIR>(wid + 8 * t, lane, n_rows - n0, row_bytes);
     const uint32_t chunk = 16 * ((KG == 1 ? g : 4 * grp + g) ^ swizzle(c16));
     const uint32_t a_read = static_cast<uint32_t>(((KG == 1 ? 128 * grp : 0) + c16) * (S::StepK * 2)) + chunk;
     const uint32_t b_read = static_cast<uint32_t>(S::ABytes + ((PAIR ? 32 : 64) * wn + c16) * (S::StepK * 2)) + chunk;
@@ -1603,13 +1599,14 @@ __global__ __launch_bounds__(512) void f16_wide_gemm(const uint8_t *__restrict__
         return *reinterpret_cast<const half8 *>(wd_lds + at + b_read + row * (S::StepK * 2));
     };
     // Step s: issues the copies of step s + 3, multiplies step s, reads step s + 1 (past
-    // K: copied from the next rows or as zeros, and not used)
+    // K: the last step, copied again and not used)
     auto step = [&](auto ic, int s, int next_buf, int copy_buf) {
         constexpr int C = decltype(ic)::value;
         // all but the copies of step s + 2 have landed
         __builtin_amdgcn_s_waitcnt((KG == 1 ? 0x0F70 : 0x0070) | (2 + S::BCopies));
         wd_barrier();
-        wf_copy<S, PAIR>(a_off, b_off, a_tile, a_extent, b_tile, b_tile2, b_extent, wid, (s + 3) * (S::StepK * 2), copy_buf);
+        wf_copy<S, PAIR>(a_off, b_off, a_tile, a_extent, b_tile, b_tile2, b_extent, wid,
+                         kk::copied_step(s + 3, steps) * (S::StepK * 2), copy_buf);
         const uint32_t at = static_cast<uint32_t>(next_buf) * S::Bytes;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1626,7 +1623,8 @@ __global__ __launch_bounds__(512) void f16_wide_gemm(const uint8_t *__restrict__
 
 #pragma unroll
     for (int s = 0; s < 3; ++s)
-        wf_copy<S, PAIR>(a_off, b_off, a_tile, a_extent, b_tile, b_tile2, b_extent, wid, s * (S::StepK * 2), s);
+        wf_copy<S, PAIR>(a_off, b_off, a_tile, a_extent, b_tile, b_tile2, b_extent, wid,
+                         kk::copied_step(s, steps) * (S::StepK * 2), s);
     __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * (2 + S::BCopies)));
     wd_barrier();
 #pragma unroll

@@ -124,12 +124,16 @@ struct QsRaw {
     uint32_t d[GEN ? 10 : 9];
 };
 
+// The step's offset soff moves GEN's base and extent: its lanes past the matrix (a last step
+// that K does not fill) are past the extent by their own offset. The others read inside a row.
 template <bool GEN>
-__device__ __forceinline__ QsRaw<GEN> qs_load(__amdgpu_buffer_rsrc_t rsrc, uint32_t off, int soff) {
+__device__ __forceinline__ QsRaw<GEN> qs_load(const uint8_t *base, uint32_t extent, uint32_t off, int soff) {
     QsRaw<GEN> r;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(base) + (GEN ? soff : 0), 0, static_cast<int>(GEN ? extent - soff : extent), 0x00020000);
     if constexpr (GEN) {
 #pragma unroll
-        for (int i = 0; i < 10; ++i) r.d[i] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, off + 4 * i, soff, 0);
+        for (int i = 0; i < 10; ++i) r.d[i] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, off + 4 * i, 0, 0);
     } else {
         const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, soff, 0);
         const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off + 16, soff, 0);
@@ -286,9 +290,7 @@ __global__ __launch_bounds__(kQsThreads) void q4_split_gemv(const QsArgs p) {
         const uint32_t pos = mis + static_cast<uint32_t>(min(row, p.n - 1)) * row_bytes + 36u * g;
         const uint32_t off = GEN ? pos & ~3u : pos, shift = pos & 3u;
         // whole dwords up to the one that holds the matrix's last byte
-        const int extent = static_cast<int>((mis + static_cast<uint32_t>(p.n) * row_bytes + 3u) & ~3u);
-        const __amdgpu_buffer_rsrc_t rsrc =
-            __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(m - mis), 0, extent, 0x00020000);
+        const uint32_t extent = (mis + static_cast<uint32_t>(p.n) * row_bytes + 3u) & ~3u;
 
         float4v tot[MT];
 #pragma unroll
@@ -319,7 +321,7 @@ __global__ __launch_bounds__(kQsThreads) void q4_split_gemv(const QsArgs p) {
 #pragma unroll
                     for (int t = 0; t < 8; ++t) v[it][t] = __uint_as_float(order[t]);
                 }
-                raw = qs_load<GEN>(rsrc, off, min(s0, last) * kStepBytes);
+                raw = qs_load<GEN>(m - mis, extent, off, min(s0, last) * kStepBytes);
                 if (c0 != step0) kk::lds_barrier();             // the last chunk's fragments are read
 #pragma unroll
                 for (int it = 0; it < Q::Items; ++it) {
@@ -329,12 +331,12 @@ __global__ __launch_bounds__(kQsThreads) void q4_split_gemv(const QsArgs p) {
                 }
                 kk::lds_barrier();
             } else {
-                raw = qs_load<GEN>(rsrc, off, min(s0, last) * kStepBytes);
+                raw = qs_load<GEN>(m - mis, extent, off, min(s0, last) * kStepBytes);
             }
             for (int s = s0; s < s1; ++s) {
                 qs_step<MT, PACK, GEN>(raw, shift, s, blocks, g, reinterpret_cast<const half8 *>(frag) +
                                        (s - c0) * (kStepBlocks * Q::Frags * kWave) + lane, inv_lds + (s - c0) * Q::Cols, tot);
-                raw = qs_load<GEN>(rsrc, off, min(s + 1, last) * kStepBytes);
+                raw = qs_load<GEN>(m - mis, extent, off, min(s + 1, last) * kStepBytes);
             }
         }
 
