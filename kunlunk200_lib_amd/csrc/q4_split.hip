@@ -179,7 +179,7 @@ __device__ __forceinline__ void qs_convert(const float (&v)[8], int item, int la
     swap16(mb, other);                                          // rows 0 1 and 2 3
     mb = max(mb, other);
     int e = __builtin_amdgcn_frexp_expf(__uint_as_float(mb));
-    e = mb < 0x7f800000u && mb != 0u ? max(min(e, 126), -100) : 14;
+    e = mb < 0x7f800000u && mb != 0u ? max(e, -100) : 14;   // at most 128: 2^(14-e) and 2^(e-14) stay normal
     const float s = ldexpf(1.0f, 14 - e);
     const int step = 2 * pr + (lane >> 5);
     if ((lane & 31) == 0 && step < Q::ChunkSteps) inv_lds[step * Q::Cols + col] = ldexpf(1.0f, e - 14);

@@ -57,6 +57,20 @@ def test_split_nonfinite(gpu, oracle, k, batch):
     assert np.all(np.isfinite(rest[:, rows])) and not np.any(np.isfinite(rest[:, 5]))
 
 
+@pytest.mark.parametrize("k,batch", [(4096, 20), (11008, 6), (1056, 12)])
+def test_split_largest_activations(gpu, oracle, k, batch):
+    # up to the largest F32 value, whose product with a small weight is finite
+    n = 40
+    rng = np.random.default_rng(k + 1)
+    q4 = kl.quantize_q4_0((rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    x = rng.standard_normal((batch, k)).astype(np.float32)
+    x[1, 3], x[2, k - 1], x[batch - 1, 300] = np.finfo(np.float32).max, -np.finfo(np.float32).max, 2.0**127
+    y, _, guard_ok = run_matmul(Q4, q4, x, k, n, batch)
+    dec = oracle.q4_decode(q4, k, n)
+    res = check_f32_accumulate(y, oracle.gold(dec, x, threads=16), dec, x)
+    assert guard_ok and res["finite"] and res["north_star"]
+
+
 @pytest.mark.parametrize("k,n,batch", [(1056, 65, 24), (4096, 300, 32), (11008, 50, 5), (2048, 1000, 30), (96, 20, 40)])
 def test_split_pair(gpu, oracle, k, n, batch):
     rng = np.random.default_rng(k + n + batch)
