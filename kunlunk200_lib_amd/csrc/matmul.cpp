@@ -71,6 +71,10 @@ bool q4_mfma_batch(int batch, bool streamed) {
     return batch >= min_b && batch <= max_b;
 }
 
+// Shapes that the batch-1 and -2 kernels take; the others are F32 arithmetic there
+// (gemv_general), which the K-split kernel follows for an infinite activation.
+bool q4_whole(const void * w, int k) { return k % 64 == 0 && ((uintptr_t)w & 3) == 0; }
+
 // Whether the K-split Q4_0 MFMA GEMV takes a call no faster route took: above
 // 16 columns always; up to 16 the single-pass MFMA GEMV's batch range, where
 // shapes the batch-1 kernels cannot take (K % 64 != 0, weights off a dword)
@@ -78,7 +82,7 @@ bool q4_mfma_batch(int batch, bool streamed) {
 // the general GEMV, 13 / 13 / 14 us split).
 bool q4_split_route(const void * w, int k, int batch) {
     if (batch > 16) return true;
-    const bool whole = k % 64 == 0 && ((uintptr_t)w & 3) == 0;
+    const bool whole = q4_whole(w, k);
     return q4_mfma_batch(batch, !whole || (k % 256 == 0 && ((uintptr_t)w & 15) == 0));
 }
 
@@ -286,7 +290,9 @@ static Q4PairRoute q4_pair_route(const void * w_gate, const void * w_up, const f
     if (kk::q4_bdiag_batch(batch) && kk_q4_bdiag_gemv_supported(w_gate, x, k, n, batch) &&
         kk_q4_bdiag_gemv_supported(w_up, x, k, n, batch))
         return Q4PairRoute::bdiag;
-    if (batch > 16 || (kk::q4_split_route(w_gate, k, batch) && kk::q4_split_route(w_up, k, batch)))
+    // (one matrix on a dword and one off it: each on its own rule for infinities)
+    if (kk::q4_split_route(w_gate, k, batch) && kk::q4_split_route(w_up, k, batch) &&
+        kk::q4_whole(w_gate, k) == kk::q4_whole(w_up, k))
         return Q4PairRoute::split;
     return Q4PairRoute::none;
 }

@@ -37,7 +37,9 @@
 //
 // Scales. Each (column, 256-value step) has its own power of two with
 // max |x * 2^s| < 2^14; a step's sums are multiplied by 2^-s and added to the
-// wave's totals. A step holding Inf or NaN makes its column NaN.
+// wave's totals. A step holding Inf or NaN makes its column NaN; for the shapes the
+// batch-1 kernels leave to F32 arithmetic (K % 64 != 0, weights off a dword) an Inf
+// is multiplied as one instead: +-Inf, NaN where its weight is zero or infinities cancel.
 #include "device_common.h"
 #include "launch.h"
 #include "lds_opt_in.h"
@@ -158,19 +160,24 @@ struct QsArgs {
     int per_group, groups;      // tiles of a workgroup, workgroups per range
     int per_xcd, total;         // workgroups
     int row_stride;             // row stride of `out` (n, or the padded rows of a partial)
+    uint32_t inf_bits;          // GEN: magnitude that is multiplied as infinity (above every value's: none)
 };
 
 // One column's 512 values (two steps; lane: block lane / 4, block positions
 // 8 (lane % 4) ..) into the chunk's A fragments and inverse scales.
-template <int MT, bool PACK>
-__device__ __forceinline__ void qs_convert(const float (&v)[8], int item, int lane, _Float16 *frag, float *inv_lds) {
+template <int MT, bool PACK, bool GEN>
+__device__ __forceinline__ void qs_convert(const float (&v)[8], int item, int lane, uint32_t inf_bits, _Float16 *frag,
+                                           float *inv_lds) {
     using Q = QsShape<MT, PACK>;
     const int col = item % Q::Cols, pr = item / Q::Cols;
     // the largest magnitude of each 32-lane half (one step) as bits: a NaN's
-    // or Inf's are above every finite value's
+    // or Inf's are above every finite value's (inf_bits: an Inf beside finite values does not count)
     uint32_t mb = 0u;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) mb = max(mb, __float_as_uint(v[t]) & 0x7fffffffu);
+    for (int t = 0; t < 8; ++t) {
+        const uint32_t bits = __float_as_uint(v[t]) & 0x7fffffffu;
+        mb = max(mb, GEN && bits == inf_bits ? 0u : bits);
+    }
     mb = max(mb, dpp_u32<0xb1>(mb));
     mb = max(mb, dpp_u32<0x4e>(mb));
     mb = max(mb, dpp_u32<0x141>(mb));
@@ -188,7 +195,8 @@ __device__ __forceinline__ void qs_convert(const float (&v)[8], int item, int la
     for (int t = 0; t < 8; ++t) {
         const float a = v[t] * s;
         hi[t] = static_cast<_Float16>(a);
-        lo[t] = static_cast<_Float16>(a - static_cast<float>(hi[t]));
+        lo[t] = static_cast<_Float16>(GEN && (__float_as_uint(v[t]) & 0x7fffffffu) == inf_bits
+                                          ? 0.0f : a - static_cast<float>(hi[t]));   // Inf - Inf: NaN, the column's
     }
     const int blk = 2 * pr * kStepBlocks + (lane >> 2);
     const int alane = (lane & 3) * 16 + (col & 15);             // A row col % 16, positions 8 (lane % 4) ..
@@ -327,7 +335,7 @@ __global__ __launch_bounds__(kQsThreads) void q4_split_gemv(const QsArgs p) {
                 for (int it = 0; it < Q::Items; ++it) {
                     const int item = wid + kQsWaves * it;       // wave-uniform
                     if (item >= items) break;
-                    qs_convert<MT, PACK>(v[it], item, lane, frag, inv_lds);
+                    qs_convert<MT, PACK, GEN>(v[it], item, lane, p.inf_bits, frag, inv_lds);
                 }
                 kk::lds_barrier();
             } else {
@@ -494,6 +502,7 @@ hipError_t qs_run(const QsPlan &p, const uint8_t *w, const uint8_t *w2, const fl
     a.row_stride = p.part_bytes ? p.stride : n;
     const uintptr_t bits = reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(w2);
     const bool gen = k % kStepK != 0 || (bits & 3) != 0;
+    a.inf_bits = k % 64 != 0 || (bits & 3) != 0 ? 0x7f800000u : 0xffffffffu;
     hipError_t rc = batch <= 8    ? qs_launch_gen<1, true>(a, gen, stream)
                     : batch <= 16 ? qs_launch_gen<1, false>(a, gen, stream)
                                   : qs_launch_gen<2, false>(a, gen, stream);

@@ -44,6 +44,7 @@ namespace kk {
 // aligned weights) and the F32/F16 single-pass MFMA GEMVs.
 int gemm_min_batch();
 bool q4_mfma_batch(int batch, bool streamed);
+bool q4_whole(const void * w, int k);
 bool q4_split_route(const void * w, int k, int batch);
 bool f32_gemm_route(int type, const void * w, const void * x, int batch);
 int gemv_chunk(int type);

@@ -40,21 +40,40 @@ def test_split_shapes(gpu, oracle, k, n, batch, w_offset, x_offset):
     assert guard_ok and res["finite"] and res["north_star"]
 
 
-@pytest.mark.parametrize("k,batch", [(4096, 20), (11008, 6), (1056, 12)])
-def test_split_nonfinite(gpu, oracle, k, batch):
-    # a non-finite activation makes its column NaN and no other; an infinite
-    # block scale makes its row's outputs infinite or NaN and no other's
+# (k, batch, w_offset): 3..63 columns with K % 64 != 0 or weights off a dword follow F32
+# arithmetic in an infinite activation, the others make its column NaN
+@pytest.mark.parametrize("k,batch,w_offset", [(4096, 20, 0), (11008, 6, 0), (4160, 7, 0), (1056, 12, 0), (1056, 5, 0),
+                                              (1056, 40, 0), (512, 9, 2), (4096, 17, 1), (96, 3, 0)])
+def test_split_nonfinite(gpu, oracle, k, batch, w_offset):
+    # a non-finite activation touches its column and no other; an infinite block
+    # scale makes its row's outputs infinite or NaN and no other's
     n = 40
     rng = np.random.default_rng(k)
     q4 = kl.quantize_q4_0((rng.standard_normal((n, k)) * 0.02).astype(np.float32)).reshape(n, k // 32, 18)
     q4[5, k // 32 - 1, :2] = np.array([np.inf], np.float16).view(np.uint8)
+    q4[6, k // 32 - 1, :2] = 0
+    q4[7, k // 32 - 1, 17] = 0x88                  # weight 0 at K - 1
     x = rng.standard_normal((batch, k)).astype(np.float32)
+    x[0] *= 1e30
     x[1, 3], x[2, k - 1] = np.nan, -np.inf
-    y, _, guard_ok = run_matmul(Q4, q4.reshape(n, -1), x, k, n, batch)
+    x[batch - 1, :2] = np.inf, np.inf
+    x[batch - 1, 40] = 3e38
+    payload = q4.reshape(n, -1)
+    y, _, guard_ok = run_matmul(Q4, payload, x, k, n, batch, w_offset=w_offset)
     rows = np.arange(n) != 5
-    assert guard_ok and np.all(np.isnan(y[1])) and np.all(np.isnan(y[2]))
-    rest = np.delete(y, (1, 2), axis=0)
+    assert guard_ok and np.all(np.isnan(y[1]))
+    rest = np.delete(y, (1, 2, batch - 1), axis=0)
     assert np.all(np.isfinite(rest[:, rows])) and not np.any(np.isfinite(rest[:, 5]))
+    w = oracle.q4_decode(payload, k, n).astype(np.float64)
+    if k % 64 == 0 and w_offset % 4 == 0:
+        assert np.all(np.isnan(y[2])) and np.all(np.isnan(y[batch - 1]))
+        return
+    for col in {2, batch - 1}:
+        with np.errstate(invalid="ignore"):
+            want = (w[rows] * x[col].astype(np.float64)).sum(1)
+        got = y[col][rows]
+        assert not np.any(np.isfinite(want)) and np.array_equal(np.isnan(got), np.isnan(want))
+        assert np.array_equal(got[~np.isnan(want)], want[~np.isnan(want)].astype(np.float32)) and np.any(np.isinf(want))
 
 
 @pytest.mark.parametrize("k,batch", [(4096, 20), (11008, 6), (1056, 12)])
