@@ -46,7 +46,8 @@ int kk_swiglu(void *y, const void *gate, const void *up, int width, int rows, in
 // over workgroups (any K % 32 == 0, any weight alignment, 4-byte aligned X);
 // `workspace` of kk_q4_split_workspace_bytes holds partial sums (at most the
 // no-allocation entry point's scratch for one matrix). w_up null: y =
-// X w^T; else y = SiLU(X w^T) * (X w_up^T), both matrices [n,k].
+// X w^T, and a null workspace gives the same sums without one, a tile's K ranges
+// in turn; else y = SiLU(X w^T) * (X w_up^T), both matrices [n,k].
 size_t kk_q4_split_workspace_bytes(int k, int n, int batch, int pair, int cus);
 int kk_q4_split_gemv(const void *w, const void *w_up, const float *x, float *y, int k, int n, int batch,
                      void *workspace, int cus, hipStream_t stream);

@@ -83,10 +83,18 @@ hipError_t small_batch(DeviceScratch &d, int type, const void *w, const float *x
         return static_cast<hipError_t>(kk_q4_bdiag_gemv(w, xf, yf, k, n, batch, d.cus, s));
     }
     if (type == 2 && kk::q4_split_route(w, k, batch)) {
-        const size_t need = kk_q4_split_workspace_bytes(k, n, batch, 0, d.cus);
+        // Calls on the array race where they overlap. Where no kernel before the split one
+        // needed scratch (shapes off the batch-1 kernels; more than 16 columns that fit the
+        // block-diagonal kernel in 16s) none is used here either: one workgroup takes a
+        // tile's ranges in turn, which gives the same sums (us, the kernels before / in turn /
+        // with the array: K5600 x N3000 at 3 columns 27 / 22 / 14, 16 123 / 40 / 15, 32 245 /
+        // 82 / 19, K2048 x N4096 at 32 24 / 18 / 13, but K16352 x N100 at 3 26 / 47 / 12).
+        const bool overlaps = !kk::q4_whole(w, k) || (batch > 16 && kk::q4_bdiag_batch(16) &&
+                                                      kk_q4_bdiag_gemv_supported(w, xf, k, n, 16));
+        const size_t need = overlaps ? 0 : kk_q4_split_workspace_bytes(k, n, batch, 0, d.cus);
         if (need > kScratchBytes) return static_cast<hipError_t>(too_large(need));
         *taken = "q4_mfma_gemv";
-        return static_cast<hipError_t>(kk_q4_split_gemv(w, nullptr, xf, yf, k, n, batch, d.ptr, d.cus, s));
+        return static_cast<hipError_t>(kk_q4_split_gemv(w, nullptr, xf, yf, k, n, batch, overlaps ? nullptr : d.ptr, d.cus, s));
     }
     return static_cast<hipError_t>(kk_dense_matmul(type, w, xf, yf, k, n, batch, s, taken));
 }

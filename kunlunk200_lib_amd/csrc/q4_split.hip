@@ -159,6 +159,7 @@ struct QsArgs {
     int tiles;                  // 16-row tiles of one matrix
     int per_group, groups;      // tiles of a workgroup, workgroups per range
     int per_xcd, total;         // workgroups
+    int at_once;                // SERIAL: ranges at a time
     int row_stride;             // row stride of `out` (n, or the padded rows of a partial)
     uint32_t inf_bits;          // GEN: magnitude that is multiplied as infinity (above every value's: none)
 };
@@ -262,26 +263,30 @@ __device__ __forceinline__ void qs_step(const QsRaw<GEN> &raw, uint32_t shift, i
 
 // GEN: any K % 32 == 0 and any weight alignment (dword loads, byte shifts,
 // blocks past K masked); else K % 256 == 0 and 4-byte aligned weights.
-template <int MT, bool PACK, bool GEN>
+// SERIAL (one matrix, one tile per wave): a workgroup takes its tiles' ranges in turn, at_once
+// of them at a time (whose fragments fit one chunk), and adds their sums in range order, as
+// q4_split_sum does, so that no partial sum leaves it.
+template <int MT, bool PACK, bool GEN, bool SERIAL>
 __global__ __launch_bounds__(kQsThreads) void q4_split_gemv(const QsArgs p) {
     using Q = QsShape<MT, PACK>;
     extern __shared__ __align__(16) uint8_t qs_lds[];
     const int bid = blockIdx.x;
     const int idx = (bid % kXcds) * p.per_xcd + bid / kXcds;    // contiguous ranges per XCD share X in its L2
     if (idx >= p.total) return;                                 // whole workgroup, before any barrier
-    const int range = idx / p.groups;
-    const int group = idx - range * p.groups;
+    const int range0 = SERIAL ? 0 : idx / p.groups, range1 = SERIAL ? p.ranges : range0 + 1;
+    const int group = SERIAL ? idx : idx - range0 * p.groups;
     const int lane = threadIdx.x & (kWave - 1);
     const int wid = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
     const int c16 = lane & 15, g = lane >> 4;
-    const int tw = kQsWaves / p.kgroups;                        // waves along the tiles
-    const int wt = wid % tw, kg = wid / tw;
-    const int step0 = p.steps * range / p.ranges, step1 = p.steps * (range + 1) / p.ranges;
+    const int at_once = SERIAL ? p.at_once : 1;
+    const int tw = kQsWaves / (p.kgroups * at_once);            // waves along the tiles
+    const int wt = wid % tw, kg = SERIAL ? wid / tw % p.kgroups : wid / tw;
+    const int slot = SERIAL ? wid / (tw * p.kgroups) : 0;       // the wave's range of those at a time
     const int blocks = p.k >> 5;
     const uint32_t row_bytes = static_cast<uint32_t>(blocks) * 18u;
     const int all_tiles = p.w2 ? 2 * p.tiles : p.tiles;         // the gate matrix's tiles, then the up matrix's
     const int first = group * p.per_group, end = min(first + p.per_group, all_tiles);
-    const int rounds = (p.per_group + tw - 1) / tw;             // tiles per wave (1 with several chunks)
+    const int rounds = SERIAL ? 1 : (p.per_group + tw - 1) / tw;   // tiles per wave (1 with several chunks)
 
     _Float16 *frag = reinterpret_cast<_Float16 *>(qs_lds);
     float *inv_lds = reinterpret_cast<float *>(qs_lds + Q::ChunkSteps * Q::StepBytes);
@@ -300,82 +305,109 @@ __global__ __launch_bounds__(kQsThreads) void q4_split_gemv(const QsArgs p) {
         // whole dwords up to the one that holds the matrix's last byte
         const uint32_t extent = (mis + static_cast<uint32_t>(p.n) * row_bytes + 3u) & ~3u;
 
-        float4v tot[MT];
+        float4v sum[MT];                                        // SERIAL: the ranges'
 #pragma unroll
-        for (int t = 0; t < MT; ++t) tot[t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int t = 0; t < MT; ++t) sum[t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int range = range0; range < range1; range += at_once) {
+            const int here = SERIAL ? min(at_once, range1 - range) : 1;
+            const int step0 = p.steps * range / p.ranges, step1 = p.steps * (range + here) / p.ranges;
+            float4v tot[MT];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) tot[t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
 
-        for (int c0 = step0; c0 < step1; c0 += Q::ChunkSteps) {
-            const int csteps = min(Q::ChunkSteps, step1 - c0);
-            const int s0 = c0 + csteps * kg / p.kgroups;
-            const int s1 = live ? c0 + csteps * (kg + 1) / p.kgroups : s0;
-            const int last = max(s1 - 1, c0);                   // past the end: re-read, not used
-            QsRaw<GEN> raw;
-            if (round == 0) {
-                // X of this chunk, then the first weight step: the memory counter
-                // is in order, so waiting for X leaves the weights in flight
-                const int items = Q::Cols * ((csteps + 1) >> 1);
-                float v[Q::Items][8];
-#pragma unroll
-                for (int it = 0; it < Q::Items; ++it) {
-                    const int item = wid + kQsWaves * it;
-                    const int col = item % Q::Cols, pr = item / Q::Cols;
-                    const int blk = (c0 + 2 * pr) * kStepBlocks + (lane >> 2);   // lane: block lane / 4, dword lane % 4
-                    const bool in = item < items && col < p.batch && blk < blocks && blk < (c0 + csteps) * kStepBlocks;
-                    // outside: past the extent, zeros without a memory access
-                    const uint32_t xo = in ? (static_cast<uint32_t>(col) * p.k + 32 * blk + 4 * (lane & 3)) * 4u : 0x80000000u;
-                    const u32x4 lo = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xo, 0, 0);
-                    const u32x4 hi = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xo, 64, 0);
-                    const uint32_t order[8] = {lo[0], lo[2], lo[1], lo[3], hi[0], hi[2], hi[1], hi[3]};
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) v[it][t] = __uint_as_float(order[t]);
+            for (int c0 = step0; c0 < step1; c0 += Q::ChunkSteps) {
+                const int csteps = min(Q::ChunkSteps, step1 - c0);
+                int from = c0, count = csteps;                  // the k-groups' steps of this chunk
+                if (SERIAL && at_once > 1) {                    // one chunk: this wave's range of it
+                    from = p.steps * min(range + slot, range1) / p.ranges;
+                    count = p.steps * min(range + slot + 1, range1) / p.ranges - from;
                 }
-                raw = qs_load<GEN>(m - mis, extent, off, min(s0, last) * kStepBytes);
-                if (c0 != step0) kk::lds_barrier();             // the last chunk's fragments are read
+                const int s0 = from + count * kg / p.kgroups;
+                const int s1 = live ? from + count * (kg + 1) / p.kgroups : s0;
+                const int last = max(s1 - 1, c0);                   // past the end: re-read, not used
+                QsRaw<GEN> raw;
+                if (round == 0) {
+                    // X of this chunk, then the first weight step: the memory counter
+                    // is in order, so waiting for X leaves the weights in flight
+                    const int items = Q::Cols * ((csteps + 1) >> 1);
+                    float v[Q::Items][8];
 #pragma unroll
-                for (int it = 0; it < Q::Items; ++it) {
-                    const int item = wid + kQsWaves * it;       // wave-uniform
-                    if (item >= items) break;
-                    qs_convert<MT, PACK, GEN>(v[it], item, lane, p.inf_bits, frag, inv_lds);
+                    for (int it = 0; it < Q::Items; ++it) {
+                        const int item = wid + kQsWaves * it;
+                        const int col = item % Q::Cols, pr = item / Q::Cols;
+                        const int blk = (c0 + 2 * pr) * kStepBlocks + (lane >> 2);   // lane: block lane / 4, dword lane % 4
+                        const bool in = item < items && col < p.batch && blk < blocks && blk < (c0 + csteps) * kStepBlocks;
+                        // outside: past the extent, zeros without a memory access
+                        const uint32_t xo = in ? (static_cast<uint32_t>(col) * p.k + 32 * blk + 4 * (lane & 3)) * 4u : 0x80000000u;
+                        const u32x4 lo = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xo, 0, 0);
+                        const u32x4 hi = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xo, 64, 0);
+                        const uint32_t order[8] = {lo[0], lo[2], lo[1], lo[3], hi[0], hi[2], hi[1], hi[3]};
+#pragma unroll
+                        for (int t = 0; t < 8; ++t) v[it][t] = __uint_as_float(order[t]);
+                    }
+                    raw = qs_load<GEN>(m - mis, extent, off, min(s0, last) * kStepBytes);
+                    if (c0 != step0 || (SERIAL && range > 0)) kk::lds_barrier();   // the last chunk's fragments are read
+#pragma unroll
+                    for (int it = 0; it < Q::Items; ++it) {
+                        const int item = wid + kQsWaves * it;       // wave-uniform
+                        if (item >= items) break;
+                        qs_convert<MT, PACK, GEN>(v[it], item, lane, p.inf_bits, frag, inv_lds);
+                    }
+                    kk::lds_barrier();
+                } else {
+                    raw = qs_load<GEN>(m - mis, extent, off, min(s0, last) * kStepBytes);
                 }
-                kk::lds_barrier();
-            } else {
-                raw = qs_load<GEN>(m - mis, extent, off, min(s0, last) * kStepBytes);
+                for (int s = s0; s < s1; ++s) {
+                    qs_step<MT, PACK, GEN>(raw, shift, s, blocks, g, reinterpret_cast<const half8 *>(frag) +
+                                           (s - c0) * (kStepBlocks * Q::Frags * kWave) + lane, inv_lds + (s - c0) * Q::Cols, tot);
+                    raw = qs_load<GEN>(m - mis, extent, off, min(s + 1, last) * kStepBytes);
+                }
             }
-            for (int s = s0; s < s1; ++s) {
-                qs_step<MT, PACK, GEN>(raw, shift, s, blocks, g, reinterpret_cast<const half8 *>(frag) +
-                                       (s - c0) * (kStepBlocks * Q::Frags * kWave) + lane, inv_lds + (s - c0) * Q::Cols, tot);
-                raw = qs_load<GEN>(m - mis, extent, off, min(s + 1, last) * kStepBytes);
-            }
-        }
 
-        // k-groups 1 .. KG-1 hand their sums to k-group 0, which adds them in
-        // order (with several rounds the fragments stay: the exchange has LDS of its own)
-        if (p.kgroups > 1) {
-            float4v *xfer = reinterpret_cast<float4v *>(qs_lds + Q::RingBytes);
-            if (round > 0) __syncthreads();                     // the round before's sums are read
-            if (kg > 0) {
+            // k-groups 1 .. KG-1 hand their sums to k-group 0, which adds them in
+            // order (with several rounds the fragments stay: the exchange has LDS of its own)
+            if (p.kgroups > 1) {
+                float4v *xfer = reinterpret_cast<float4v *>(qs_lds + Q::RingBytes);
+                if (round > 0) __syncthreads();                     // the round before's sums are read
+                if (kg > 0) {
 #pragma unroll
-                for (int t = 0; t < MT; ++t) xfer[((wid - tw) * MT + t) * kWave + lane] = tot[t];
+                    for (int t = 0; t < MT; ++t) xfer[((wid - tw) * MT + t) * kWave + lane] = tot[t];
+                }
+                __syncthreads();
+                if (kg == 0)
+                    for (int h = 1; h < p.kgroups; ++h)
+#pragma unroll
+                        for (int t = 0; t < MT; ++t) tot[t] += xfer[((wid + (h - 1) * tw) * MT + t) * kWave + lane];
             }
-            __syncthreads();
-            if (kg == 0)
-                for (int h = 1; h < p.kgroups; ++h)
+            if constexpr (PACK) {
+                // A rows 8..15 (lanes 32..63) are the lo parts of columns 0..7
 #pragma unroll
-                    for (int t = 0; t < MT; ++t) tot[t] += xfer[(((h - 1) * tw + wt) * MT + t) * kWave + lane];
-        }
-        if constexpr (PACK) {
-            // A rows 8..15 (lanes 32..63) are the lo parts of columns 0..7
+                for (int r = 0; r < 4; ++r) tot[0][r] += __shfl_down(tot[0][r], 32);
+            }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) tot[0][r] += __shfl_down(tot[0][r], 32);
+            for (int t = 0; t < MT; ++t) sum[t] = SERIAL ? sum[t] + tot[t] : tot[t];
+            if (SERIAL && at_once > 1) {
+                // slots 1 .. hand theirs to slot 0 (in places that no k-group used)
+                float4v *xfer = reinterpret_cast<float4v *>(qs_lds + Q::RingBytes);
+                if (slot > 0 && kg == 0) {
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) xfer[((wid - tw) * MT + t) * kWave + lane] = tot[t];
+                }
+                __syncthreads();
+                if (slot == 0 && kg == 0)
+                    for (int h = 1; h < here; ++h)
+#pragma unroll
+                        for (int t = 0; t < MT; ++t) sum[t] += xfer[((wid + (h * p.kgroups - 1) * tw) * MT + t) * kWave + lane];
+            }
         }
-        if (live && kg == 0 && row < p.n && !(PACK && g >= 2)) {
-            float *out = p.out + (static_cast<size_t>(range) * (p.w2 ? 2 : 1) + (up ? 1 : 0)) * p.batch * p.row_stride + row;
+        if (live && kg == 0 && slot == 0 && row < p.n && !(PACK && g >= 2)) {
+            float *out = p.out + (SERIAL ? 0 : static_cast<size_t>(range0) * (p.w2 ? 2 : 1) + (up ? 1 : 0)) * p.batch * p.row_stride + row;
 #pragma unroll
             for (int t = 0; t < MT; ++t)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int col = 16 * t + 4 * g + r;
-                    if (col < p.batch) out[static_cast<size_t>(col) * p.row_stride] = tot[t][r];
+                    if (col < p.batch) out[static_cast<size_t>(col) * p.row_stride] = sum[t][r];
                 }
         }
     }
@@ -431,6 +463,12 @@ int floor_pow2(int v) {
     return p;
 }
 
+// Steps whose fragments fit in LDS.
+int qs_chunk(int batch) {
+    return batch <= 8    ? QsShape<1, true>::ChunkSteps
+           : batch <= 16 ? QsShape<1, false>::ChunkSteps : QsShape<2, false>::ChunkSteps;
+}
+
 // S: at most 6 steps (1536 values) per range, 4 above 16 columns, as a power of
 // two, so that the fragments fit one chunk and the ranges' workgroups fill the
 // CUs; up to 8 steps in one range where they fit one chunk, which saves the
@@ -444,8 +482,7 @@ int floor_pow2(int v) {
 QsPlan qs_plan(int k, int n, int batch, bool pair, int cus) {
     QsPlan p;
     const int steps = (k + kStepK - 1) / kStepK;
-    const int chunk = batch <= 8 ? QsShape<1, true>::ChunkSteps
-                      : batch <= 16 ? QsShape<1, false>::ChunkSteps : QsShape<2, false>::ChunkSteps;
+    const int chunk = qs_chunk(batch);
     p.stride = (n + 3) & ~3;
     p.ranges = 1;
     if (steps > 8 || steps > chunk)
@@ -466,28 +503,31 @@ QsPlan qs_plan(int k, int n, int batch, bool pair, int cus) {
     return p;
 }
 
-template <int MT, bool PACK, bool GEN>
+template <int MT, bool PACK, bool GEN, bool SERIAL>
 hipError_t qs_launch(const QsArgs &a, hipStream_t stream) {
     using Q = QsShape<MT, PACK>;
-    const hipError_t rc = kk::opt_in_lds(reinterpret_cast<const void *>(&q4_split_gemv<MT, PACK, GEN>), Q::LdsBytes);
+    const hipError_t rc = kk::opt_in_lds(reinterpret_cast<const void *>(&q4_split_gemv<MT, PACK, GEN, SERIAL>), Q::LdsBytes);
     if (rc != hipSuccess) return rc;
-    hipLaunchKernelGGL((q4_split_gemv<MT, PACK, GEN>), dim3(a.per_xcd * kXcds), dim3(kQsThreads), Q::LdsBytes, stream, a);
+    hipLaunchKernelGGL((q4_split_gemv<MT, PACK, GEN, SERIAL>), dim3(a.per_xcd * kXcds), dim3(kQsThreads), Q::LdsBytes, stream, a);
     return hipGetLastError();
 }
 
 template <int MT, bool PACK>
-hipError_t qs_launch_gen(const QsArgs &a, bool gen, hipStream_t stream) {
-    return gen ? qs_launch<MT, PACK, true>(a, stream) : qs_launch<MT, PACK, false>(a, stream);
+hipError_t qs_launch_form(const QsArgs &a, bool gen, bool serial, hipStream_t stream) {
+    if (serial) return gen ? qs_launch<MT, PACK, true, true>(a, stream) : qs_launch<MT, PACK, false, true>(a, stream);
+    return gen ? qs_launch<MT, PACK, true, false>(a, stream) : qs_launch<MT, PACK, false, false>(a, stream);
 }
 
-// Runs `p` (w2 null: one matrix); `workspace` holds p.part_bytes.
+// Runs `p` (w2 null: one matrix); `workspace` holds p.part_bytes, or is null for one matrix:
+// then the ranges of a tile run in one workgroup, with the same sums.
 hipError_t qs_run(const QsPlan &p, const uint8_t *w, const uint8_t *w2, const float *x, float *y, int k, int n,
-                  int batch, void *workspace, hipStream_t stream) {
+                  int batch, void *workspace, int cus, hipStream_t stream) {
     QsArgs a;
     a.w = w;
     a.w2 = w2;
     a.x = x;
-    a.out = p.part_bytes ? static_cast<float *>(workspace) : y;
+    const bool serial = p.part_bytes && !workspace, split = p.part_bytes && workspace;
+    a.out = split ? static_cast<float *>(workspace) : y;
     a.k = k;
     a.n = n;
     a.batch = batch;
@@ -497,16 +537,23 @@ hipError_t qs_run(const QsPlan &p, const uint8_t *w, const uint8_t *w2, const fl
     a.tiles = p.tiles;
     a.per_group = p.per_group;
     a.groups = p.groups;
-    a.total = p.groups * p.ranges;
+    a.at_once = 1;
+    if (serial) {   // one tile per wave, over all of K; the waves that the CUs' tiles leave idle take more ranges at a time
+        a.per_group = std::min(kQsWaves / p.kgroups, (p.tiles + cus - 1) / cus);
+        a.groups = (p.tiles + a.per_group - 1) / a.per_group;
+        const int fit = qs_chunk(batch) / ((a.steps + p.ranges - 1) / p.ranges);
+        while (2 * a.at_once <= std::min(fit, p.ranges) && 2 * a.at_once * p.kgroups * a.per_group <= kQsWaves) a.at_once *= 2;
+    }
+    a.total = serial ? a.groups : p.groups * p.ranges;
     a.per_xcd = (a.total + kXcds - 1) / kXcds;
-    a.row_stride = p.part_bytes ? p.stride : n;
+    a.row_stride = split ? p.stride : n;
     const uintptr_t bits = reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(w2);
     const bool gen = k % kStepK != 0 || (bits & 3) != 0;
     a.inf_bits = k % 64 != 0 || (bits & 3) != 0 ? 0x7f800000u : 0xffffffffu;
-    hipError_t rc = batch <= 8    ? qs_launch_gen<1, true>(a, gen, stream)
-                    : batch <= 16 ? qs_launch_gen<1, false>(a, gen, stream)
-                                  : qs_launch_gen<2, false>(a, gen, stream);
-    if (rc != hipSuccess || !p.part_bytes) return rc;
+    hipError_t rc = batch <= 8    ? qs_launch_form<1, true>(a, gen, serial, stream)
+                    : batch <= 16 ? qs_launch_form<1, false>(a, gen, serial, stream)
+                                  : qs_launch_form<2, false>(a, gen, serial, stream);
+    if (rc != hipSuccess || !split) return rc;
     const int threads = batch * (p.stride / 4);
     const dim3 grid((threads + kSumThreads - 1) / kSumThreads), block(kSumThreads);
     if (w2)
@@ -530,7 +577,7 @@ extern "C" int kk_q4_split_gemv(const void *w, const void *w_up, const float *x,
         static_cast<size_t>(n) * (k / 32 * 18) > 0x7fffffffu || (reinterpret_cast<uintptr_t>(x) & 3))
         return hipErrorInvalidValue;
     const QsPlan p = qs_plan(k, n, batch, w_up != nullptr, cus);
-    if (p.part_bytes && !workspace) return hipErrorInvalidValue;
+    if (p.part_bytes && !workspace && w_up) return hipErrorInvalidValue;
     return qs_run(p, static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(w_up), x, y, k, n, batch, workspace,
-                  stream);
+                  cus, stream);
 }

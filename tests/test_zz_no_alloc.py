@@ -23,7 +23,10 @@ CASES = [
     (Q4, "q4_stream_gemv", (4096, 2048, 8), (4096, 300, 5)),      # streamed MFMA GEMV (K = 4096), no scratch
     (Q4, "q4_bdiag_gemv", (1024, 2048, 8), (1024, 300, 4)),       # block-diagonal MFMA GEMV, no scratch
     (Q4, "q4_mfma_gemv", (4096, 2048, 16), (4096, 300, 12)),      # LDS-staged MFMA GEMV, scratch: X fragments
-    (Q4, "q4_mfma_gemv", (4096, 520, 40), (4096, 300, 33)),       # chunks of 16 columns, the array reused in order
+    (Q4, "q4_mfma_gemv", (4096, 520, 40), (4096, 300, 33)),       # chunks of 32 columns, the array reused in order
+    (Q4, "q4_mfma_gemv", (5600, 2999, 24), (1056, 300, 9)),       # K % 64 != 0: K ranges in turn, no scratch
+    (Q4, "q4_mfma_gemv", (11040, 65, 63), (16352, 17, 5)),        # likewise, a pass of 32 and one of 31, up to 16 ranges
+    (Q4, "q4_mfma_gemv", (2048, 5000, 32), (1088, 100, 17)),      # more than 16 columns of a block-diagonal shape, no scratch
     (Q4, "q4_gemv_dot8", (4096, 1024, 1), (1024, 129, 1)),        # no scratch
     (F32, "f32_mfma_gemv", (1024, 256, 8), (512, 65, 2)),         # no scratch
 ]
@@ -101,8 +104,10 @@ hip.hipStreamCreate.argtypes = [ctypes.POINTER(ctypes.c_void_p)]
 hip.hipStreamSynchronize.argtypes = [ctypes.c_void_p]
 hip.hipStreamDestroy.argtypes = [ctypes.c_void_p]
 Q4, F32 = kl.WeightType.q4_0, kl.WeightType.f32
-# scratch-free routes: batch-1 dot8, block-diagonal, F32 MFMA, streamed Q4_0, F32 MFMA (small)
-CASES = [(Q4, 4096, 3000, 1), (Q4, 1024, 2048, 4), (F32, 1024, 256, 8), (Q4, 4096, 1000, 8), (F32, 512, 65, 2)]
+# scratch-free routes: batch-1 dot8, block-diagonal, F32 MFMA, streamed Q4_0, F32 MFMA (small), K-split
+# Q4_0 with its K ranges in turn (K % 64 != 0; 17 .. 63 columns of a block-diagonal shape)
+CASES = [(Q4, 4096, 3000, 1), (Q4, 1024, 2048, 4), (F32, 1024, 256, 8), (Q4, 4096, 1000, 8), (F32, 512, 65, 2),
+         (Q4, 5600, 2999, 16), (Q4, 5600, 1500, 32), (Q4, 2976, 3001, 7), (Q4, 2048, 4096, 48)]
 rng = np.random.default_rng(7)
 jobs = []
 for type_, k, n, batch in CASES:
@@ -125,9 +130,9 @@ start = threading.Barrier(2)
 
 def worker(t):
     kl.select(0)
-    order = range(len(jobs)) if t == 0 else reversed(range(len(jobs)))
+    order = list(range(len(jobs))) if t == 0 else list(reversed(range(len(jobs))))
     start.wait()
-    for i in order:
+    for i in 20 * order:
         type_, k, n, batch, wb, xb = jobs[i]
         status[t][i] = kl.matmul_noalloc(0, outs[t][i].data, wb.data, xb.data, k, n, batch, type_, streams[t].value)
     assert hip.hipStreamSynchronize(streams[t]) == 0
