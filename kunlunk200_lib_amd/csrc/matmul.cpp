@@ -75,15 +75,26 @@ bool q4_mfma_batch(int batch, bool streamed) {
 // (gemv_general), which the K-split kernel follows for an infinite activation.
 bool q4_whole(const void * w, int k) { return k % 64 == 0 && ((uintptr_t)w & 3) == 0; }
 
-// Whether the K-split Q4_0 MFMA GEMV takes a call no faster route took: above
-// 16 columns always; up to 16 the single-pass MFMA GEMV's batch range, where
-// shapes the batch-1 kernels cannot take (K % 64 != 0, weights off a dword)
+// Whether the K-split Q4_0 MFMA GEMV may take a call (or a gate/up pair) that no faster
+// route took: above 16 columns always; up to 16 the single-pass MFMA GEMV's batch range,
+// where shapes the batch-1 kernels cannot take (K % 64 != 0, weights off a dword)
 // count from 3 columns (K5600 x N3000: 3 / 8 / 16 columns 27 / 63 / 123 us on
 // the general GEMV, 13 / 13 / 14 us split).
-bool q4_split_route(const void * w, int k, int batch) {
+bool q4_split_range(const void * w, int k, int batch) {
     if (batch > 16) return true;
     const bool whole = q4_whole(w, k);
     return q4_mfma_batch(batch, !whole || (k % 256 == 0 && ((uintptr_t)w & 15) == 0));
+}
+
+// One matrix: not where the general GEMV has little to do. It gives a wave one row of 64
+// blocks at a time and up to 8 columns per pass, so its time goes with those passes x
+// columns x the workgroups (4 rows) that share a CU. us general / split at N300, N1000:
+// K544 8 columns 7.3 / 8.1, K1056 3 columns 6.7 / 8.9, 8 columns 8.5 / 8.9, 12 columns
+// 12.6 / 9.5; K2976 (two passes) 3 columns 8.6 / 11.6, 5 columns 11.3 / 11.7, 6 columns
+// 12.6 / 11.7; K4128 3 columns 11.2 / 11.2; at N3000 K544 3 columns 7.7 / 8.2, 4 columns 8.9 / 8.2.
+bool q4_split_route(const void * w, int k, int n, int batch, int cus) {
+    const long general = (k + 2047L) / 2048 * batch * ((n + 4L * cus - 1) / (4L * cus));
+    return q4_split_range(w, k, batch) && (q4_whole(w, k) || batch > 8 || general > 10);
 }
 
 // F32 weights above the single-pass GEMV's 16 columns (K4096 x N4096 at 17
@@ -209,7 +220,7 @@ static void dispatch_dense(Kernel::Impl & impl, detail::DeviceContext & ctx, int
                                                        batch, ctx.cus, ctx.stream),
                           "kk_q4_bdiag_gemv");
         impl.route = "q4_bdiag_gemv";
-    } else if (type == WeightType::q4_0 && kk::q4_split_route(w, k, batch)) {
+    } else if (type == WeightType::q4_0 && kk::q4_split_route(w, k, n, batch, ctx.cus)) {
         grow_split(id, ctx, impl, kk_q4_split_workspace_bytes(k, n, batch, 0, ctx.cus));
         detail::check_hip((hipError_t)kk_q4_split_gemv(w, nullptr, static_cast<const float *>(x),
                                                        static_cast<float *>(y), k, n, batch, impl.gemm_workspace,
@@ -291,7 +302,7 @@ static Q4PairRoute q4_pair_route(const void * w_gate, const void * w_up, const f
         kk_q4_bdiag_gemv_supported(w_up, x, k, n, batch))
         return Q4PairRoute::bdiag;
     // (one matrix on a dword and one off it: each on its own rule for infinities)
-    if (kk::q4_split_route(w_gate, k, batch) && kk::q4_split_route(w_up, k, batch) &&
+    if (kk::q4_split_range(w_gate, k, batch) && kk::q4_split_range(w_up, k, batch) &&
         kk::q4_whole(w_gate, k) == kk::q4_whole(w_up, k))
         return Q4PairRoute::split;
     return Q4PairRoute::none;

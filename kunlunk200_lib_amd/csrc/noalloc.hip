@@ -82,7 +82,7 @@ hipError_t small_batch(DeviceScratch &d, int type, const void *w, const float *x
         *taken = "q4_bdiag_gemv";
         return static_cast<hipError_t>(kk_q4_bdiag_gemv(w, xf, yf, k, n, batch, d.cus, s));
     }
-    if (type == 2 && kk::q4_split_route(w, k, batch)) {
+    if (type == 2 && kk::q4_split_route(w, k, n, batch, d.cus)) {
         // Calls on the array race where they overlap. Where no kernel before the split one
         // needed scratch (shapes off the batch-1 kernels; more than 16 columns that fit the
         // block-diagonal kernel in 16s) none is used here either: one workgroup takes a

@@ -17,16 +17,23 @@ pytestmark = pytest.mark.gpu
 
 Q4 = kl.WeightType.q4_0
 
-# (k, n, batch, w_offset, x_offset)
-SHAPES = [(32, 7, 9, 0, 0), (96, 33, 17, 0, 0), (544, 70, 3, 0, 0), (1056, 65, 24, 0, 0),    # K % 64 == 32
-          (2048, 129, 20, 2, 0), (1024, 50, 12, 1, 0), (512, 40, 7, 3, 4), (4096, 33, 31, 4, 8),   # misaligned
-          (4096, 16, 16, 0, 0), (4096, 17, 32, 0, 0), (4096, 300, 33, 0, 0), (4096, 300, 63, 0, 0),
-          (11008, 257, 8, 0, 0), (11008, 40, 12, 0, 0), (16384, 48, 32, 0, 0), (2304, 33000, 32, 0, 0),
-          (512, 20000, 30, 0, 0), (8192, 1, 5, 0, 0)]
+SPLIT, GENERAL = "q4_mfma_gemv", "gemv_general"
+
+# (k, n, batch, w_offset, x_offset, route): the route of the first pass of 32 columns
+SHAPES = [(32, 7, 9, 0, 0, SPLIT), (96, 33, 17, 0, 0, SPLIT), (1056, 65, 24, 0, 0, SPLIT),      # K % 64 == 32
+          (544, 7000, 3, 0, 0, SPLIT), (4128, 70, 4, 0, 0, SPLIT),
+          # misaligned
+          (2048, 129, 20, 2, 0, SPLIT), (1024, 50, 12, 1, 0, SPLIT), (5120, 40, 7, 3, 4, SPLIT), (4096, 33, 31, 4, 8, SPLIT),
+          (4096, 16, 16, 0, 0, SPLIT), (4096, 17, 32, 0, 0, SPLIT), (4096, 300, 33, 0, 0, SPLIT), (4096, 300, 63, 0, 0, SPLIT),
+          (11008, 257, 8, 0, 0, SPLIT), (11008, 40, 12, 0, 0, SPLIT), (16384, 48, 32, 0, 0, SPLIT),
+          (2304, 33000, 32, 0, 0, SPLIT), (512, 20000, 30, 0, 0, SPLIT), (8192, 1, 5, 0, 0, SPLIT),
+          # shapes off the batch-1 kernels with little work: a wave's row per pass of 64 blocks and 8 columns
+          (544, 70, 3, 0, 0, GENERAL), (512, 40, 7, 3, 4, GENERAL), (1056, 1000, 8, 0, 0, GENERAL), (1056, 1000, 9, 0, 0, SPLIT),
+          (2976, 300, 5, 0, 0, GENERAL), (2976, 300, 6, 0, 0, SPLIT), (2976, 1100, 3, 0, 0, SPLIT)]
 
 
-@pytest.mark.parametrize("k,n,batch,w_offset,x_offset", SHAPES)
-def test_split_shapes(gpu, oracle, k, n, batch, w_offset, x_offset):
+@pytest.mark.parametrize("k,n,batch,w_offset,x_offset,expected", SHAPES)
+def test_split_shapes(gpu, oracle, k, n, batch, w_offset, x_offset, expected):
     rng = np.random.default_rng(k + 3 * n + batch)
     q4 = kl.quantize_q4_0((rng.standard_normal((n, k)) * 0.02).astype(np.float32))
     x = rng.standard_normal((batch, k)).astype(np.float32)
@@ -36,14 +43,14 @@ def test_split_shapes(gpu, oracle, k, n, batch, w_offset, x_offset):
     dec = oracle.q4_decode(q4, k, n)
     res = check_f32_accumulate(y, oracle.gold(dec, x, threads=16), dec, x)
     print(f"  split k={k} n={n} b={batch} route={route} {res}", flush=True)
-    assert route in ("q4_mfma_gemv", "q4_bdiag_gemv", "q4_stream_gemv")
+    assert route == expected
     assert guard_ok and res["finite"] and res["north_star"]
 
 
 # (k, batch, w_offset): 3..63 columns with K % 64 != 0 or weights off a dword follow F32
 # arithmetic in an infinite activation, the others make its column NaN
-@pytest.mark.parametrize("k,batch,w_offset", [(4096, 20, 0), (11008, 6, 0), (4160, 7, 0), (1056, 12, 0), (1056, 5, 0),
-                                              (1056, 40, 0), (512, 9, 2), (4096, 17, 1), (96, 3, 0)])
+@pytest.mark.parametrize("k,batch,w_offset", [(4096, 20, 0), (11008, 6, 0), (4160, 7, 0), (1056, 12, 0), (5600, 5, 0),
+                                              (1056, 40, 0), (512, 9, 2), (4096, 17, 1), (4128, 4, 0), (96, 3, 0)])
 def test_split_nonfinite(gpu, oracle, k, batch, w_offset):
     # a non-finite activation touches its column and no other; an infinite block
     # scale makes its row's outputs infinite or NaN and no other's
@@ -57,7 +64,7 @@ def test_split_nonfinite(gpu, oracle, k, batch, w_offset):
     x[0] *= 1e30
     x[1, 3], x[2, k - 1] = np.nan, -np.inf
     x[batch - 1, :2] = np.inf, np.inf
-    x[batch - 1, 40] = 3e38
+    x[batch - 1, 40] = 1e37
     payload = q4.reshape(n, -1)
     y, _, guard_ok = run_matmul(Q4, payload, x, k, n, batch, w_offset=w_offset)
     rows = np.arange(n) != 5
