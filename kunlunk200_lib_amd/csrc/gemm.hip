@@ -359,7 +359,7 @@ constexpr size_t gemm_lds_bytes() {
 // tile from matrix (j >> 5) & 1, so each wave's first 32-column MFMA tile is
 // gate and its second is up for the same 32 output columns, and the epilogue
 // writes y = SiLU(gate) * up.
-template <bool F16W, int BN, bool PAIR>
+template <bool F16W, int BN, bool PAIR, bool SPLIT>
 __global__ __launch_bounds__(kGemmThreads) void mfma_gemm(const uint8_t *__restrict__ w,
                                                          const uint8_t *__restrict__ w2,
                                                          const _Float16 *__restrict__ x16,
@@ -379,17 +379,21 @@ __global__ __launch_bounds__(kGemmThreads) void mfma_gemm(const uint8_t *__restr
     int tile = (bid % kXcds) * tiles_per_xcd + bid / kXcds;
     if (tile >= tiles) return;                           // whole workgroup, before any barrier
     const size_t row_bytes = F16W ? static_cast<size_t>(k) * 2 : static_cast<size_t>(k >> 5) * 18;
-    // this workgroup's K range (all of K without a split): from here on k, the
-    // weight rows and the activations begin there
-    const int range = tile / range_tiles;
-    tile -= range * range_tiles;
-    const int k0 = range * range_k;
-    k = min(range_k, k - k0);
-    const size_t w_skip = F16W ? static_cast<size_t>(k0) * 2 : static_cast<size_t>(k0 >> 5) * 18;
-    w += w_skip;
-    w2 += w_skip;
-    w_bytes -= w_skip;
-    x16 += k0;
+    // SPLIT: this workgroup's K range; from here on k, the weight rows and the activations
+    // begin there (an instance of its own: without a split the division, the moved pointers
+    // and the second epilogue cost a call of one K step 0.3 - 0.6 of 10 us)
+    int range = 0;
+    if constexpr (SPLIT) {
+        range = tile / range_tiles;
+        tile -= range * range_tiles;
+        const int k0 = range * range_k;
+        k = min(range_k, k - k0);
+        const size_t w_skip = F16W ? static_cast<size_t>(k0) * 2 : static_cast<size_t>(k0 >> 5) * 18;
+        w += w_skip;
+        w2 += w_skip;
+        w_bytes -= w_skip;
+        x16 += k0;
+    }
     const int mt = tile / n_tiles;
     const int nt = tile - mt * n_tiles;
 
@@ -610,7 +614,7 @@ __global__ __launch_bounds__(kGemmThreads) void mfma_gemm(const uint8_t *__restr
             }
         }
     }
-    if (part) {   // split K: this range's plain sums, for gemm_split_sum
+    if constexpr (SPLIT) {   // this range's plain sums, for gemm_split_sum
         const int stride = part_stride(n_rows);
 #pragma unroll
         for (int it = 0; it < 2; ++it)
@@ -862,8 +866,9 @@ __device__ void build_tiny_masks_rows(int rows, int blocks, RowPtr row_ptr, uint
 // p into B buffer p % 2. Offsets are per lane and fixed over stages; the stage
 // offset is the SGPR soffset. (Separate functions, not lambdas of the kernel:
 // the host pass rejects a kernel-local lambda that hands captured values to
-// these builtins, and then drops the launch stub.)
-template <typename S>
+// these builtins, and then drops the launch stub; and a function that two kernels
+// instantiate alike, so each kernel has its own: SPLIT.)
+template <typename S, bool SPLIT>
 __device__ __forceinline__ void ql_copy_a(const uint32_t (&a_off)[S::ACopiesPerWave], _Float16 *a_tile, int a_extent,
                                           int wid, int s) {
     extern __shared__ __align__(16) uint8_t ql_lds[];
@@ -875,7 +880,7 @@ __device__ __forceinline__ void ql_copy_a(const uint32_t (&a_off)[S::ACopiesPerW
                                                  16, a_off[t], s * (S::KS * 2), 0, 0);
 }
 
-template <typename S, bool PAIR>
+template <typename S, bool PAIR, bool SPLIT>
 __device__ __forceinline__ void ql_copy_b(const uint32_t (&b_off)[S::BCopiesPerWave], uint8_t *b_tile,
                                           uint8_t *b_tile2, int b_extent, int wid, int p) {
     extern __shared__ __align__(16) uint8_t ql_lds[];
@@ -896,7 +901,7 @@ __device__ __forceinline__ void ql_copy_b(const uint32_t (&b_off)[S::BCopiesPerW
 // its BN/2 up rows (matrix w2, from S::UpBase); waves 0-1 (tile columns
 // 0 .. BN/2) take the gate rows and waves 2-3 the up rows of the same output
 // columns, which the epilogue pairs in LDS.
-template <int BM, int WN, bool PAIR, bool LONG, int CW = 4>
+template <int BM, int WN, bool PAIR, bool LONG, int CW, bool SPLIT>
 __global__ __launch_bounds__(128 * CW) void q4_lds_gemm(const uint8_t *__restrict__ w, const uint8_t *__restrict__ w2,
                                                          const _Float16 *__restrict__ x16,
                                                          const float *__restrict__ row_inv, float *__restrict__ y,
@@ -911,16 +916,20 @@ __global__ __launch_bounds__(128 * CW) void q4_lds_gemm(const uint8_t *__restric
     const int bid = blockIdx.x;
     int tile = (bid % kXcds) * tiles_per_xcd + bid / kXcds;
     if (tile >= tiles) return;                                  // whole workgroup, before any barrier
-    // this workgroup's K range of whole stages (all of K without a split): from here
-    // on the stages, the weight rows and the activations begin there
-    const int range = tile / range_tiles;
-    tile -= range * range_tiles;
-    const int stage0 = range * range_stages;
-    stages = min(range_stages, stages - stage0);
-    const uint32_t w_skip = static_cast<uint32_t>(stage0) * (S::KS / 32 * 18);
-    w += w_skip;
-    w2 += w_skip;
-    x16 += static_cast<size_t>(stage0) * S::KS;
+    // SPLIT: this workgroup's K range of whole stages; from here on the stages, the weight
+    // rows and the activations begin there
+    int range = 0, stage0 = 0;
+    uint32_t w_skip = 0;
+    if constexpr (SPLIT) {
+        range = tile / range_tiles;
+        tile -= range * range_tiles;
+        stage0 = range * range_stages;
+        stages = min(range_stages, stages - stage0);
+        w_skip = static_cast<uint32_t>(stage0) * (S::KS / 32 * 18);
+        w += w_skip;
+        w2 += w_skip;
+        x16 += static_cast<size_t>(stage0) * S::KS;
+    }
     const int nt = tile / m_tiles;
     const int mt = tile - nt * m_tiles;
     const int m0 = mt * BM, n0 = nt * kOut;
@@ -1082,11 +1091,11 @@ __global__ __launch_bounds__(128 * CW) void q4_lds_gemm(const uint8_t *__restric
     // buffers): A(0), B(0), A(1), B(1); at stage s A(s+2) and B(s+2); the top
     // of stage s leaves A(s+1) and B(s+1) in flight. The k-groups take the
     // same blocks in the same order as two 128-K stages would give them.
-    ql_copy_a<S>(a_off, a_tile, a_extent, wid, 0);
-    ql_copy_b<S, PAIR>(b_off, b_tile, b_tile2, b_extent, wid, 0);
+    ql_copy_a<S, SPLIT>(a_off, a_tile, a_extent, wid, 0);
+    ql_copy_b<S, PAIR, SPLIT>(b_off, b_tile, b_tile2, b_extent, wid, 0);
     if (stages > 1) {
-        ql_copy_a<S>(a_off, a_tile, a_extent, wid, 1);
-        if (LONG) ql_copy_b<S, PAIR>(b_off, b_tile, b_tile2, b_extent, wid, 1);
+        ql_copy_a<S, SPLIT>(a_off, a_tile, a_extent, wid, 1);
+        if (LONG) ql_copy_b<S, PAIR, SPLIT>(b_off, b_tile, b_tile2, b_extent, wid, 1);
     }
     for (int s = 0; s < stages; ++s) {
         if (s + 1 >= stages)
@@ -1103,11 +1112,11 @@ __global__ __launch_bounds__(128 * CW) void q4_lds_gemm(const uint8_t *__restric
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("" ::: "memory");
         if (s + 2 < stages) {
-            ql_copy_a<S>(a_off, a_tile, a_extent, wid, s + 2);
+            ql_copy_a<S, SPLIT>(a_off, a_tile, a_extent, wid, s + 2);
             if (LONG)
-                ql_copy_b<S, PAIR>(b_off, b_tile, b_tile2, b_extent, wid, s + 2);
+                ql_copy_b<S, PAIR, SPLIT>(b_off, b_tile, b_tile2, b_extent, wid, s + 2);
             else if ((s & 1) == 0)
-                ql_copy_b<S, PAIR>(b_off, b_tile, b_tile2, b_extent, wid, s / 2 + 1);
+                ql_copy_b<S, PAIR, SPLIT>(b_off, b_tile, b_tile2, b_extent, wid, s / 2 + 1);
         }
         const uint8_t *a_lds = ql_lds + (s % kQlABufs) * S::ABytes;
         if (LONG) {
@@ -1127,7 +1136,7 @@ __global__ __launch_bounds__(128 * CW) void q4_lds_gemm(const uint8_t *__restric
     __syncthreads();                                            // ring idle
     constexpr int kTs = S::TileStride;
     float *tile_lds = reinterpret_cast<float *>(ql_lds);
-    if (threadIdx.x < BM) scale_lds[threadIdx.x] = part ? 1.0f : row_inv_raw * 8.0f;
+    if (threadIdx.x < BM) scale_lds[threadIdx.x] = SPLIT ? 1.0f : row_inv_raw * 8.0f;
     if (kh == 1) {
 #pragma unroll
         for (int rg = 0; rg < S::RG; ++rg)
@@ -1176,7 +1185,7 @@ __global__ __launch_bounds__(128 * CW) void q4_lds_gemm(const uint8_t *__restric
     __syncthreads();
     // PAIR: output column c is SiLU(tile column c) * (tile column BN/2 + c)
     constexpr int kQuads = kOut / 4;
-    if (part) {   // split K: this range's plain sums, for gemm_split_sum
+    if constexpr (SPLIT) {   // this range's plain sums, for gemm_split_sum
         const int stride = part_stride(n_rows);
         const size_t plane = static_cast<size_t>(m_rows) * stride;
         float *const base = part + static_cast<size_t>(PAIR ? 2 * range : range) * plane;
@@ -1765,6 +1774,7 @@ int device_cus();
 KRanges pick_ranges(const GemmPlan &p, int tiles, int k, int n, int batch, bool pair) {
     const int units = (k + kKAlign - 1) / kKAlign;
     KRanges r = {1, units, 0};
+    if (units < 2 * kMinUnitsSaved) return r;   // two units per range: no split saves that many
     const size_t one = static_cast<size_t>(pair ? 2 : 1) * batch * part_stride(n) * 4;
     const size_t fixed = p.x16_bytes + p.row_inv_bytes;
     if (fixed >= KUNLUN_NOALLOC_SCRATCH_BYTES || tiles <= 0) return r;
@@ -1809,15 +1819,15 @@ template <bool F16W, int BN, bool PAIR = false>
 hipError_t launch_gemm(const void *w, const void *w2, const _Float16 *x16, const float *row_inv, float *y, float *part,
                        int batch, int n, int k, const GemmPlan &p, const KRanges &kr, size_t w_bytes,
                        hipStream_t stream) {
-    const hipError_t rc =
-        kk::opt_in_lds(reinterpret_cast<const void *>(&mfma_gemm<F16W, BN, PAIR>), gemm_lds_bytes<BN>());
+    const auto kernel = kr.ranges > 1 ? &mfma_gemm<F16W, BN, PAIR, true> : &mfma_gemm<F16W, BN, PAIR, false>;
+    const hipError_t rc = kk::opt_in_lds(reinterpret_cast<const void *>(kernel), gemm_lds_bytes<BN>());
     if (rc != hipSuccess) return rc;
     const int range_tiles = p.m_tiles * p.n_tiles, tiles = range_tiles * kr.ranges;
     const int tiles_per_xcd = (tiles + kXcds - 1) / kXcds;
-    hipLaunchKernelGGL((mfma_gemm<F16W, BN, PAIR>), dim3(tiles_per_xcd * kXcds), dim3(kGemmThreads),
+    hipLaunchKernelGGL(kernel, dim3(tiles_per_xcd * kXcds), dim3(kGemmThreads),
                        gemm_lds_bytes<BN>(), stream, static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(w2),
                        x16, row_inv, y, batch, n, k, p.k_pad, w_bytes, p.n_tiles, tiles, tiles_per_xcd, range_tiles,
-                       kr.units * kKAlign, kr.ranges > 1 ? part : nullptr);
+                       kr.units * kKAlign, part);
     const hipError_t launched = hipGetLastError();
     if (launched != hipSuccess || kr.ranges == 1) return launched;
     return launch_split_sum<PAIR>(part, row_inv, F16W ? 1.0f : 8.0f, y, batch, n, kr.ranges, stream);
@@ -1858,11 +1868,11 @@ QlTile pick_ql_tile(int batch, int n, bool pair) {
     return pick;
 }
 
-template <int BM, int WN, bool PAIR, bool LONG = false, int CW = 4>
+template <int BM, int WN, bool PAIR, bool LONG = false, int CW = 4, bool SPLIT = false>
 hipError_t launch_ql_gemm(const void *w, const void *w2, const _Float16 *x16, const float *row_inv, float *y, int batch,
                           int n, int k, int k_pad, hipStream_t stream, const KRanges *kr = nullptr, float *part = nullptr) {
     using S = QlShape<BM, WN, PAIR, LONG, CW>;
-    hipError_t rc = kk::opt_in_lds(reinterpret_cast<const void *>(&q4_lds_gemm<BM, WN, PAIR, LONG, CW>), S::LdsBytes);
+    hipError_t rc = kk::opt_in_lds(reinterpret_cast<const void *>(&q4_lds_gemm<BM, WN, PAIR, LONG, CW, SPLIT>), S::LdsBytes);
     if (rc != hipSuccess) return rc;
     const int out = PAIR ? S::BN / 2 : S::BN;
     const int m_tiles = (batch + BM - 1) / BM;
@@ -1870,7 +1880,7 @@ hipError_t launch_ql_gemm(const void *w, const void *w2, const _Float16 *x16, co
     const int tiles_per_xcd = (tiles + kXcds - 1) / kXcds;
     const uint32_t row_bytes = static_cast<uint32_t>(k / 32 * 18);
     const int stages = k / S::KS, range_stages = kr ? kr->units * (2 * kQlK / S::KS) : stages;
-    hipLaunchKernelGGL((q4_lds_gemm<BM, WN, PAIR, LONG, CW>), dim3(tiles_per_xcd * kXcds), dim3(S::Threads), S::LdsBytes,
+    hipLaunchKernelGGL((q4_lds_gemm<BM, WN, PAIR, LONG, CW, SPLIT>), dim3(tiles_per_xcd * kXcds), dim3(S::Threads), S::LdsBytes,
                        stream, static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(w2), x16, row_inv, y, batch,
                        n, k_pad, stages, row_bytes, m_tiles, tiles, tiles_per_xcd, range_tiles, range_stages, part);
     return hipGetLastError();
@@ -1899,8 +1909,8 @@ hipError_t launch_ql(const void *w, const void *w2, const _Float16 *x16, const f
     const KRanges kr = ranges_ql(p, k, n, batch, PAIR);
     if (kr.ranges > 1) {   // few tiles: K split over workgroups, 64 x 128 tiles (as below)
         hipError_t rc;
-        if constexpr (PAIR) rc = launch_ql_gemm<64, 32, true, true>(w, w2, x16, row_inv, y, batch, n, k, k_pad, stream, &kr, part);
-        else rc = launch_ql_gemm<64, 16, false, true, 8>(w, w2, x16, row_inv, y, batch, n, k, k_pad, stream, &kr, part);
+        if constexpr (PAIR) rc = launch_ql_gemm<64, 32, true, true, 4, true>(w, w2, x16, row_inv, y, batch, n, k, k_pad, stream, &kr, part);
+        else rc = launch_ql_gemm<64, 16, false, true, 8, true>(w, w2, x16, row_inv, y, batch, n, k, k_pad, stream, &kr, part);
         return rc != hipSuccess ? rc : launch_split_sum<PAIR>(part, row_inv, 8.0f, y, batch, n, kr.ranges, stream);
     }
     const QlTile t = pick_ql_tile(batch, n, PAIR);
