@@ -1734,7 +1734,10 @@ struct GemmPlan {
     size_t x16_bytes, row_inv_bytes;
 };
 
-// K ranges of a call: how many, and the 256-K units of each.
+// K ranges of a call: how many, and the units of kSplitK of each: whole main-loop
+// iterations of the register-staged kernel and whole stages of the LDS-copy kernel.
+constexpr int kSplitK = kKAlign;
+static_assert(kSplitK % (2 * kQlK) == 0, "ranges end where both kernels' loops can");
 struct KRanges {
     int ranges, units;
     size_t part_bytes;
@@ -1772,7 +1775,7 @@ int device_cus();
 // b100 13.7 / 13.4 (the line: 3 units saved; K1024 is not split); F16 K4096 x N4096
 // b64 32.1 / 18.5, b256 34.2 / 27.5.
 KRanges pick_ranges(const GemmPlan &p, int tiles, int k, int n, int batch, bool pair) {
-    const int units = (k + kKAlign - 1) / kKAlign;
+    const int units = (k + kSplitK - 1) / kSplitK;
     KRanges r = {1, units, 0};
     if (units < 2 * kMinUnitsSaved) return r;   // two units per range: no split saves that many
     const size_t one = static_cast<size_t>(pair ? 2 : 1) * batch * part_stride(n) * 4;
@@ -1793,7 +1796,7 @@ KRanges pick_ranges(const GemmPlan &p, int tiles, int k, int n, int batch, bool 
 // kernel's 128 x 64 (pair: 64 columns of each matrix in both).
 int range_tiles_ql(int n, int batch, bool pair) { return (batch + 63) / 64 * ((n + (pair ? 63 : 127)) / (pair ? 64 : 128)); }
 KRanges ranges_ql(const GemmPlan &p, int k, int n, int batch, bool pair) {
-    if (kk::tuning(kk::kGemmTile) > 0) return {1, k / 256, 0};
+    if (kk::tuning(kk::kGemmTile) > 0) return {1, k / kSplitK, 0};
     return pick_ranges(p, range_tiles_ql(n, batch, pair), k, n, batch, pair);
 }
 KRanges ranges_staged(const GemmPlan &p, int k, int n, int batch, bool pair) {
@@ -1827,7 +1830,7 @@ hipError_t launch_gemm(const void *w, const void *w2, const _Float16 *x16, const
     hipLaunchKernelGGL(kernel, dim3(tiles_per_xcd * kXcds), dim3(kGemmThreads),
                        gemm_lds_bytes<BN>(), stream, static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(w2),
                        x16, row_inv, y, batch, n, k, p.k_pad, w_bytes, p.n_tiles, tiles, tiles_per_xcd, range_tiles,
-                       kr.units * kKAlign, part);
+                       kr.units * kSplitK, part);
     const hipError_t launched = hipGetLastError();
     if (launched != hipSuccess || kr.ranges == 1) return launched;
     return launch_split_sum<PAIR>(part, row_inv, F16W ? 1.0f : 8.0f, y, batch, n, kr.ranges, stream);
@@ -1879,7 +1882,7 @@ hipError_t launch_ql_gemm(const void *w, const void *w2, const _Float16 *x16, co
     const int range_tiles = m_tiles * ((n + out - 1) / out), tiles = range_tiles * (kr ? kr->ranges : 1);
     const int tiles_per_xcd = (tiles + kXcds - 1) / kXcds;
     const uint32_t row_bytes = static_cast<uint32_t>(k / 32 * 18);
-    const int stages = k / S::KS, range_stages = kr ? kr->units * (2 * kQlK / S::KS) : stages;
+    const int stages = k / S::KS, range_stages = kr ? kr->units * (kSplitK / S::KS) : stages;
     hipLaunchKernelGGL((q4_lds_gemm<BM, WN, PAIR, LONG, CW, SPLIT>), dim3(tiles_per_xcd * kXcds), dim3(S::Threads), S::LdsBytes,
                        stream, static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(w2), x16, row_inv, y, batch,
                        n, k_pad, stages, row_bytes, m_tiles, tiles, tiles_per_xcd, range_tiles, range_stages, part);
