@@ -1763,7 +1763,7 @@ int device_cus();
 // K ranges for `tiles` tiles of at most 128 rows (64 x 128 or 128 x 64 outputs each):
 // as many as the CUs hold in one round, of at least two units of 256; none where
 // the split would not take three units off every tile's serial loop (the summing
-// launch costs 2 - 4 us, a unit 1.1 - 2.2), nor for a forced tile. The partial sums
+// launch costs 2 - 4 us, a unit 1.1 - 2.2), nor for a forced LDS-copy or wide tile. The partial sums
 // of one call, with the activations, stay within the no-allocation entry point's
 // scratch, so both entry points split alike (and a call that it refuses is not split).
 //
@@ -1954,10 +1954,13 @@ hipError_t launch_f16_wide(const void *w, const void *w2, const _Float16 *x16, c
 // ones. us per call, register-staged / wide: K4096 x N4096 b1024 62 / 56 (128 rows; 88 with
 // 256), b2048 117 / 76, K4096 x N11008 b512 103 / 61, b1024 164 / 102 (256 rows; 114 with
 // 128), b2048 322 / 205, K4096 x N4096 b512 43 / 52 (stays). KUNLUN_GEMM_TILE=256x64 and
-// 128x64 force the wide tiles, another tile none of them.
-int pick_f16_wide(const GemmPlan &p, int batch, int n, int k, bool pair) {
+// 128x64 force the wide tiles (and K is not split), another tile none of them.
+int forced_f16_wide(int k) {
     const int forced = kk::tuning(kk::kGemmTile);
-    if (forced > 0) return forced == 256 * 1000 + 64 ? 256 : forced == 128 * 1000 + 64 && k % 64 == 0 ? 128 : 0;
+    return forced == 256 * 1000 + 64 ? 256 : forced == 128 * 1000 + 64 && k % 64 == 0 ? 128 : 0;
+}
+int pick_f16_wide(const GemmPlan &p, int batch, int n, int k, bool pair) {
+    if (kk::tuning(kk::kGemmTile) > 0) return forced_f16_wide(k);
     const long cus = device_cus(), columns = (n + (pair ? 127 : 255)) / (pair ? 128 : 256);
     auto rounds = [&](long tiles) { return (tiles + cus - 1) / cus; };
     const bool wide_staged = pair || p.bn == 128;
@@ -1977,7 +1980,7 @@ int pick_f16_wide(const GemmPlan &p, int batch, int n, int k, bool pair) {
 template <bool PAIR>
 hipError_t launch_f16(const void *w, const void *w2, const _Float16 *x16, const float *row_inv, float *y, float *part,
                       int batch, int n, int k, const GemmPlan &p, const KRanges &kr, hipStream_t stream) {
-    const int wide = kr.ranges > 1 ? 0 : pick_f16_wide(p, batch, n, k, PAIR);
+    const int wide = kr.ranges > 1 ? forced_f16_wide(k) : pick_f16_wide(p, batch, n, k, PAIR);
     if (wide == 256) return launch_f16_wide<PAIR, 1>(w, w2, x16, row_inv, y, batch, n, k, p.k_pad, stream);
     if (wide == 128) return launch_f16_wide<PAIR, 2>(w, w2, x16, row_inv, y, batch, n, k, p.k_pad, stream);
     const size_t w_bytes = static_cast<size_t>(n) * k * 2;

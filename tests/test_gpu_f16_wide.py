@@ -1,5 +1,6 @@
 """GPU parity of the wide F16 prefill tiles (256 and 128 activation rows x 256
-weight rows, forced by KUNLUN_GEMM_TILE=256x64 and 128x64): one to many K steps
+weight rows, forced by KUNLUN_GEMM_TILE=256x64 and 128x64, and by the dispatch;
+sums that show which kernel ran): one to many K steps
 (odd and even counts, K % 64 == 32 on the 256-row tile), partial row and column
 tiles, the gate/up pair, extreme F16 values and rows, non-finite weights.
 Bound as for the other GEMM tiles: 2e-3 * ||x_b|| * ||w_r|| per element.
@@ -16,6 +17,55 @@ pytestmark = pytest.mark.gpu
 
 F16 = kl.WeightType.f16
 WIDE = ["256x64", "128x64"]
+
+
+# Sums that tell the kernels apart (all take the same route): 2^30 at K 0 and -2^30 in the
+# fourth last K32 block, ones in `blocks`. An F32 chain that holds 2^30 drops the ones added to
+# it (half a unit there is 64, an MFMA adds at most 32), one without it keeps them.
+def order_probe(k, n, batch, blocks):
+    x, w = np.zeros((batch, k // 32, 32), np.float32), np.ones((n, k), np.float32)
+    x[:, blocks] = 1.0
+    x = x.reshape(batch, k)
+    at = k - 128
+    x[:, 0] = x[:, at] = 2.0**15
+    w[:, 0], w[:, at] = 2.0**15, -(2.0**15)
+    y, route, guard_ok = run_matmul(F16, w.astype(np.float16).view(np.uint8), x, k, n, batch)
+    assert route == "f16_gemm_mfma" and guard_ok
+    return y
+
+
+def rows_256(k, n, batch):
+    # one chain over all of K: 31 ones at most beside -2^30, and the last three blocks
+    y = order_probe(k, n, batch, slice(None))
+    return bool(np.all((y >= 96) & (y <= 128)))
+
+
+def rows_128(k, n, batch):
+    # a chain of the even blocks (with 2^30) and one of the odd ones; the register-staged
+    # kernel has blocks 0, 1 of every four in one chain, a split has whole ranges
+    return bool(np.all(order_probe(k, n, batch, slice(1, None, 4)) == k // 128 * 32))
+
+
+@pytest.mark.parametrize("k,n,batch", [(4096, 300, 513), (5632, 511, 300), (16384, 256, 65), (4096, 11008, 512)])
+def test_f16_forced_tile_runs(gpu, knobs, k, n, batch):
+    knobs("KUNLUN_GEMM_TILE", "256x64")
+    assert rows_256(k, n, batch) and not rows_128(k, n, batch)
+    knobs("KUNLUN_GEMM_TILE", "128x64")
+    assert rows_128(k, n, batch) and not rows_256(k, n, batch)
+    knobs("KUNLUN_GEMM_TILE", "128x48")            # another tile: no wide one
+    assert not rows_128(k, n, batch) and not rows_256(k, n, batch)
+
+
+# Calls that the dispatch gives to the wide tiles (128 and 256 rows) by itself
+@pytest.mark.parametrize("k,n,batch,runs", [(4096, 11008, 512, rows_128), (4096, 11008, 1024, rows_256)])
+def test_f16_wide_dispatch(gpu, oracle, k, n, batch, runs):
+    assert runs(k, n, batch)
+    x = gaussian((batch, k), 1.0, 8)
+    payload, dec = weight_payload(F16, gaussian((n, k), 0.02, 9), oracle)
+    y, route, guard_ok = run_matmul(F16, payload, x, k, n, batch)
+    some = np.r_[0:40, 4000:4100, n - 40:n]
+    finite, ok, _ = check_gemm(y[:, some], oracle.gold(dec[some], x, threads=16), dec[some], x)
+    assert route == "f16_gemm_mfma" and guard_ok and finite and ok and np.all(np.isfinite(y))
 
 
 @pytest.mark.parametrize("tile", WIDE)
