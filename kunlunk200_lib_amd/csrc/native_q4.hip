@@ -518,9 +518,18 @@ hipError_t launch_mfma(const uint8_t *w, const uint16_t *scales, const void *x, 
     const int column_groups = (batch + columns - 1) / columns, tiles = (n + 31) / 32;
     const int chunk = nm_chunk(k >> 5, columns);
     const size_t lds = std::max<size_t>(static_cast<size_t>(chunk) * columns * 100, kNmPart);
-    hipLaunchKernelGGL(native_q4_mfma<F16X>, dim3(static_cast<unsigned>((tiles + 7) / 8) * 8 * column_groups),
-                       dim3(kNmThreads), lds, stream, w, scales, x, y, k, n, batch, columns, chunk, column_groups, tiles);
-    return hipGetLastError();
+    // a launch holds fewer than 2^32 threads: many columns of few rows take several
+    const int tile_slots = (tiles + 7) / 8 * 8, most = static_cast<int>(0xffffffffu / kNmThreads) / tile_slots;
+    for (int g0 = 0; g0 < column_groups; g0 += most) {
+        const int groups_here = std::min(most, column_groups - g0);
+        const size_t c0 = static_cast<size_t>(g0) * columns;
+        hipLaunchKernelGGL(native_q4_mfma<F16X>, dim3(static_cast<unsigned>(tile_slots) * groups_here), dim3(kNmThreads), lds,
+                           stream, w, scales, static_cast<const uint8_t *>(x) + c0 * k * (F16X ? 2 : 4), y + c0 * n, k, n,
+                           batch - static_cast<int>(c0), columns, chunk, groups_here, tiles);
+        const hipError_t rc = hipGetLastError();
+        if (rc != hipSuccess) return rc;
+    }
+    return hipSuccess;
 }
 
 } // namespace

@@ -39,3 +39,14 @@ def test_native_columns_nonfinite(gpu, oracle, batch):
     keep = np.delete(np.arange(batch), (1, 2))
     assert np.all(np.isnan(y[1:3]))
     check(oracle, case, y[keep], x[keep])
+
+
+def test_native_more_columns_than_a_launch_holds(gpu, oracle):
+    # 8 workgroups of 512 threads per 5 columns: more than 2^32 threads, in two launches
+    k, n, batch = 32, 1, 5_300_000
+    case = NativeCase(oracle, k, n)
+    x = np.random.default_rng(3).standard_normal((1000, k)).astype(np.float16).astype(np.float32)
+    small, _ = case.run(kl.NativeQ4Workspace(), x, 1000, f16=True)
+    check(oracle, case, small, x)
+    y, _ = case.run(kl.NativeQ4Workspace(), np.tile(x.astype(np.float16), (batch // 1000, 1)), batch, f16=True)
+    assert np.array_equal(y.reshape(-1, 1000).view(np.uint32), np.broadcast_to(small.view(np.uint32).T, (batch // 1000, 1000)))
