@@ -476,6 +476,12 @@ int qs_chunk(int batch) {
 // 10.3 / 13.9, S = 2 10.4 / 10.8 / 19.9, S = 8 10.3 / 10.6 / 13.8; K11008 x
 // N4096 S = 16 13.8 / 15.1 / 19.5, 8 13.0 / 14.6 / 22.2, 4 13.4 / 18.4 / 29.8;
 // K2048 x N5632 at 16 S = 1 8.7, 2 10.0, 4 9.8.
+// Up to 16 columns, wide matrices take fewer and longer ranges as long as one chunk holds
+// them: where a range's tiles are more than the 16 waves of its workgroups, each S writes
+// and re-reads sums for nothing (S that the rule above gives / this, us): K8192 x N14336 at
+// 8 columns 23.6 / 22.0 (S = 4), N28672 41.3 / 36.4 (2), K16384 x N14336 42.5 / 36.4 (4);
+// at 16 K4096 x N32000 28.8 / 25.5 (2), K8192 x N28672 44.9 / 40.1 (4), pair K8192 x 2 x
+// N14336 45.7 / 41.0; but K4096 x N14336 at 16 S = 4 16.4, 2 17.1, K8192 x N8192 at 8 S = 8 16.6.
 // KG: the waves a CU's tiles leave idle (K4096 x N4096 S = 4: KG = 4 10.3,
 // KG = 2 10.5, KG = 1 12.1). A pair takes its matrices' S and KG, so its sums
 // are those of two single calls.
@@ -487,12 +493,16 @@ QsPlan qs_plan(int k, int n, int batch, bool pair, int cus) {
     p.ranges = 1;
     if (steps > 8 || steps > chunk)
         while (p.ranges * (batch <= 16 ? 6 : 4) < steps) p.ranges *= 2;
+    p.tiles = (n + 15) / 16;
+    if (batch <= 16)
+        while (p.ranges > 1 && static_cast<long>(p.tiles) * p.ranges > static_cast<long>(kQsWaves) * cus &&
+               steps <= p.ranges / 2 * chunk)
+            p.ranges /= 2;
     const size_t one = static_cast<size_t>(batch) * p.stride * 4;   // one range's sums
     while (p.ranges > 1 && p.ranges * one > kMaxPartBytes) p.ranges /= 2;
     p.part_bytes = p.ranges == 1 && !pair ? 0 : static_cast<size_t>(p.ranges) * (pair ? 2 : 1) * one;
     // one workgroup per CU where the tiles allow; a range of several chunks
     // holds one tile per wave
-    p.tiles = (n + 15) / 16;
     const int max_groups = std::max(1, cus / p.ranges);
     auto per_cu = [&](int tiles) { return (tiles + max_groups - 1) / max_groups; };
     p.kgroups = floor_pow2(std::max(1, std::min(kQsWaves / std::min(kQsWaves, per_cu(p.tiles)), steps / p.ranges)));
