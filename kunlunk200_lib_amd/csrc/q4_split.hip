@@ -213,9 +213,13 @@ __device__ __forceinline__ void qs_convert(const float (&v)[8], int item, int la
 }
 
 // One step of one tile: tot += 2^-s * (the step's products). a: the step's
-// fragments at this lane, inv: the step's inverse scales.
-template <int MT, bool PACK, bool GEN>
-__device__ __forceinline__ void qs_step(const QsRaw<GEN> &raw, uint32_t shift, int step, int blocks, int g,
+// fragments at this lane, inv: the step's inverse scales. `next` loads the next
+// step into raw: behind the products, once this step's bytes are in operand order
+// (after them the products do not cover its latency: K4096 x N14336 at 16 columns 16.4
+// against 16.9 us, N11008 14.6 / 15.6); with two column tiles, whose registers are full,
+// after them (K4096 x N4096 at 32 columns 13.8 against 14.1).
+template <int MT, bool PACK, bool GEN, typename Next>
+__device__ __forceinline__ void qs_step(QsRaw<GEN> &raw, Next next, uint32_t shift, int step, int blocks, int g,
                                         const half8 *a, const float *inv, float4v (&tot)[MT]) {
     using Q = QsShape<MT, PACK>;
     uint32_t d[9], ev[4], od[4], sc[4];
@@ -234,6 +238,11 @@ __device__ __forceinline__ void qs_step(const QsRaw<GEN> &raw, uint32_t shift, i
     transpose4(ev);
     transpose4(od);
     gather4(s2, sc);
+    if (MT == 1) {
+        __builtin_amdgcn_sched_barrier(0);
+        raw = next();
+        __builtin_amdgcn_sched_barrier(0);
+    }
     float4v acc[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
@@ -259,6 +268,7 @@ __device__ __forceinline__ void qs_step(const QsRaw<GEN> &raw, uint32_t shift, i
 #pragma unroll
         for (int r = 0; r < 4; ++r) tot[t][r] = fmaf(acc[t][r], iv[r], tot[t][r]);
     }
+    if (MT != 1) raw = next();
 }
 
 // GEN: any K % 32 == 0 and any weight alignment (dword loads, byte shifts,
@@ -358,9 +368,9 @@ __global__ __launch_bounds__(kQsThreads) void q4_split_gemv(const QsArgs p) {
                     raw = qs_load<GEN>(m - mis, extent, off, min(s0, last) * kStepBytes);
                 }
                 for (int s = s0; s < s1; ++s) {
-                    qs_step<MT, PACK, GEN>(raw, shift, s, blocks, g, reinterpret_cast<const half8 *>(frag) +
+                    auto next = [&] { return qs_load<GEN>(m - mis, extent, off, min(s + 1, last) * kStepBytes); };
+                    qs_step<MT, PACK, GEN>(raw, next, shift, s, blocks, g, reinterpret_cast<const half8 *>(frag) +
                                            (s - c0) * (kStepBlocks * Q::Frags * kWave) + lane, inv_lds + (s - c0) * Q::Cols, tot);
-                    raw = qs_load<GEN>(m - mis, extent, off, min(s + 1, last) * kStepBytes);
                 }
             }
 
