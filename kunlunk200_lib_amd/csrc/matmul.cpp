@@ -76,14 +76,13 @@ bool q4_mfma_batch(int batch, bool streamed) {
 bool q4_whole(const void * w, int k) { return k % 64 == 0 && ((uintptr_t)w & 3) == 0; }
 
 // Whether the K-split Q4_0 MFMA GEMV may take a call (or a gate/up pair) that no faster
-// route took: above 16 columns always; up to 16 the single-pass MFMA GEMV's batch range,
-// where shapes the batch-1 kernels cannot take (K % 64 != 0, weights off a dword)
+// route took: the single-pass MFMA GEMV's batch range (above 16 columns: where it holds
+// 16), in which shapes the batch-1 kernels cannot take (K % 64 != 0, weights off a dword)
 // count from 3 columns (K5600 x N3000: 3 / 8 / 16 columns 27 / 63 / 123 us on
 // the general GEMV, 13 / 13 / 14 us split).
 bool q4_split_range(const void * w, int k, int batch) {
-    if (batch > 16) return true;
     const bool whole = q4_whole(w, k);
-    return q4_mfma_batch(batch, !whole || (k % 256 == 0 && ((uintptr_t)w & 15) == 0));
+    return q4_mfma_batch(std::min(batch, 16), !whole || (k % 256 == 0 && ((uintptr_t)w & 15) == 0));
 }
 
 // One matrix: not where the general GEMV has little to do. It gives a wave one row of 64
@@ -104,7 +103,7 @@ bool f32_gemm_route(int type, const void * w, const void * x, int batch) {
 }
 
 // Columns of one pass of batches above the small-batch kernels and off the GEMM.
-int gemv_chunk(int type) { return type == 2 && kk::tuning_or(kk::kQ4MfmaMax, 16) >= 16 ? 32 : 16; }
+int gemv_chunk(int type) { return type == 2 && q4_mfma_batch(16, true) ? 32 : 16; }
 
 // Batch range of the block-diagonal Q4_0 MFMA GEMV (the single-pass kernel's
 // range, unless KUNLUN_Q4_BDIAG=0 leaves it to the LDS-staged kernels).

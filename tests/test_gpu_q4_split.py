@@ -47,6 +47,21 @@ def test_split_shapes(gpu, oracle, k, n, batch, w_offset, x_offset, expected):
     assert guard_ok and res["finite"] and res["north_star"]
 
 
+# the knobs' batch range holds above 16 columns too
+@pytest.mark.parametrize("knob,value", [("KUNLUN_Q4_MFMA_MIN", "17"), ("KUNLUN_Q4_MFMA_MAX", "15")])
+@pytest.mark.parametrize("k,route", [(4096, "q4_gemv_dot8"), (1056, GENERAL)])
+def test_split_off_by_knob(gpu, oracle, knobs, knob, value, k, route):
+    n, batch = 70, 32
+    rng = np.random.default_rng(k)
+    q4 = kl.quantize_q4_0((rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    x = rng.standard_normal((batch, k)).astype(np.float32)
+    knobs(knob, value)
+    y, taken, guard_ok = run_matmul(Q4, q4, x, k, n, batch)
+    dec = oracle.q4_decode(q4, k, n)
+    res = check_f32_accumulate(y, oracle.gold(dec, x, threads=16), dec, x)
+    assert taken == route and guard_ok and res["finite"] and res["north_star"]
+
+
 # (k, batch, w_offset): 3..63 columns with K % 64 != 0 or weights off a dword follow F32
 # arithmetic in an infinite activation, the others make its column NaN
 @pytest.mark.parametrize("k,batch,w_offset", [(4096, 20, 0), (11008, 6, 0), (4160, 7, 0), (1056, 12, 0), (5600, 5, 0),
