@@ -1698,7 +1698,6 @@ __global__ __launch_bounds__(512) void f16_wide_gemm(const uint8_t *__restrict__
 // y[m][n] = the ranges' partial sums, added in range order, times the row's scale
 // (PAIR: SiLU(gate) * up of the two matrices' values). Four columns per thread.
 constexpr int kSumThreads = 256;
-constexpr int kMinUnitsSaved = 3;              // see pick_ranges
 
 template <bool PAIR>
 __global__ __launch_bounds__(kSumThreads) void gemm_split_sum(const float *__restrict__ part,
@@ -1762,7 +1761,7 @@ int device_cus();
 
 // K ranges for `tiles` tiles of at most 128 rows (64 x 128 or 128 x 64 outputs each):
 // as many as the CUs hold in one round, of at least two units of 256; none where
-// the split would not take three units off every tile's serial loop (the summing
+// the split would not take `min_saved` units off every tile's serial loop (the summing
 // launch costs 2 - 4 us, a unit 1.1 - 2.2), nor for a forced LDS-copy or wide tile. The partial sums
 // of one call, with the activations, stay within the no-allocation entry point's
 // scratch, so both entry points split alike (and a call that it refuses is not split).
@@ -1771,13 +1770,12 @@ int device_cus();
 // barriers and load latencies. us per call before / after: Q4_0 K5600 x N2999
 // b77 (47 tiles, 5 ranges) 52.1 / 21.7, K4096 x N4096 b64 (8 ranges) 26.0 / 15.6,
 // b128 (4) 27.3 / 18.3, b256 (2) 27.7 / 24.3, K11008 x N4096 b128 57.9 / 29.4,
-// K4096 x N11008 b64 (2) 26.4 / 21.8, K2048 x N4096 b64 16.4 / 14.0, K1280 x N4096
-// b100 13.7 / 13.4 (the line: 3 units saved; K1024 is not split); F16 K4096 x N4096
+// K4096 x N11008 b64 (2) 26.4 / 21.8; F16 K4096 x N4096
 // b64 32.1 / 18.5, b256 34.2 / 27.5.
-KRanges pick_ranges(const GemmPlan &p, int tiles, int k, int n, int batch, bool pair) {
+KRanges pick_ranges(const GemmPlan &p, int tiles, int k, int n, int batch, bool pair, int min_saved) {
     const int units = (k + kSplitK - 1) / kSplitK;
     KRanges r = {1, units, 0};
-    if (units < 2 * kMinUnitsSaved) return r;   // two units per range: no split saves that many
+    if (units - 2 - units % 2 < min_saved) return r;   // with the most ranges, of two units (one of three)
     const size_t one = static_cast<size_t>(pair ? 2 : 1) * batch * part_stride(n) * 4;
     const size_t fixed = p.x16_bytes + p.row_inv_bytes;
     if (fixed >= KUNLUN_NOALLOC_SCRATCH_BYTES || tiles <= 0) return r;
@@ -1785,7 +1783,7 @@ KRanges pick_ranges(const GemmPlan &p, int tiles, int k, int n, int batch, bool 
     const long want = std::min<long>(std::min<long>(device_cus() / tiles, units / 2), room);
     if (want < 2) return r;
     const int per = static_cast<int>((units + want - 1) / want);
-    if (units - per < kMinUnitsSaved) return r;
+    if (units - per < min_saved) return r;
     r.units = per;
     r.ranges = (units + per - 1) / per;
     r.part_bytes = r.ranges * one;
@@ -1795,12 +1793,20 @@ KRanges pick_ranges(const GemmPlan &p, int tiles, int k, int n, int batch, bool 
 // Tiles of one K range: the LDS-copy kernel's 64 x 128, the register-staged
 // kernel's 128 x 64 (pair: 64 columns of each matrix in both).
 int range_tiles_ql(int n, int batch, bool pair) { return (batch + 63) / 64 * ((n + (pair ? 63 : 127)) / (pair ? 64 : 128)); }
+// The least units saved: the LDS-copy kernel's loop is the shorter one (us, without / with the
+// split, cold weights: one matrix, saved 3 K1536 x N11008 b64 15.1 / 17.1, N3000 b300 16.5 / 18.7,
+// saved 4 K1536 x N6000 b64 15.0 / 15.5, K2048 x N11008 b64 17.3 / 18.1, N6000 b77 17.8 / 16.9, saved 6
+// K2048 x N4096 b64 17.4 / 17.4; pair, saved 3 K1536 x N6000 b64 17.1 / 18.3, saved 4 K1536 x N1000 b130
+// 18.3 / 15.6, but with 6.3 MB of sums, N4096 b64, 17.2 / 17.7; register-staged, saved 4 F16 K2048 x
+// N1000 b1024 24.9 / 23.3, pair b700 34.1 / 27.2).
 KRanges ranges_ql(const GemmPlan &p, int k, int n, int batch, bool pair) {
-    if (kk::tuning(kk::kGemmTile) > 0) return {1, k / kSplitK, 0};
-    return pick_ranges(p, range_tiles_ql(n, batch, pair), k, n, batch, pair);
+    const KRanges none = {1, k / kSplitK, 0};
+    if (kk::tuning(kk::kGemmTile) > 0) return none;
+    const KRanges r = pick_ranges(p, range_tiles_ql(n, batch, pair), k, n, batch, pair, pair ? 4 : 5);
+    return k / kSplitK - r.units < 5 && r.part_bytes > (size_t{5} << 20) ? none : r;
 }
 KRanges ranges_staged(const GemmPlan &p, int k, int n, int batch, bool pair) {
-    return pick_ranges(p, p.m_tiles * (pair ? (n + 63) / 64 : p.n_tiles), k, n, batch, pair);
+    return pick_ranges(p, p.m_tiles * (pair ? (n + 63) / 64 : p.n_tiles), k, n, batch, pair, 3);
 }
 
 template <bool PAIR>

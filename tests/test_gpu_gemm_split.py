@@ -19,7 +19,7 @@ Q4, F16 = kl.WeightType.q4_0, kl.WeightType.f16
 
 # (type, k, n, batch, w_offset): the LDS-copy kernel takes Q4_0 with K % 256 == 0 and
 # 16-byte aligned weights, the register-staged one the rest
-SHAPES = [(Q4, 4096, 300, 64, 0), (Q4, 2304, 1, 65, 0), (Q4, 16384, 129, 130, 0), (Q4, 1280, 4096, 100, 0),
+SHAPES = [(Q4, 4096, 300, 64, 0), (Q4, 2304, 1, 65, 0), (Q4, 16384, 129, 130, 0), (Q4, 2048, 1000, 100, 0),
           (Q4, 5600, 131, 77, 0), (Q4, 1312, 64, 200, 0), (Q4, 4096, 257, 70, 2), (Q4, 16352, 33, 64, 1),
           (F16, 4096, 300, 64, 0), (F16, 5600, 2999, 77, 0), (F16, 1312, 1, 129, 0), (F16, 16384, 65, 256, 0)]
 
