@@ -1954,32 +1954,37 @@ hipError_t launch_f16_wide(const void *w, const void *w2, const _Float16 *x16, c
     return hipGetLastError();
 }
 
-// The wide F16 tile of a call (its rows: 256 or 128), or 0 for the register-staged
-// kernel: the least time in whole rounds of the CUs, a round of K4096 taking 37 us of 128 x
-// 64 register-staged tiles, 49 of 128 x 128, 78 of 256 x 256 and 44 of 128 x 256 wide
-// ones. us per call, register-staged / wide: K4096 x N4096 b1024 62 / 56 (128 rows; 88 with
-// 256), b2048 117 / 76, K4096 x N11008 b512 103 / 61, b1024 164 / 102 (256 rows; 114 with
-// 128), b2048 322 / 205, K4096 x N4096 b512 43 / 52 (stays). KUNLUN_GEMM_TILE=256x64 and
-// 128x64 force the wide tiles (and K is not split), another tile none of them.
+// KUNLUN_GEMM_TILE=256x64 and 128x64 force the wide F16 tiles (and K is not split), another
+// tile none of them.
 int forced_f16_wide(int k) {
     const int forced = kk::tuning(kk::kGemmTile);
     return forced == 256 * 1000 + 64 ? 256 : forced == 128 * 1000 + 64 && k % 64 == 0 ? 128 : 0;
 }
+
+// The wide F16 tile of a call (its rows: 256 or 128), or 0 for the register-staged
+// kernel: the least time in whole rounds of the CUs. A round of tiles takes a + b K / 1024 us,
+// fitted to calls whose weights come from HBM (K 1024 .. 11008, N 1000 .. 11008, 64 .. 2048 rows):
+// with them in the cache the wide tiles gain up to a quarter more, but a call of at most half
+// as many of them as CUs then waits for the weights where the register-staged kernel, with
+// twice to eight times the workgroups, does not. us per call, register-staged / 128 rows / 256
+// rows: K4096 x N4096 b512 43 / 52 (stays), b700 66 / 64 / 104, b1024 62 / 65 / 104 (stays), b2048
+// 120 / 79 / 113; K4096 x N11008 b520 107 / 70 / 99, b1024 162 / 131 / 114; K11008 x N4096 b1024
+// 155 / 171 (stays); K1024 x N4096 b1024 30 / 24. A pair's 128-row tile reads two matrices: K2048 x
+// N4096 b300 36 / 41, K1536 x N8192 b130 34 / 40 (stay). Rows of K % 64 == 32 lie off 128 bytes and cost the 256-row tile a
+// quarter more (K5600 x N6000 b700 135 / 178, stays; N11008 b1024 221 / 200).
 int pick_f16_wide(const GemmPlan &p, int batch, int n, int k, bool pair) {
     if (kk::tuning(kk::kGemmTile) > 0) return forced_f16_wide(k);
     const long cus = device_cus(), columns = (n + (pair ? 127 : 255)) / (pair ? 128 : 256);
-    auto rounds = [&](long tiles) { return (tiles + cus - 1) / cus; };
-    const bool wide_staged = pair || p.bn == 128;
-    const long staged = rounds(static_cast<long>(p.m_tiles) * (pair ? (n + 63) / 64 : p.n_tiles)) * (wide_staged ? 49 : 37);
-    const long rows256 = rounds((batch + 255) / 256 * columns) * 78;
-    const long rows128 = k % 64 == 0 ? rounds((batch + 127) / 128 * columns) * 44 : rows256 + 1;
+    const double kib = k / 1024.0;
+    auto rounds = [&](long tiles) { return static_cast<double>((tiles + cus - 1) / cus); };
+    const long tiles = static_cast<long>(p.m_tiles) * (pair ? (n + 63) / 64 : p.n_tiles);
+    const double staged = !pair && p.bn == 64 ? rounds(tiles) * (6 + 5.5 * kib)
+                          : tiles <= cus      ? (11 + 10.7 * kib) * (0.7 + 0.3 * tiles / cus)   // (a part of a round)
+                                              : rounds(tiles) * (7 + 9.6 * kib);
+    const double rows256 = rounds((batch + 255) / 256 * columns) * ((pair ? 12 : 6) + 23.6 * kib) * (k % 64 ? 1.25 : 1.0);
+    const double rows128 =
+        k % 64 ? rows256 + 1 : rounds((batch + 127) / 128 * columns) * (pair ? 6 + 15 * kib : 3 + 13.2 * kib);
     if (std::min(rows256, rows128) >= staged) return 0;
-    // few tiles that each stream activations past an XCD's L2 (4 MiB) wait for them: 96
-    // tiles of K8192 x N8192 b300 (4.7 MiB) 119 against 117 register-staged, of K8128 120 / 115,
-    // 100 of K11008 x N5000 b640 (13 MiB) 170 / 152, but K6144 x N8192 b300 (3.5 MiB) 71 / 86 and
-    // 120 of K4096 x N6000 b520 (4.1 MiB) 51 / 68
-    const long tiles = (batch + 127) / 128 * columns;
-    if (tiles < cus / 2 && static_cast<size_t>(batch) * k * 2 > (size_t{9} << 19)) return 0;
     return rows128 <= rows256 ? 128 : 256;
 }
 
