@@ -1806,7 +1806,9 @@ KRanges ranges_ql(const GemmPlan &p, int k, int n, int batch, bool pair) {
     return k / kSplitK - r.units < 5 && r.part_bytes > (size_t{5} << 20) ? none : r;
 }
 KRanges ranges_staged(const GemmPlan &p, int k, int n, int batch, bool pair) {
-    return pick_ranges(p, p.m_tiles * (pair ? (n + 63) / 64 : p.n_tiles), k, n, batch, pair, 3);
+    const KRanges none = {1, (k + kSplitK - 1) / kSplitK, 0};
+    const KRanges r = pick_ranges(p, p.m_tiles * (pair ? (n + 63) / 64 : p.n_tiles), k, n, batch, pair, 3);
+    return none.units - r.units < 4 && r.part_bytes > (size_t{7} << 20) ? none : r;   // F16 K1536 x N1000 b1024 21.9 / 22.5
 }
 
 template <bool PAIR>
