@@ -97,10 +97,18 @@ bool q4_split_route(const void * w, int k, int n, int batch, int cus) {
 }
 
 // F32 weights above the single-pass GEMV's 16 columns (K4096 x N4096 at 17
-// columns: 28.4 us in passes of 16, 18.4 us).
-bool f32_gemm_route(int type, const void * w, const void * x, int batch) {
-    return type == 0 && batch > 16 && dense_mfma_batch(16) && (((uintptr_t)w | (uintptr_t)x) & 15) == 0;
+// columns: 28.4 us in passes of 16, 18.4 us), except up to 48 columns of a part of one
+// row tile (K8192 x N1 at 17 / 33 / 48 / 64 columns: 22.9 / 38.1 / 46.0 / 61.0 us in passes, 30.0 /
+// 48.5 / 48.5 / 48.7).
+bool f32_gemm_route(int type, const void * w, const void * x, int n, int batch) {
+    return type == 0 && batch > 16 && (n >= 16 || batch > 48) && dense_mfma_batch(16) &&
+           (((uintptr_t)w | (uintptr_t)x) & 15) == 0;
 }
+
+// Columns of such a call on the F32 GEMM: its 33rd alone would double the column tile, which
+// on few and long rows takes longer than a pass of its own (K8192 x N65 at 33 columns: 47.7 us
+// in passes of 16, 49.2 in one tile of 64, 42.0 as 32 + 1; K11008 x N300 66.7 / 65.5 / 55.3).
+int f32_gemm_columns(int k, int n, int batch) { return batch == 33 && k >= 4096 && n <= 1024 ? 32 : batch; }
 
 // Columns of one pass of batches above the small-batch kernels and off the GEMM.
 int gemv_chunk(int type) { return type == 2 && q4_mfma_batch(16, true) ? 32 : 16; }
@@ -174,10 +182,14 @@ static void dispatch_dense(Kernel::Impl & impl, detail::DeviceContext & ctx, int
                     const void * x, int k, int n, int batch, WeightType type) {
     const bool gemm = (type == WeightType::q4_0 || (type == WeightType::f16 && ((uintptr_t)w & 15) == 0)) &&
                       batch >= gemm_min_batch() && ((uintptr_t)x & 15) == 0;
-    if (kk::f32_gemm_route((int)type, w, x, batch)) {
-        detail::check_hip((hipError_t)kk_f32_gemm(w, static_cast<const float *>(x), static_cast<float *>(y), k, n, batch,
-                                                  ctx.cus, ctx.stream),
+    if (kk::f32_gemm_route((int)type, w, x, n, batch)) {
+        const int columns = kk::f32_gemm_columns(k, n, batch);
+        detail::check_hip((hipError_t)kk_f32_gemm(w, static_cast<const float *>(x), static_cast<float *>(y), k, n,
+                                                  columns, ctx.cus, ctx.stream),
                           "kk_f32_gemm");
+        if (columns < batch)
+            dispatch_dense(impl, ctx, id, static_cast<char *>(y) + (size_t)columns * n * 4, w,
+                           static_cast<const char *>(x) + (size_t)columns * k * 4, k, n, batch - columns, type);
         impl.route = "f32_mfma_gemv";
         return;
     }

@@ -133,9 +133,14 @@ extern "C" int kunlun_matmul_noalloc(int device, void *y, const void *w, const v
         const size_t need = kk_gemm_workspace_bytes(k, n, batch, 0);
         if (need > kScratchBytes) return too_large(need);
         rc = static_cast<hipError_t>(kk_gemm(type, w, xf, yf, k, n, batch, d.ptr, s, &taken));
-    } else if (kk::f32_gemm_route(type, w, x, batch)) {
+    } else if (kk::f32_gemm_route(type, w, x, n, batch)) {
         taken = "f32_mfma_gemv";
-        rc = static_cast<hipError_t>(kk_f32_gemm(w, xf, yf, k, n, batch, d.cus, s));
+        const int columns = kk::f32_gemm_columns(k, n, batch);
+        rc = static_cast<hipError_t>(kk_f32_gemm(w, xf, yf, k, n, columns, d.cus, s));
+        const char *rest = nullptr;
+        if (rc == hipSuccess && columns < batch)
+            rc = small_batch(d, type, w, xf + static_cast<size_t>(columns) * k, yf + static_cast<size_t>(columns) * n, k, n,
+                             batch - columns, wa, s, &rest);
     } else {
         // kunlun_matmul's small-batch routes, in its chunks of columns, in
         // stream order on the one array

@@ -47,7 +47,8 @@ bool q4_mfma_batch(int batch, bool streamed);
 bool q4_whole(const void * w, int k);
 bool q4_split_range(const void * w, int k, int batch);
 bool q4_split_route(const void * w, int k, int n, int batch, int cus);
-bool f32_gemm_route(int type, const void * w, const void * x, int batch);
+bool f32_gemm_route(int type, const void * w, const void * x, int n, int batch);
+int f32_gemm_columns(int k, int n, int batch);
 int gemv_chunk(int type);
 bool q4_bdiag_batch(int batch);
 bool q4_stream_batch(int batch);

@@ -17,7 +17,8 @@ F32 = kl.WeightType.f32
 
 
 @pytest.mark.parametrize("k,n,batch", [(32, 7, 17), (96, 40, 33), (1056, 65, 70), (160, 5000, 30), (4096, 300, 100),
-                                       (16384, 17, 64), (256, 4200, 65), (1152, 16, 32)])
+                                       (16384, 17, 64), (256, 4200, 65), (1152, 16, 32), (1056, 40, 33),
+                                       (8192, 65, 33), (4096, 1024, 33), (4096, 1, 17), (1152, 15, 48), (96, 3, 49)])
 def test_f32_gemm_shapes(gpu, oracle, k, n, batch):
     rng = np.random.default_rng(k + n + batch)
     w = (rng.standard_normal((n, k)) * 0.02).astype(np.float32)

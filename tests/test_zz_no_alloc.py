@@ -29,6 +29,7 @@ CASES = [
     (Q4, "q4_mfma_gemv", (2048, 5000, 32), (1088, 100, 17)),      # more than 16 columns of a block-diagonal shape, no scratch
     (Q4, "q4_gemv_dot8", (4096, 1024, 1), (1024, 129, 1)),        # no scratch
     (F32, "f32_mfma_gemv", (1024, 256, 8), (512, 65, 2)),         # no scratch
+    (F32, "f32_mfma_gemv", (4096, 300, 33), (1056, 7, 48)),       # 32 columns and one; passes of 16 (part of a row tile)
 ]
 
 
