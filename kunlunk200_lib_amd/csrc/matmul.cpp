@@ -99,9 +99,9 @@ bool q4_split_route(const void * w, int k, int n, int batch, int cus) {
 // F32 weights above the single-pass GEMV's 16 columns (K4096 x N4096 at 17
 // columns: 28.4 us in passes of 16, 18.4 us), except up to 48 columns of a part of one
 // row tile (K8192 x N1 at 17 / 33 / 48 / 64 columns: 22.9 / 38.1 / 46.0 / 61.0 us in passes, 30.0 /
-// 48.5 / 48.5 / 48.7).
+// 48.5 / 48.5 / 48.7) and 17 of few rows (K4096 x N17 16.1 / 17.6, at 18 20.2 / 16.8).
 bool f32_gemm_route(int type, const void * w, const void * x, int n, int batch) {
-    return type == 0 && batch > 16 && (n >= 16 || batch > 48) && dense_mfma_batch(16) &&
+    return type == 0 && batch > 16 && batch > (n < 16 ? 48 : n <= 48 ? 17 : 16) && dense_mfma_batch(16) &&
            (((uintptr_t)w | (uintptr_t)x) & 15) == 0;
 }
 
