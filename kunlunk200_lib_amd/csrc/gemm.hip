@@ -1505,7 +1505,11 @@ __global__ __launch_bounds__(512) void q4_wide_gemm(const uint8_t *__restrict__ 
             for (int c = 0; c < (PAIR ? 2 : 4); ++c) {
                 const int n = n0 + (PAIR ? 32 : 64) * wn + 16 * c + c16;
                 const float v = PAIR ? kk::swiglu_value(acc[i][c][r] * sc, acc[i][(c + 2) & 3][r] * sc) : acc[i][c][r] * sc;
-                if (n < n_rows) __builtin_nontemporal_store(v, dst + n);
+                // a wave's 64 columns of a row are four 64-byte stores: through the L2, which makes
+                // whole lines of them (K512 x N8192 b4096 68 us, past it 108, K4096 x N11008 b2048 204 / 209);
+                // a pair's 32, with half the output, past it (K4096 x 2 x N11008 b2048 366 / 370)
+                if (n < n_rows && PAIR) __builtin_nontemporal_store(v, dst + n);
+                else if (n < n_rows) dst[n] = v;
             }
         }
 }
