@@ -304,10 +304,11 @@ bool exact_route(const CommonQ4Info & a) { return (size_t)a.np * a.kp > kExactRo
 // Rows quantized and multiplied in one launch each: what the workspace holds.
 constexpr int kGroupRows = 512;
 
-// Quantizes `rows` rows (chunks of 128, chunk_stride apart in `values`; M = 1:
-// the per-tensor pair). The counters are the reference's, one chunk at a time.
+// Quantizes `rows` rows (chunks of 128; the codes of those from view_from on,
+// chunk_stride apart, into `values`; M = 1: the per-tensor pair). The counters
+// are the reference's, one chunk at a time.
 void quantize_rows(CommonQ4Workspace::Impl & s, hipStream_t stream, const void * x, int x_f16, const CommonQ4Info & a,
-                   int m, int rows, size_t chunk_stride, void * values, void * scales, void * tiled) {
+                   int m, int rows, int view_from, size_t chunk_stride, void * values, void * scales, void * tiled) {
     ActivationStorage & st = *s.activation;
     const uint64_t t0 = st.profile ? now_ns() : 0;
     const int last = (rows - 1) % 128 + 1;
@@ -317,7 +318,7 @@ void quantize_rows(CommonQ4Workspace::Impl & s, hipStream_t stream, const void *
     else
         detail::check_hip((hipError_t)kk_common_quant_rows(x, x_f16, a.k, a.kp, rows,
                                                            rows - last + round_up(padded_rows(m, last), 32),
-                                                           chunk_stride, values, scales, tiled, stream),
+                                                           view_from, chunk_stride, values, scales, tiled, stream),
                           "kk_common_quant_rows");
     if (st.profile) {
         detail::check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize");
@@ -369,17 +370,21 @@ bool execute(CommonQ4Workspace::Impl & s, int id, void * y, const CommonQ4Info &
         // a lease's rows in one GEMM (its chunks' fragments and scales are
         // contiguous), else groups of rows quantized here
         const int group = prepared ? m : std::min(m, kGroupRows);
+        // (the view is the last chunk's, so the codes of the others are written as
+        // fragments only: 512 rows' codes were a second allocation of 2 MiB and more,
+        // which costs a new workspace 12 us and at times 300)
         const size_t capacity = (size_t)round_up(group, 128);
         if (!prepared) {
-            reserve(st, id, st.quant, st.quant_bytes, capacity * a.kp + 1024);
+            reserve(st, id, st.quant, st.quant_bytes, (size_t)128 * a.kp + 1024);
             reserve(st, id, st.scale, st.scale_bytes, capacity * 64);
             reserve(st, id, st.tiled, st.tiled_bytes, capacity * a.kp * 2);
         }
         for (int first = 0; first < m; first += group) {
             const int rows = std::min(group, m - first);
+            const size_t last = ((size_t)rows - 1) / 128;
             if (!prepared)
                 quantize_rows(s, ctx.stream, static_cast<const char *>(input) + (size_t)first * a.k * bytes, x_f16, a, m,
-                              rows, (size_t)128 * a.kp, st.quant, st.scale, st.tiled);
+                              rows, (int)last * 128, (size_t)128 * a.kp, st.quant, st.scale, st.tiled);
             const void * frags = prepared ? prepared->tiled[0] : st.tiled;
             const void * scales = prepared ? prepared->chunks[0].scales : st.scale;
             detail::check_hip((hipError_t)kk_common_gemm(w, frags, scales, static_cast<float *>(y) + (size_t)first * a.n,
@@ -389,10 +394,7 @@ bool execute(CommonQ4Workspace::Impl & s, int id, void * y, const CommonQ4Info &
                 ++s.stats.paths[gemm_path(padded_rows(m, std::min(128, rows - r)), a.kp)];
                 ++s.stats.chunks;
             }
-            // the view is the last chunk's
-            const size_t last = ((size_t)rows - 1) / 128;
-            s.last_values = prepared ? prepared->chunks[last].values
-                                     : static_cast<const char *>(st.quant) + last * 128 * a.kp;
+            s.last_values = prepared ? prepared->chunks[last].values : st.quant;
             s.last_scales = prepared ? prepared->chunks[last].scales
                                      : static_cast<const char *>(st.scale) + last * 128 * 64;
             s.last_rows = rows - (int)last * 128;
@@ -477,7 +479,7 @@ bool common_q4_prepare(CommonQ4Workspace & work, int id, const void * input, int
     l.type = type;
     l.input = input;
     l.input_bytes = input_bytes;
-    quantize_rows(s, ctx.stream, input, bytes == 2, a, m, m, qstride, st.quant, st.scale, st.tiled);
+    quantize_rows(s, ctx.stream, input, bytes == 2, a, m, m, 0, qstride, st.quant, st.scale, st.tiled);
     size_t index = 0;
     for (int first = 0; first < m; ++index) {
         const int rows = std::min(128, m - first), padded = padded_rows(m, rows);

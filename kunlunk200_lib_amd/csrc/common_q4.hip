@@ -179,7 +179,8 @@ __global__ __launch_bounds__(kQuantThreads) void common_quant_pair(const void *_
 // 3, 7) of the block, the order in which a weight dword's nibbles decode.
 template <bool F16>
 __global__ __launch_bounds__(kRowThreads) void common_quant_rows(const void *__restrict__ x, int k, int kp, int rows,
-                                                                size_t chunk_stride, int8_t *__restrict__ values,
+                                                                int view_from, size_t chunk_stride,
+                                                                int8_t *__restrict__ values,
                                                                 float *__restrict__ params,
                                                                 _Float16 *__restrict__ frags) {
 #pragma clang fp contract(off)
@@ -198,15 +199,18 @@ __global__ __launch_bounds__(kRowThreads) void common_quant_rows(const void *__r
     m = block_max_bits<kRowThreads>(m, scratch);
     const float mx = m ? __uint_as_float(m) : 1.0f;
     const float scale = mx / 127.0f, inv = 127.0f / mx;
-    // eight values per thread and step: two code dwords and one lane's 16 fragment bytes
-    uint2 *out = reinterpret_cast<uint2 *>(values + static_cast<size_t>(row >> 7) * chunk_stride +
-                                           static_cast<size_t>(row & 127) * kp);
+    // eight values per thread and step: two code dwords (in the view's rows) and one lane's 16
+    // fragment bytes
+    const bool viewed = row >= view_from;
+    const int view_row = viewed ? row - view_from : 0;
+    uint2 *out = reinterpret_cast<uint2 *>(values + static_cast<size_t>(view_row >> 7) * chunk_stride +
+                                           static_cast<size_t>(view_row & 127) * kp);
     kk::half8 *frag = reinterpret_cast<kk::half8 *>(frags) + static_cast<size_t>(row >> 4) * (kp >> 5) * 64 + (row & 15);
     for (int d = threadIdx.x; d < kp / 8; d += kRowThreads) {
         int q[8];
 #pragma unroll
         for (int t = 0; t < 8; ++t) q[t] = kk::round_clamp(x_value<F16>(xr, 8 * d + t) * inv, 127);
-        out[d] = make_uint2(pack4(q[0], q[1], q[2], q[3]), pack4(q[4], q[5], q[6], q[7]));
+        if (viewed) out[d] = make_uint2(pack4(q[0], q[1], q[2], q[3]), pack4(q[4], q[5], q[6], q[7]));
         kk::half8 h;
         h[0] = static_cast<_Float16>(q[0]); h[1] = static_cast<_Float16>(q[4]);
         h[2] = static_cast<_Float16>(q[2]); h[3] = static_cast<_Float16>(q[6]);
@@ -655,18 +659,18 @@ extern "C" int kk_common_quant_pair(const void *x, int x_f16, int k, int kp, voi
 }
 
 extern "C" int kk_common_quant_rows(const void *x, int x_f16, int k, int kp, int rows, int defined_rows,
-                                    size_t chunk_stride, void *values, void *params, void *frags, hipStream_t stream) {
+                                    int view_from, size_t chunk_stride, void *values, void *params, void *frags, hipStream_t stream) {
     if (!x || !values || !params || !frags || k <= 0 || kp < k || kp % 256 != 0 || rows <= 0 ||
-        defined_rows < rows || defined_rows % 32 != 0 || (reinterpret_cast<uintptr_t>(values) & 7) || (chunk_stride & 7) ||
+        defined_rows < rows || defined_rows % 32 != 0 || view_from < 0 || view_from >= rows || (reinterpret_cast<uintptr_t>(values) & 7) || (chunk_stride & 7) ||
         (reinterpret_cast<uintptr_t>(frags) & 15))
         return hipErrorInvalidValue;
     if (x_f16)
         hipLaunchKernelGGL(common_quant_rows<true>, dim3(defined_rows), dim3(kRowThreads), 0, stream, x, k, kp, rows,
-                           chunk_stride, static_cast<int8_t *>(values), static_cast<float *>(params),
+                           view_from, chunk_stride, static_cast<int8_t *>(values), static_cast<float *>(params),
                            static_cast<_Float16 *>(frags));
     else
         hipLaunchKernelGGL(common_quant_rows<false>, dim3(defined_rows), dim3(kRowThreads), 0, stream, x, k, kp, rows,
-                           chunk_stride, static_cast<int8_t *>(values), static_cast<float *>(params),
+                           view_from, chunk_stride, static_cast<int8_t *>(values), static_cast<float *>(params),
                            static_cast<_Float16 *>(frags));
     return hipGetLastError();
 }

@@ -102,11 +102,12 @@ int kk_native_q4_gemv(const void *weights, const void *x, int x_f16, float *y, i
 // the view buffer `values` (4*kp + 1024 bytes) and `params` (16 floats).
 int kk_common_quant_pair(const void *x, int x_f16, int k, int kp, void *values, void *params, hipStream_t stream);
 // M > 1 per-row int8 quantization of `rows` rows (zero rows up to
-// defined_rows, a multiple of 32): row r's codes at values[(r/128) *
-// chunk_stride + (r%128) * kp ..], params [defined_rows][16], and the same
-// codes as the GEMM's fp16 operands in `frags` (defined_rows * kp * 2 bytes).
-int kk_common_quant_rows(const void *x, int x_f16, int k, int kp, int rows, int defined_rows, size_t chunk_stride,
-                         void *values, void *params, void *frags, hipStream_t stream);
+// defined_rows, a multiple of 32): the codes of row view_from + r at values[(r/128) *
+// chunk_stride + (r%128) * kp ..] (none of the rows before it), params
+// [defined_rows][16], and every row's codes as the GEMM's fp16 operands in
+// `frags` (defined_rows * kp * 2 bytes).
+int kk_common_quant_rows(const void *x, int x_f16, int k, int kp, int rows, int defined_rows, int view_from,
+                         size_t chunk_stride, void *values, void *params, void *frags, hipStream_t stream);
 // M = 1 GEMV over one weight (w1 null) or two sharing the activations.
 // mode 0: act = the quantized view, params its scales; mode 1: act = X,
 // quantized in the kernel, the view written to view_values / params; mode 2:

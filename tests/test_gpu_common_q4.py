@@ -182,6 +182,30 @@ def test_gemm_row_a8(gpu, oracle, k, n, m):
     assert sum(paths[1:7]) == -(-m // 128) and paths[0] == 0
 
 
+# one and several launch groups of 512 rows: the view is the last chunk of 128, the only one
+# whose codes are kept (one byte per value), beside the scales and a group's fp16 operands
+@pytest.mark.parametrize("m", [128, 200, 512, 513, 1100])
+def test_view_and_workspace_of_many_rows(gpu, oracle, m):
+    k, n = 4096, 40
+    case = Case(oracle, k, n)
+    ws = kl.CommonQ4Workspace()
+    x = oracle.fixture_input(k, m, 5)
+    y = case.run(ws, x, m)
+    first = (m - 1) // 128 * 128
+    rows, defined = m - first, -(-(m - first) // 32) * 32
+    q = ws.quantization()
+    assert q["components"] == 1 and q["rows"] == rows and q["kp"] == k
+    ref_values, ref_params = oracle.common_quant_rows(x[first:], k, rows, defined)
+    assert np.array_equal(view_bytes(ws, rows * k, np.int8, "values"), ref_values[:rows * k])
+    assert np.array_equal(view_bytes(ws, rows * 64, np.float32, "scales"), ref_params[:rows * 16])
+    group = -(-min(m, 512) // 128) * 128
+    assert ws.statistics()["hbm_workspace_bytes"] == 128 * k + 1024 + group * (64 + 2 * k)
+    fresh = kl.CommonQ4Workspace()
+    for r in range(0, m, 128):          # the rows of a call are independent
+        part = case.run(fresh, x[r:r + 128], len(x[r:r + 128])) if len(x[r:r + 128]) > 1 else None
+        assert part is None or np.array_equal(part.view(np.uint32), y[r:r + 128].view(np.uint32))
+
+
 def test_state_bench_mixed_m(gpu, oracle):
     """reference bench/common-q4-state-bench.cpp: one weight, mixed M on one
     workspace, bitwise equal to fresh workspaces, stable device memory."""
