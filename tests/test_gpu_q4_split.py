@@ -11,7 +11,7 @@ import pytest
 
 import kunlunk200_lib_amd as kl
 from gpu_util import check_f32_accumulate, run_matmul
-from test_gpu_swiglu import check_pair, run_pair
+from test_gpu_swiglu import check_pair, device_swiglu, run_pair
 
 pytestmark = pytest.mark.gpu
 
@@ -27,6 +27,8 @@ SHAPES = [(32, 7, 9, 0, 0, SPLIT), (96, 33, 17, 0, 0, SPLIT), (1056, 65, 24, 0, 
           (4096, 16, 16, 0, 0, SPLIT), (4096, 17, 32, 0, 0, SPLIT), (4096, 300, 33, 0, 0, SPLIT), (4096, 300, 63, 0, 0, SPLIT),
           (11008, 257, 8, 0, 0, SPLIT), (11008, 40, 12, 0, 0, SPLIT), (16384, 48, 32, 0, 0, SPLIT),
           (2304, 33000, 32, 0, 0, SPLIT), (512, 20000, 30, 0, 0, SPLIT), (8192, 1, 5, 0, 0, SPLIT),
+          # more row tiles per workgroup than it has waves: a second round on the same fragments
+          (4096, 17000, 32, 0, 0, SPLIT), (544, 66000, 9, 0, 0, SPLIT), (1056, 65600, 8, 0, 0, SPLIT),
           # shapes off the batch-1 kernels with little work: a wave's row per pass of 64 blocks and 8 columns
           (544, 70, 3, 0, 0, GENERAL), (512, 40, 7, 3, 4, GENERAL), (1056, 1000, 8, 0, 0, GENERAL), (1056, 1000, 9, 0, 0, SPLIT),
           (2976, 300, 5, 0, 0, GENERAL), (2976, 300, 6, 0, 0, SPLIT), (2976, 1100, 3, 0, 0, SPLIT)]
@@ -112,7 +114,10 @@ def test_split_largest_activations(gpu, oracle, k, batch):
     assert guard_ok and res["finite"] and res["north_star"]
 
 
-@pytest.mark.parametrize("k,n,batch", [(1056, 65, 24), (4096, 300, 32), (11008, 50, 5), (2048, 1000, 30), (96, 20, 40)])
+# the last five: second rounds, with one k-group and with four (which use their exchange
+# area again), in one K range and in several
+@pytest.mark.parametrize("k,n,batch", [(1056, 65, 24), (4096, 300, 32), (11008, 50, 5), (2048, 1000, 30), (96, 20, 40),
+                                       (4096, 4096, 16), (4096, 4090, 32), (2080, 4200, 8), (1056, 8500, 12), (4096, 8300, 32)])
 def test_split_pair(gpu, oracle, k, n, batch):
     rng = np.random.default_rng(k + n + batch)
     pg, pu = (kl.quantize_q4_0((rng.standard_normal((n, k)) * 0.02).astype(np.float32)) for _ in range(2))
@@ -121,3 +126,9 @@ def test_split_pair(gpu, oracle, k, n, batch):
     finite, ok, worst = check_pair(y, x, oracle.q4_decode(pg, k, n), oracle.q4_decode(pu, k, n), oracle, 1e-4)
     print(f"  split pair k={k} n={n} b={batch} {route} worst/bound={worst:.3g}", flush=True)
     assert route == "q4_mfma_pair_swiglu" and finite and ok
+    # a row's sums are those of a call on its matrix (whose columns past 32 may take another route)
+    (g, rg, _), (u, ru, _) = (run_matmul(Q4, w, x, k, n, batch) for w in (pg, pu))
+    if rg == ru == SPLIT:
+        assert np.array_equal(y[:32].view(np.uint32), device_swiglu(g, u)[:32].view(np.uint32))
+    else:
+        assert (k, n) == (2048, 1000) and rg == ru == "q4_bdiag_gemv"
