@@ -467,12 +467,13 @@ __global__ __launch_bounds__(kCqThreads) void common_gemv(GemvMatrix m0, GemvMat
 // wave copies RT SB / 8 fragments (1 KB each, in operand order), 1 KB of weights
 // and 128 B of scales into LDS (global_load_lds), into a ring of SLOTS stages.
 //
-// Bound: MFMA and VALU issue, which hardly overlap here (a probe of independent
-// chains, two waves per SIMD: 16 MFMAs 253 cycles, 64 fmas 158, both 380): K4096
-// x N11008 at 512 rows needs 29 us of it. 16 CG columns per fragment read keep
-// the LDS reads (CG = 2: 85 B per cycle and CU, which bound the kernel) below
-// that; KG splits K over the waves rather than the tile, so that few rows and
-// columns per workgroup still fill the CUs. kk_common_gemm has the times.
+// MFMA and VALU issue hardly overlap here (a probe of independent chains, two
+// waves per SIMD: 16 MFMAs 253 cycles, 64 fmas 158, both 380): K4096 x N11008 at
+// 512 rows needs 29 us of it, of the 75 that the kernel takes. The rest is what a
+// stage does before its first product: the wait for its copies, the barrier and
+// the operand reads (CG = 2: 85 B per cycle and CU at full MFMA rate). KG splits K
+// over the waves rather than the tile, so that few rows and columns per workgroup
+// still fill the CUs. kk_common_gemm has the times.
 template <int RT, int CG, int KG, int BPW, int SLOTS>
 struct CgShape {
     static constexpr int CW = 8 / KG;                                   // column waves
@@ -659,10 +660,11 @@ extern "C" int kk_common_quant_pair(const void *x, int x_f16, int k, int kp, voi
 }
 
 extern "C" int kk_common_quant_rows(const void *x, int x_f16, int k, int kp, int rows, int defined_rows,
-                                    int view_from, size_t chunk_stride, void *values, void *params, void *frags, hipStream_t stream) {
+                                    int view_from, size_t chunk_stride, void *values, void *params, void *frags,
+                                    hipStream_t stream) {
     if (!x || !values || !params || !frags || k <= 0 || kp < k || kp % 256 != 0 || rows <= 0 ||
-        defined_rows < rows || defined_rows % 32 != 0 || view_from < 0 || view_from >= rows || (reinterpret_cast<uintptr_t>(values) & 7) || (chunk_stride & 7) ||
-        (reinterpret_cast<uintptr_t>(frags) & 15))
+        defined_rows < rows || defined_rows % 32 != 0 || view_from < 0 || view_from >= rows ||
+        (reinterpret_cast<uintptr_t>(values) & 7) || (chunk_stride & 7) || (reinterpret_cast<uintptr_t>(frags) & 15))
         return hipErrorInvalidValue;
     if (x_f16)
         hipLaunchKernelGGL(common_quant_rows<true>, dim3(defined_rows), dim3(kRowThreads), 0, stream, x, k, kp, rows,

@@ -11,7 +11,7 @@
 // read hit 16 distinct bank quads; lane (n, g) reads K 8g .. 8g + 7 of its row.
 //
 // 16 rows per workgroup, for 256 workgroups at N4096. K4096 x N4096 at 64 columns
-// has 14.5 us of fp32 MFMA and 13 us of weight reads; the kernel takes 29.6 us (51
+// has 14.5 us of fp32 MFMA and 13 us of weight reads; the kernel takes 27.5 us (51
 // in passes of 16 columns), 1900 cycles per stage for 1024 of MFMA on each SIMD:
 // the waves of a SIMD read their operands together after each barrier. Where
 // there are more workgroups than CUs, two per CU with half the ring each overlap

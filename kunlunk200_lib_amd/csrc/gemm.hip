@@ -1523,8 +1523,9 @@ __global__ __launch_bounds__(512) void q4_wide_gemm(const uint8_t *__restrict__ 
 // read in step s - 1, so those reads are waited for before the barrier.
 // Bound by the MFMAs, and the clock under them once all CUs run (K4096 x N4096: 192 tiles of
 // 128 x 256 take 57 us, 256 tiles 70); the register-staged kernel reads 85 - 128 bytes of
-// operands per cycle and CU from LDS at full MFMA rate, these 48 and 80. K4096 x N11008,
-// 2048 rows: 322 -> 205 us per call (930 TFLOP/s; a library fp16 GEMM 203).
+// operands per cycle and CU from LDS at full MFMA rate, these 48 and 80. us per call with
+// weights from HBM, register-staged / these: K4096 x N11008 at 512 rows 107 / 71, 1024 164 /
+// 116, 2048 314 / 214 (kernel 205: 900 TFLOP/s), K4096 x N4096 at 2048 120 / 80.
 template <int KG>
 struct WfShape {
     static constexpr int Rows = 256 / KG, StepK = 32 * KG, Bufs = KG == 1 ? 4 : 3;

@@ -114,7 +114,7 @@ int f32_gemm_columns(int k, int n, int batch) { return batch == 33 && k >= 4096 
 int gemv_chunk(int type) { return type == 2 && q4_mfma_batch(16, true) ? 32 : 16; }
 
 // Batch range of the block-diagonal Q4_0 MFMA GEMV (the single-pass kernel's
-// range, unless KUNLUN_Q4_BDIAG=0 leaves it to the LDS-staged kernels).
+// range, unless KUNLUN_Q4_BDIAG=0 leaves it to the K-split kernel).
 bool q4_bdiag_batch(int batch) {
     return kk::tuning_or(kk::kQ4Bdiag, 1) != 0 && q4_mfma_batch(batch, true);
 }

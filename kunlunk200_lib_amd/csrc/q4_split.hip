@@ -1,9 +1,9 @@
-// Q4_0 GEMV for 3..64 activation columns in one pass over the weights, on
+// Q4_0 GEMV for 3..32 activation columns in one pass over the weights, on
 // gfx950 fp16 MFMA, with K split over workgroups.
 //
 // Y[b, r] = sum_k X[b, k] * W[r, k] (reference kernels/kunlun-matvec.xpu:24-79).
 //
-// Products as in mgemv.hip: per 32-value block the exact fp16 q - 8 (B) times
+// Products: per 32-value block the exact fp16 q - 8 (B) times
 // the activations as fp16 hi + lo of x * 2^s (A, about 22 bits), block sums in
 // F32, scaled by the block's F16 scale in F32.
 //

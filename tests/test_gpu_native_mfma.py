@@ -1,8 +1,9 @@
-"""GPU parity of native_q4_matmul above one column (int8 MFMA, up to 16
-columns per launch): one column per digit slot and three MFMAs per block
-(1..5 and 6..16 columns), blocks that do not fill the waves, one and several
-LDS chunks of activations, remainders of N, unaligned F32 and F16 X, columns of
-very different size and non-finite activations. Same bounds as the other
+"""GPU parity of native_q4_matmul above one column (int8 MFMA, the three digits
+of up to 5 columns in one MFMA per block, a call's column groups in one launch
+as long as it holds them): full and partial column groups, blocks that do not
+fill the waves, one and several LDS chunks of activations, remainders of N,
+unaligned F32 and F16 X, columns of very different size and non-finite
+activations. Same bounds as the other
 native Q4 tests: exact up to the activations' 23-bit block fixed point.
 """
 import numpy as np
