@@ -339,7 +339,7 @@ static void run_q4_pair(Q4PairRoute route, Kernel::Impl & impl, detail::DeviceCo
         impl.route = "q4_bdiag_pair_swiglu";
         break;
     case Q4PairRoute::split:
-        // both products' K ranges in one launch, their sums and SwiGLU in the next
+        // both products' K ranges in one launch, their sums and SwiGLU in the next (one range: in the same)
         grow_split(id, ctx, impl, kk_q4_split_workspace_bytes(k, n, batch, 1, ctx.cus));
         detail::check_hip((hipError_t)kk_q4_split_gemv(w_gate, w_up, x, y, k, n, batch, impl.gemm_workspace, ctx.cus,
                                                        ctx.stream),

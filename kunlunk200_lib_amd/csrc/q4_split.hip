@@ -11,7 +11,7 @@
 // 16-row weight tiles; wave (wt, kg) sums tiles wt, wt + 16 / KG, ... over k-group
 // kg's part of the range. The range's activations are converted into MFMA A
 // fragments in LDS by the workgroup itself (no prepass launch), in chunks of
-// at most 128 KiB. With S > 1 (and for a pair) the F32 sums go to a workspace
+// at most 128 KiB. With S > 1 the F32 sums go to a workspace
 // [range][matrix][column][row], and q4_split_sum adds the ranges in order (and
 // applies SiLU * up); one range stores y directly. A range of one chunk keeps
 // its fragments for any number of tiles; one of several chunks keeps one
@@ -273,12 +273,20 @@ __device__ __forceinline__ void qs_step(QsRaw<GEN> &raw, Next next, uint32_t shi
 
 // GEN: any K % 32 == 0 and any weight alignment (dword loads, byte shifts,
 // blocks past K masked); else K % 256 == 0 and 4-byte aligned weights.
-// SERIAL (one matrix, one tile per wave): a workgroup takes its tiles' ranges in turn, at_once
+// kSerial (one matrix, one tile per wave): a workgroup takes its tiles' ranges in turn, at_once
 // of them at a time (whose fragments fit one chunk), and adds their sums in range order, as
 // q4_split_sum does, so that no partial sum leaves it.
-template <int MT, bool PACK, bool GEN, bool SERIAL>
+// kFused (a pair of one range): a gate tile and the up tile of the same rows go to two waves
+// side by side, and the gate tile's wave stores SiLU(gate) * up; the summing launch and the
+// trip through the workspace are 1.5 - 2 us of such a call (K1536 at 9 / 16 columns, us: N1000
+// 11.0 / 11.2 with them, 9.2 / 9.4 without; N4096 11.2 / 11.4, 9.3 / 9.6; N11008 15.4 / 15.8,
+// 13.8 / 14.0).
+constexpr int kRanges = 0, kSerial = 1, kFused = 2;
+
+template <int MT, bool PACK, bool GEN, int FORM>
 __global__ __launch_bounds__(kQsThreads) void q4_split_gemv(const QsArgs p) {
     using Q = QsShape<MT, PACK>;
+    constexpr bool SERIAL = FORM == kSerial, FUSED = FORM == kFused;
     extern __shared__ __align__(16) uint8_t qs_lds[];
     const int bid = blockIdx.x;
     const int idx = (bid % kXcds) * p.per_xcd + bid / kXcds;    // contiguous ranges per XCD share X in its L2
@@ -294,7 +302,8 @@ __global__ __launch_bounds__(kQsThreads) void q4_split_gemv(const QsArgs p) {
     const int slot = SERIAL ? wid / (tw * p.kgroups) : 0;       // the wave's range of those at a time
     const int blocks = p.k >> 5;
     const uint32_t row_bytes = static_cast<uint32_t>(blocks) * 18u;
-    const int all_tiles = p.w2 ? 2 * p.tiles : p.tiles;         // the gate matrix's tiles, then the up matrix's
+    // of a pair the gate matrix's tiles, then the up matrix's (FUSED: in turn, from an even tile)
+    const int all_tiles = p.w2 ? 2 * p.tiles : p.tiles;
     const int first = group * p.per_group, end = min(first + p.per_group, all_tiles);
     const int rounds = SERIAL ? 1 : (p.per_group + tw - 1) / tw;   // tiles per wave (1 with several chunks)
 
@@ -306,8 +315,8 @@ __global__ __launch_bounds__(kQsThreads) void q4_split_gemv(const QsArgs p) {
     for (int round = 0; round < rounds; ++round) {
         const int tile = first + round * tw + wt;
         const bool live = tile < end;                           // wave-uniform; an idle wave helps to convert X
-        const bool up = live && tile >= p.tiles;
-        const int row = (up ? tile - p.tiles : tile) * 16 + c16;
+        const bool up = FUSED ? tile & 1 : live && tile >= p.tiles;
+        const int row = (FUSED ? tile >> 1 : up ? tile - p.tiles : tile) * 16 + c16;
         const uint8_t *m = up ? p.w2 : p.w;
         const uint32_t mis = GEN ? static_cast<uint32_t>(reinterpret_cast<uintptr_t>(m) & 3) : 0u;
         const uint32_t pos = mis + static_cast<uint32_t>(min(row, p.n - 1)) * row_bytes + 36u * g;
@@ -410,7 +419,25 @@ __global__ __launch_bounds__(kQsThreads) void q4_split_gemv(const QsArgs p) {
                         for (int t = 0; t < MT; ++t) sum[t] += xfer[((wid + (h * p.kgroups - 1) * tw) * MT + t) * kWave + lane];
             }
         }
-        if (live && kg == 0 && slot == 0 && row < p.n && !(PACK && g >= 2)) {
+        if constexpr (FUSED) {
+            // in places that no k-group used (tw / 2 of the tw - 1 that are left)
+            float4v *xfer = reinterpret_cast<float4v *>(qs_lds + Q::RingBytes) + (kQsWaves - tw + (wt >> 1)) * MT * kWave + lane;
+            if (p.kgroups == 1 && round > 0) __syncthreads();   // the round before's are read
+            if (up && kg == 0) {
+#pragma unroll
+                for (int t = 0; t < MT; ++t) xfer[t * kWave] = sum[t];
+            }
+            __syncthreads();
+            if (!up && kg == 0) {
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    const float4v u = xfer[t * kWave];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sum[t][r] = kk::swiglu_value(sum[t][r], u[r]);
+                }
+            }
+        }
+        if (live && kg == 0 && slot == 0 && !(FUSED && up) && row < p.n && !(PACK && g >= 2)) {
             float *out = p.out + (SERIAL ? 0 : static_cast<size_t>(range0) * (p.w2 ? 2 : 1) + (up ? 1 : 0)) * p.batch * p.row_stride + row;
 #pragma unroll
             for (int t = 0; t < MT; ++t)
@@ -461,6 +488,7 @@ struct QsPlan {
     int tiles, per_group, groups;   // 16-row tiles of one matrix; tiles of a workgroup; workgroups per range
     int stride;            // row stride of a partial sum
     size_t part_bytes;     // partial sums (0: one range stores y directly)
+    bool fused;            // a pair of one range: kFused
 };
 
 // The partial sums of one matrix stay within the no-allocation entry point's
@@ -510,32 +538,34 @@ QsPlan qs_plan(int k, int n, int batch, bool pair, int cus) {
             p.ranges /= 2;
     const size_t one = static_cast<size_t>(batch) * p.stride * 4;   // one range's sums
     while (p.ranges > 1 && p.ranges * one > kMaxPartBytes) p.ranges /= 2;
-    p.part_bytes = p.ranges == 1 && !pair ? 0 : static_cast<size_t>(p.ranges) * (pair ? 2 : 1) * one;
     // one workgroup per CU where the tiles allow; a range of several chunks
     // holds one tile per wave
     const int max_groups = std::max(1, cus / p.ranges);
     auto per_cu = [&](int tiles) { return (tiles + max_groups - 1) / max_groups; };
     p.kgroups = floor_pow2(std::max(1, std::min(kQsWaves / std::min(kQsWaves, per_cu(p.tiles)), steps / p.ranges)));
     const int all = pair ? 2 * p.tiles : p.tiles;
-    p.per_group = per_cu(all);
+    p.fused = pair && p.ranges == 1 && p.kgroups <= kQsWaves / 2;   // two waves for a k-group's two tiles
+    p.part_bytes = p.ranges == 1 && (!pair || p.fused) ? 0 : static_cast<size_t>(p.ranges) * (pair ? 2 : 1) * one;
+    p.per_group = p.fused ? 2 * per_cu(p.tiles) : per_cu(all);
     if ((steps + p.ranges - 1) / p.ranges > chunk) p.per_group = std::min(p.per_group, kQsWaves / p.kgroups);
     p.groups = (all + p.per_group - 1) / p.per_group;
     return p;
 }
 
-template <int MT, bool PACK, bool GEN, bool SERIAL>
+template <int MT, bool PACK, bool GEN, int FORM>
 hipError_t qs_launch(const QsArgs &a, hipStream_t stream) {
     using Q = QsShape<MT, PACK>;
-    const hipError_t rc = kk::opt_in_lds(reinterpret_cast<const void *>(&q4_split_gemv<MT, PACK, GEN, SERIAL>), Q::LdsBytes);
+    const hipError_t rc = kk::opt_in_lds(reinterpret_cast<const void *>(&q4_split_gemv<MT, PACK, GEN, FORM>), Q::LdsBytes);
     if (rc != hipSuccess) return rc;
-    hipLaunchKernelGGL((q4_split_gemv<MT, PACK, GEN, SERIAL>), dim3(a.per_xcd * kXcds), dim3(kQsThreads), Q::LdsBytes, stream, a);
+    hipLaunchKernelGGL((q4_split_gemv<MT, PACK, GEN, FORM>), dim3(a.per_xcd * kXcds), dim3(kQsThreads), Q::LdsBytes, stream, a);
     return hipGetLastError();
 }
 
 template <int MT, bool PACK>
-hipError_t qs_launch_form(const QsArgs &a, bool gen, bool serial, hipStream_t stream) {
-    if (serial) return gen ? qs_launch<MT, PACK, true, true>(a, stream) : qs_launch<MT, PACK, false, true>(a, stream);
-    return gen ? qs_launch<MT, PACK, true, false>(a, stream) : qs_launch<MT, PACK, false, false>(a, stream);
+hipError_t qs_launch_form(const QsArgs &a, bool gen, int form, hipStream_t stream) {
+    if (form == kSerial) return gen ? qs_launch<MT, PACK, true, kSerial>(a, stream) : qs_launch<MT, PACK, false, kSerial>(a, stream);
+    if (form == kFused) return gen ? qs_launch<MT, PACK, true, kFused>(a, stream) : qs_launch<MT, PACK, false, kFused>(a, stream);
+    return gen ? qs_launch<MT, PACK, true, kRanges>(a, stream) : qs_launch<MT, PACK, false, kRanges>(a, stream);
 }
 
 // Runs `p` (w2 null: one matrix); `workspace` holds p.part_bytes, or is null for one matrix:
@@ -570,9 +600,10 @@ hipError_t qs_run(const QsPlan &p, const uint8_t *w, const uint8_t *w2, const fl
     const uintptr_t bits = reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(w2);
     const bool gen = k % kStepK != 0 || (bits & 3) != 0;
     a.inf_bits = k % 64 != 0 || (bits & 3) != 0 ? 0x7f800000u : 0xffffffffu;
-    hipError_t rc = batch <= 8    ? qs_launch_form<1, true>(a, gen, serial, stream)
-                    : batch <= 16 ? qs_launch_form<1, false>(a, gen, serial, stream)
-                                  : qs_launch_form<2, false>(a, gen, serial, stream);
+    const int form = serial ? kSerial : p.fused ? kFused : kRanges;
+    hipError_t rc = batch <= 8    ? qs_launch_form<1, true>(a, gen, form, stream)
+                    : batch <= 16 ? qs_launch_form<1, false>(a, gen, form, stream)
+                                  : qs_launch_form<2, false>(a, gen, form, stream);
     if (rc != hipSuccess || !split) return rc;
     const int threads = batch * (p.stride / 4);
     const dim3 grid((threads + kSumThreads - 1) / kSumThreads), block(kSumThreads);

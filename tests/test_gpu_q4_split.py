@@ -114,10 +114,13 @@ def test_split_largest_activations(gpu, oracle, k, batch):
     assert guard_ok and res["finite"] and res["north_star"]
 
 
-# the last five: second rounds, with one k-group and with four (which use their exchange
-# area again), in one K range and in several
+# the second line: second rounds, with one k-group and with four (which use their exchange
+# area again), in one K range and in several; the third: one range, whose products and
+# SwiGLU are one launch, with one to eight k-groups and one to three rounds
 @pytest.mark.parametrize("k,n,batch", [(1056, 65, 24), (4096, 300, 32), (11008, 50, 5), (2048, 1000, 30), (96, 20, 40),
-                                       (4096, 4096, 16), (4096, 4090, 32), (2080, 4200, 8), (1056, 8500, 12), (4096, 8300, 32)])
+                                       (4096, 4096, 16), (4096, 4090, 32), (2080, 4200, 8), (1056, 8500, 12), (4096, 8300, 32),
+                                       (1536, 1000, 16), (1536, 4097, 9), (544, 300, 12), (32, 50, 16), (2080, 17, 10),
+                                       (512, 66000, 17), (1024, 9000, 32), (1056, 33000, 8)])
 def test_split_pair(gpu, oracle, k, n, batch):
     rng = np.random.default_rng(k + n + batch)
     pg, pu = (kl.quantize_q4_0((rng.standard_normal((n, k)) * 0.02).astype(np.float32)) for _ in range(2))
@@ -129,6 +132,8 @@ def test_split_pair(gpu, oracle, k, n, batch):
     # a row's sums are those of a call on its matrix (whose columns past 32 may take another route)
     (g, rg, _), (u, ru, _) = (run_matmul(Q4, w, x, k, n, batch) for w in (pg, pu))
     if rg == ru == SPLIT:
-        assert np.array_equal(y[:32].view(np.uint32), device_swiglu(g, u)[:32].view(np.uint32))
+        expected = np.hstack([device_swiglu(np.ascontiguousarray(g[:32, c:c + 16384]), np.ascontiguousarray(u[:32, c:c + 16384]))
+                              for c in range(0, n, 16384)])
+        assert np.array_equal(y[:32].view(np.uint32), expected.view(np.uint32))
     else:
         assert (k, n) == (2048, 1000) and rg == ru == "q4_bdiag_gemv"
