@@ -1985,6 +1985,10 @@ int pick_f16_wide(const GemmPlan &p, int batch, int n, int k, bool pair) {
     const double kib = k / 1024.0;
     auto rounds = [&](long tiles) { return static_cast<double>((tiles + cus - 1) / cus); };
     const long tiles = static_cast<long>(p.m_tiles) * (pair ? (n + 63) / 64 : p.n_tiles);
+    // one round of 128 x 64 register-staged tiles is faster above K128 (the fits err below 512): us
+    // staged / 128 rows, K128 x N4096 b256 12.6 / 11.8, K256 b64 10.8 / 12.0, N1000 b512 11.4 / 12.9, K384 x
+    // N4096 b100 13.7 / 14.5
+    if (!pair && p.bn == 64 && tiles <= cus && k > 128) return 0;
     const double staged = !pair && p.bn == 64 ? rounds(tiles) * (6 + 5.5 * kib)
                           : tiles <= cus      ? (11 + 10.7 * kib) * (0.7 + 0.3 * tiles / cus)   // (a part of a round)
                                               : rounds(tiles) * (7 + 9.6 * kib);

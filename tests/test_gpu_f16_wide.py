@@ -68,6 +68,12 @@ def test_f16_wide_dispatch(gpu, oracle, k, n, batch, runs):
     assert route == "f16_gemm_mfma" and guard_ok and finite and ok and np.all(np.isfinite(y))
 
 
+# One round of register-staged tiles stays there from K 192 on, two rounds do not (the probe needs K 256)
+@pytest.mark.parametrize("k,n,batch,runs", [(256, 1000, 512, False), (384, 16384, 100, False), (256, 9434, 222, True)])
+def test_f16_short_k_dispatch(gpu, k, n, batch, runs):
+    assert rows_128(k, n, batch) == runs
+
+
 @pytest.mark.parametrize("tile", WIDE)
 @pytest.mark.parametrize("k,n,batch", [(32, 64, 64), (64, 700, 200), (96, 33, 70), (192, 257, 129), (4096, 300, 513),
                                        (320, 1, 256), (16384, 256, 65), (5600, 511, 300)])
