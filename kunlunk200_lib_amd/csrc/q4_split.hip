@@ -31,9 +31,9 @@
 // 5.4 us for reading its 25 MB. Against the kernels before (64 rows per
 // workgroup over all of K, activations from a prepass, 16 columns per pass),
 // us per call: K11008 x N4096 at 8 / 16 / 32 columns 37.8 / 38.0 / 75.6 -> 13.0 /
-// 14.6 / 19.5; K4096 x N11008 at 16 / 32 15.6 / 30.9 -> 15.0 / 20.1; K4096 x
+// 14.6 / 19.5; K4096 x N11008 at 16 / 32 15.7 / 30.9 -> 14.5 / 20.6; K4096 x
 // N4096 14.6 / 28.6 -> 10.3 / 13.9; pair K4096 x 2 x N11008 27.5 / 54.4 ->
-// 23.0 / 31.
+// 23.2 / 33.
 //
 // Scales. Each (column, 256-value step) has its own power of two with
 // max |x * 2^s| < 2^14; a step's sums are multiplied by 2^-s and added to the
